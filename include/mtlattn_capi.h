@@ -157,6 +157,8 @@ int mtlattn_varlen_fwd_noalloc(const mtlattn_problem* p,
  * problems whose dQ or dK/dV grid would leave CUs idle, the size query adds
  * room (after delta, 256-byte aligned) for fp32 partials of 2-8 splits,
  * summed in a fixed order; a workspace of only the delta size runs unsplit.
+ * The same holds for the dK/dV of fp16/bf16 problems whose key blocks would
+ * leave CUs idle (up to 1 GiB of fp32 partials, by the number of tokens).
  */
 size_t mtlattn_varlen_bwd_workspace_size(const mtlattn_problem* p);
 int mtlattn_varlen_bwd(const mtlattn_problem* p,

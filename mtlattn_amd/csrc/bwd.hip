@@ -26,6 +26,7 @@
 //   causal only, src/attn_mpp.metal:591). At head dims <= 64 without a bias
 //   a variant runs 4-wave workgroups (two per CU) in which every wave
 //   computes all four products for its own 32 keys.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -40,6 +41,12 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kKW = 32;   // dK/dV: keys per wave
+// make_dkv_plan: the most pieces per key block and bytes of partials, and the
+// cost of a piece besides its stages (its first tiles' latency, the partials
+// it writes; the same again for adding them) in 32-query stages.
+constexpr int kDkvMaxPieces = 16;
+constexpr double kDkvPieceCost = 8.;
+constexpr int64_t kDkvPartBytes = (int64_t)1 << 30;
 
 // ---------------------------------------------------------------------------
 // dQ.  8 waves (2 per SIMD), 32 query rows x 1 head per wave, the heads of a
@@ -350,8 +357,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void bwd_dq_kernel(BwdKParams p) {
 // D is the tile width (64, 128 or 256) and DV <= D the head dim; a
 // workgroup outputs the DO columns of dK and dV from C0 + DO * blockIdx.y
 // (DO < DV: the slices run as workgroups of one launch, each recomputing the
-// S and dP products). A stage holds 32 * NQB queries.
-template <typename T, int D, int DV, int DO, int C0, int NQB, bool BIAS, bool OUT_F32>
+// S and dP products). A stage holds 32 * NQB queries. SPLIT (grids that
+// leave CUs idle, make_dkv_plan): a workgroup takes one piece of a key block's
+// stages.
+template <typename T, int D, int DV, int DO, int C0, int NQB, bool BIAS, bool OUT_F32, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     constexpr int DC = (DV + 15) / 16, DB = (DO + 31) / 32;
     static_assert(C0 % 32 == 0 && C0 + DO <= D, "output slice");
@@ -388,9 +397,15 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     const int l32 = lane & 31, hi = lane >> 5;
     const bool role_a = w < NP;
     const int pair = w & (NP - 1);
-    const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-    const int hk = L / p.n_tiles;
-    const int t = L - hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    SplitPiece pc{};
+    if constexpr (SPLIT) {
+        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+    } else {
+        const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
+        pc.hk = L / p.n_tiles;
+        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    }
+    const int hk = pc.hk, t = pc.t;
     const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
     const int tb = tile_base(p.cu_kv, s, KB, p.total_kv);
     if (t < tb) return;
@@ -407,6 +422,16 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     const int key = kw + l32;                    // this lane's key column
     const bool key_ok = key < kv_len;
 
+    // Query tiles that can see any key of this workgroup; this workgroup's
+    // stages and the first of them.
+    const QWalk walk = query_walk(k0, KB, coff, q_len, kv_len, p.causal, p.window, QTL);
+    const int q_lo = walk.q_lo, n_q_tiles = walk.n_tiles;
+    int n_stages = n_q_tiles * p.g, st0 = 0;
+    if constexpr (SPLIT) {
+        st0 = pc.st0;
+        n_stages = pc.n;
+    }
+
     // B operand of this wave's first product: K^T (wave A) or V^T (wave B),
     // lane = key, d = 16 kc + 8 hi + j.
     u32x4_t kvf[DC];
@@ -419,14 +444,6 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
             kvf[kc] = (DV % 16 == 0 || 16 * kc + 8 * hi < DV) ? ld16(kp + 16 * kc) : u32x4_t{};
     }
 
-    // Query range that can see any key of this workgroup.
-    const int k_last_wg = min(kv_len, k0 + KB) - 1;
-    // (tile grid aligned to QTL so workgroups of a sequence share tiles)
-    const int q_lo = p.causal ? max(0, k0 - coff) / QTL * QTL : 0;
-    const int q_hi = p.window > 0 ? min(q_len, k_last_wg - coff + p.window) : q_len;
-    const int n_q_tiles = q_hi > q_lo ? (q_hi - q_lo + QTL - 1) / QTL : 0;
-    const int n_stages = n_q_tiles * p.g;
-
     // Stages run over the query tiles top-down with the heads inner, so every
     // workgroup of a sequence reads the same (tile, head) at the same time and
     // the L2 serves the repeats (each workgroup stops at its own causal start
@@ -435,8 +452,15 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     // Stages are visited in order, so each per-stage quantity (head, first
     // query, ring slot, source rows) is a cursor advanced one stage at a time:
     // no division by g or by the ring depth in the loop.
-    const int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0);
     const int64_t cyc = (int64_t)n_q_tiles * QTL;        // rows of the walk's wrap
+    int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0), hl_first = 0;
+    if constexpr (SPLIT) {   // the walk's position at stage st0
+        const int t0 = st0 / p.g;
+        hl_first = st0 - t0 * p.g;
+        qt_first -= t0 * QTL;
+        if (qt_first < q_lo) qt_first += (int)cyc;
+    }
+    const int h_first = hk * p.g + hl_first;
     // Direct loads of stage `st`: Q and dO tiles by four loader waves
     // (ldw = 0..3); lse by loaders 0 (and 2), delta by loaders 1 (and 3):
     // column ldw & 1, rows 64 (ldw >> 1) + lane, 4 bytes per lane.
@@ -449,11 +473,11 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     // Loader cursor: the next stage to issue. Advancing to the next head
     // moves the rows by DV columns (lse / delta by one); past the group's
     // last head they move to head 0 of the tile QTL rows up.
-    int ld_hl = 0, ld_qt = qt_first, ld_slot = 0, ld_dslot = 0;
+    int ld_hl = hl_first, ld_qt = qt_first, ld_slot = 0, ld_dslot = 0;
     const int l_col = ldw & 1, l_piece = ldw >> 1;   // (loaders with ldw < 2 * LPIECES)
-    const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)hk * p.g * DV;
-    const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)hk * p.g * DV;
-    const float* ld_l = (l_col == 0 ? p.lse : p.delta) + (int64_t)(qr.start + qt_first) * p.hq + hk * p.g;
+    const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)h_first * DV;
+    const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)h_first * DV;
+    const float* ld_l = (l_col == 0 ? p.lse : p.delta) + (int64_t)(qr.start + qt_first) * p.hq + h_first;
     const int64_t q_wrap = -(int64_t)(p.g - 1) * DV - (int64_t)QTL * p.q_rs;
     const int64_t do_wrap = -(int64_t)(p.g - 1) * DV - (int64_t)QTL * p.do_rs;
     const int64_t l_wrap = -(int64_t)(p.g - 1) - (int64_t)QTL * p.hq;
@@ -505,7 +529,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     constexpr bool SPREAD = !BIAS && D > 128 && NQB * DC >= 4 * ((QTL * D * 2 / 1024 + NP - 1) / NP);
     // Compute cursor: stage st (wave A, and wave B's dP) and the ring slot of
     // stage st - 1 (wave B's dS and dK).
-    int c_hl = 0, c_qt = qt_first, c_slot = 0, p_slot = NBUF - 1, c_dslot = 0;
+    int c_hl = hl_first, c_qt = qt_first, c_slot = 0, p_slot = NBUF - 1, c_dslot = 0;
     float bvals[NQB][16];                       // wave A: bias of the current query tile
 #pragma unroll
     for (int qb = 0; qb < NQB; ++qb)
@@ -574,7 +598,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
             // scalar offset (no per-element address arithmetic, no select).
             const bool fast_bias = BIAS && p.bias_b32 && (qt + QTL <= q_len) &&
                                    ((p.bias_ss < 0) | (qt + QTL <= p.bias_rows)) && (kw + kKW <= p.bias_cols);
-            const bool load_bias = BIAS && ((c_hl == 0) | (p.bias_hs != 0));
+            const bool load_bias = BIAS && ((c_hl == 0) | (p.bias_hs != 0) | (SPLIT && st == 0));
             if (!load_bias) {
             } else if (fast_bias) {
                 const float* b0 = p.bias + bias_row_offset(qr.start + qt, s, qr.start, p.bias_qs, p.bias_ss,
@@ -795,8 +819,10 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     }
 
     if (pair_active && key_ok) {
-        const int64_t off = (int64_t)(kr.start + key) * ((int64_t)p.hkv * DV) + (int64_t)hk * DV + c0;
+        const int64_t row = (int64_t)p.hkv * DV;
+        const int64_t off = (int64_t)(kr.start + key) * row + (int64_t)hk * DV + c0;
         void* dst = role_a ? p.dv : p.dk;
+        if constexpr (SPLIT) dst = p.part + part_offset(pc.z, role_a ? 1 : 0, p.total_kv, row);
         const float sc = role_a ? 1.f : p.scale;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
@@ -824,9 +850,9 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
 // D = 64, which stage each Q / dO tile for 256 keys but keep both waves of
 // a SIMD in step). The arithmetic is that of the wave-pair kernel (P
 // rounded to T, dP accumulated onto -delta, dS = P * (dP - delta) rounded
-// to T), visited in 64-query stages.
+// to T), visited in 64-query stages. SPLIT as in the wave-pair kernel.
 // ---------------------------------------------------------------------------
-template <typename T, int D, int DV, bool OUT_F32, int NW>
+template <typename T, int D, int DV, bool OUT_F32, int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKParams p) {
     static_assert(D == 64, "64-wide tiles");
     constexpr int NQB = 2;
@@ -841,9 +867,15 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
     const int l32 = lane & 31, hi = lane >> 5;
-    const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-    const int hk = L / p.n_tiles;
-    const int t = L - hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    SplitPiece pc{};
+    if constexpr (SPLIT) {
+        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+    } else {
+        const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
+        pc.hk = L / p.n_tiles;
+        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    }
+    const int hk = pc.hk, t = pc.t;
     const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
     const int tb = tile_base(p.cu_kv, s, KB, p.total_kv);
     if (t < tb) return;
@@ -860,6 +892,16 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     const int key = kw + l32;                    // this lane's key column
     const bool key_ok = key < kv_len;
 
+    // Query tiles that can see any key of this workgroup; this workgroup's
+    // stages and the first of them.
+    const QWalk walk = query_walk(k0, KB, coff, q_len, kv_len, p.causal, p.window, QTL);
+    const int q_lo = walk.q_lo, n_q_tiles = walk.n_tiles;
+    int n_stages = n_q_tiles * p.g, st0 = 0;
+    if constexpr (SPLIT) {
+        st0 = pc.st0;
+        n_stages = pc.n;
+    }
+
     // B operands of the S and dP products: K^T and V^T, lane = key,
     // d = 16 kc + 8 hi + j (rows past the end read the last key: masked)
     u32x4_t kf[DC], vf[DC];
@@ -875,25 +917,27 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
         }
     }
 
-    // Query tiles that can see any key of the workgroup, visited top-down
-    // with the GQA group's heads inner (as in the wave-pair kernel).
-    const int k_last_wg = min(kv_len, k0 + KB) - 1;
-    const int q_lo = p.causal ? max(0, k0 - coff) / QTL * QTL : 0;
-    const int q_hi = p.window > 0 ? min(q_len, k_last_wg - coff + p.window) : q_len;
-    const int n_q_tiles = q_hi > q_lo ? (q_hi - q_lo + QTL - 1) / QTL : 0;
-    const int n_stages = n_q_tiles * p.g;
-    const int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0);
+    // The query tiles are visited top-down with the GQA group's heads inner
+    // (as in the wave-pair kernel).
     const int64_t cyc = (int64_t)n_q_tiles * QTL;        // rows of the walk's wrap
+    int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0), hl_first = 0;
+    if constexpr (SPLIT) {   // the walk's position at stage st0
+        const int t0 = st0 / p.g;
+        hl_first = st0 - t0 * p.g;
+        qt_first -= t0 * QTL;
+        if (qt_first < q_lo) qt_first += (int)cyc;
+    }
+    const int h_first = hk * p.g + hl_first;
 
     // Direct loads of a stage: the Q and dO tiles by all NW waves, the lse
     // column by wave 0 and the delta column by wave 1 (one row per lane).
     TileStager<D, QTL, NW, DV> qst, dost;
     qst.init(p.q_rs, w, lane);
     dost.init(p.do_rs, w, lane);
-    int ld_hl = 0, ld_qt = qt_first, ld_slot = 0;
-    const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)hk * p.g * DV;
-    const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)hk * p.g * DV;
-    const float* ld_l = (w == 0 ? p.lse : p.delta) + (int64_t)(qr.start + qt_first) * p.hq + hk * p.g;
+    int ld_hl = hl_first, ld_qt = qt_first, ld_slot = 0;
+    const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)h_first * DV;
+    const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)h_first * DV;
+    const float* ld_l = (w == 0 ? p.lse : p.delta) + (int64_t)(qr.start + qt_first) * p.hq + h_first;
     const int64_t q_wrap = -(int64_t)(p.g - 1) * DV - (int64_t)QTL * p.q_rs;
     const int64_t do_wrap = -(int64_t)(p.g - 1) * DV - (int64_t)QTL * p.do_rs;
     const int64_t l_wrap = -(int64_t)(p.g - 1) - (int64_t)QTL * p.hq;
@@ -927,7 +971,7 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
         }
     };
 
-    int c_hl = 0, c_qt = qt_first, c_slot = 0;
+    int c_hl = hl_first, c_qt = qt_first, c_slot = 0;
     const uint32_t rbase = row_base<D>(l32, hi), tbase = tr_base<D>(lane);
     const float c2 = p.scale_log2;
     f32x16_t accv[DB], acck[DB];                 // dV^T, dK^T
@@ -1047,20 +1091,86 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     }
 
     if (wave_active && key_ok) {
-        const int64_t off = (int64_t)(kr.start + key) * ((int64_t)p.hkv * DV) + (int64_t)hk * DV;
+        const int64_t row = (int64_t)p.hkv * DV;
+        const int64_t off = (int64_t)(kr.start + key) * row + (int64_t)hk * DV;
+        void* dk = SPLIT ? p.part + part_offset(pc.z, 0, p.total_kv, row) : p.dk;
+        void* dv = SPLIT ? p.part + part_offset(pc.z, 1, p.total_kv, row) : p.dv;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg) {
                 const int d = 32 * db + 8 * rg + 4 * hi;
                 if (DV % 32 != 0 && d >= DV) continue;
-                store4<T, OUT_F32>(p.dv, off + d, accv[db][4 * rg], accv[db][4 * rg + 1], accv[db][4 * rg + 2],
+                store4<T, OUT_F32>(dv, off + d, accv[db][4 * rg], accv[db][4 * rg + 1], accv[db][4 * rg + 2],
                                    accv[db][4 * rg + 3]);
-                store4<T, OUT_F32>(p.dk, off + d, acck[db][4 * rg] * p.scale, acck[db][4 * rg + 1] * p.scale,
+                store4<T, OUT_F32>(dk, off + d, acck[db][4 * rg] * p.scale, acck[db][4 * rg + 1] * p.scale,
                                    acck[db][4 * rg + 2] * p.scale, acck[db][4 * rg + 3] * p.scale);
             }
         }
     }
+}
+
+// Zero the rows of a [total_rows, row_halves] tensor of 16-bit halves outside
+// [first, last), with all threads of grid x.
+__device__ inline void zero_outside(uint16_t* ptr, int64_t row_halves, int64_t total_rows, int64_t first, int64_t last) {
+    first = first < 0 ? 0 : (first > total_rows ? total_rows : first);
+    last = last < first ? first : (last > total_rows ? total_rows : last);
+    const int64_t head_end = first * row_halves, tail_begin = last * row_halves, end = total_rows * row_halves;
+    const int64_t n = head_end + (end - tail_begin);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        ptr[i < head_end ? i : tail_begin + (i - head_end)] = 0;
+}
+
+// ---------------------------------------------------------------------------
+// The second pass of a split dK/dV: one thread per 4 columns of a key row
+// adds its block's fp32 partials in piece order and writes dK and dV; rows
+// that no sequence owns are cleared, dQ's by grid row 1. Bound by the
+// partials' bytes, each read once.
+// ---------------------------------------------------------------------------
+struct FinishKParams {
+    const float* part;
+    uint16_t* dq; uint16_t* dk; uint16_t* dv;
+    const int* cu_q; const int* cu_kv;
+    int64_t total_q, total_kv, dq_row;
+    const int* piece;              // the piece length the split launch worked with
+    int num_seqs, row, g, causal, window, kb, qtl;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void dkv_finish_kernel(FinishKParams p) {
+    if (blockIdx.y == 1) {
+        zero_outside(p.dq, p.dq_row, p.total_q, p.cu_q[0], p.cu_q[p.num_seqs]);
+        return;
+    }
+    const uint32_t units = (uint32_t)p.row / 4;                  // 4-column units of a row
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t r = i / units;
+    if (r >= p.total_kv) return;
+    const int64_t off = (int64_t)i * 4;
+    int lo = 0, hi = p.num_seqs - 1;                             // largest s with cu_kv[s] <= r
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (p.cu_kv[mid] <= (int)r) lo = mid; else hi = mid - 1;
+    }
+    const SeqRange kr = seq_range(p.cu_kv, lo, p.total_kv);
+    float k4[4] = {0.f, 0.f, 0.f, 0.f}, v4[4] = {0.f, 0.f, 0.f, 0.f};
+    if ((int)r >= kr.start && (int)r < kr.end) {
+        const SeqRange qr = seq_range(p.cu_q, lo, p.total_q);
+        const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
+        const int k0 = ((int)r - kr.start) / p.kb * p.kb;
+        const QWalk walk = query_walk(k0, p.kb, kv_len - q_len, q_len, kv_len, p.causal, p.window, p.qtl);
+        const int pieces = split_pieces(walk.n_tiles * p.g, *p.piece);
+        const int64_t step = p.total_kv * p.row;
+        const float* src = p.part + off;
+#pragma unroll 4
+        for (int z = 0; z < pieces; ++z, src += 2 * step) {
+            const f32x4_t a = *reinterpret_cast<const f32x4_t*>(src);
+            const f32x4_t b = *reinterpret_cast<const f32x4_t*>(src + step);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { k4[e] += a[e]; v4[e] += b[e]; }
+        }
+    }
+    store4<T, false>(p.dk, off, k4[0], k4[1], k4[2], k4[3]);
+    store4<T, false>(p.dv, off, v4[0], v4[1], v4[2], v4[3]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1121,15 +1231,7 @@ struct ZeroJobs {
 };
 __global__ __launch_bounds__(256) void zero_outside_kernel(ZeroJobs jobs) {
     const ZeroJob& j = jobs.job[blockIdx.y];
-    uint16_t* __restrict__ ptr = j.ptr;
-    const int64_t row_halves = j.row_halves, total_rows = j.total_rows;
-    int64_t first = j.cu[0], last = j.cu[jobs.num_seqs];
-    first = first < 0 ? 0 : (first > total_rows ? total_rows : first);
-    last = last < first ? first : (last > total_rows ? total_rows : last);
-    const int64_t head_end = first * row_halves, tail_begin = last * row_halves, end = total_rows * row_halves;
-    const int64_t n = head_end + (end - tail_begin);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        ptr[i < head_end ? i : tail_begin + (i - head_end)] = 0;
+    zero_outside(j.ptr, j.row_halves, j.total_rows, j.cu[0], j.cu[jobs.num_seqs]);
 }
 
 int gcd_int(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
@@ -1173,37 +1275,78 @@ hipError_t launch_dq_typed(const BwdArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <typename T, int D, int DV, int DO, int C0, int NQB, bool OUT_F32>
-hipError_t launch_dkv_typed(const BwdArgs& a, hipStream_t st) {
+template <typename T>
+hipError_t launch_finish(const BwdArgs& a, int kb, int qtl, hipStream_t st) {
+    const Geometry& g = a.geo;
+    FinishKParams p;
+    p.part = a.dkv_part;
+    p.dq = (uint16_t*)a.dq; p.dk = (uint16_t*)a.dk; p.dv = (uint16_t*)a.dv;
+    p.cu_q = g.cu_q; p.cu_kv = g.cu_kv;
+    p.total_q = a.dq != nullptr ? g.total_q : 0; p.total_kv = g.total_kv;
+    p.dq_row = (int64_t)g.hq * g.d;
+    p.num_seqs = g.num_seqs; p.row = g.hkv * g.d; p.g = g.g;
+    p.causal = g.causal; p.window = g.window > 0 ? g.window : 0;
+    p.kb = kb; p.qtl = qtl; p.piece = make_params(a).piece_out;
+    const int64_t blocks = (g.total_kv * (p.row / 4) + 255) / 256;   // (make_dkv_plan bounds the partials)
+    hipLaunchKernelGGL(dkv_finish_kernel<T>, dim3((unsigned)blocks, 2), dim3(256), 0, st, p);
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess && a.cleared != nullptr) *a.cleared = true;
+    return e;
+}
+
+template <typename T, int D, int DV, int DO, int C0, int NQB, bool BIAS, bool OUT_F32>
+hipError_t launch_dkv_pair(const BwdArgs& a, hipStream_t st) {
     BwdKParams p = make_params(a);
-    constexpr int NW = kWaves;
-    p.n_tiles = (int)(a.geo.total_kv / (NW / 2 * kKW)) + a.geo.num_seqs + 1;
+    constexpr int KB = kWaves / 2 * kKW;
+    p.n_tiles = (int)(a.geo.total_kv / KB) + a.geo.num_seqs + 1;
     const int64_t blocks = (int64_t)p.n_tiles * a.geo.hkv;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
     // column slices (DO < DV) are the grid's second dimension: one launch,
     // so the slices' workgroups share the GPU instead of running one after
     // the other (a causal grid's tail is one heavy workgroup per CU)
-    const dim3 grid((unsigned)blocks, (unsigned)((DV - C0 + DO - 1) / DO));
+    const unsigned slices = (DV - C0 + DO - 1) / DO;
+    if constexpr (!OUT_F32) {
+        if (use_split(a, p.n_tiles)) {
+            hipLaunchKernelGGL((bwd_dkv_kernel<T, D, DV, DO, C0, NQB, BIAS, true, true>),
+                               dim3((unsigned)a.dkv_plan.grid, slices), dim3(kThreads), 0, st, p);
+            const hipError_t e = hipGetLastError();
+            return e != hipSuccess ? e : launch_finish<T>(a, KB, 32 * NQB, st);
+        }
+    }
+    hipLaunchKernelGGL((bwd_dkv_kernel<T, D, DV, DO, C0, NQB, BIAS, OUT_F32, false>), dim3((unsigned)blocks, slices),
+                       dim3(kThreads), 0, st, p);
+    return hipGetLastError();
+}
+
+template <typename T, int D, int DV, int DO, int C0, int NQB, bool OUT_F32>
+hipError_t launch_dkv_typed(const BwdArgs& a, hipStream_t st) {
     if constexpr (NQB > 2) {
         if (a.geo.bias != nullptr) return hipErrorInvalidValue;   // (not dispatched: registers)
     } else if (a.geo.bias != nullptr) {
-        hipLaunchKernelGGL((bwd_dkv_kernel<T, D, DV, DO, C0, NQB, true, OUT_F32>), grid, dim3(NW * 64), 0, st, p);
-        return hipGetLastError();
+        return launch_dkv_pair<T, D, DV, DO, C0, NQB, true, OUT_F32>(a, st);
     }
-    hipLaunchKernelGGL((bwd_dkv_kernel<T, D, DV, DO, C0, NQB, false, OUT_F32>), grid, dim3(NW * 64), 0, st, p);
-    return hipGetLastError();
+    return launch_dkv_pair<T, D, DV, DO, C0, NQB, false, OUT_F32>(a, st);
 }
 
 template <typename T, int D, int DV, bool OUT_F32, int NW>
 hipError_t launch_dkv_sym(const BwdArgs& a, hipStream_t st) {
     BwdKParams p = make_params(a);
-    p.n_tiles = (int)(a.geo.total_kv / (NW * kKW)) + a.geo.num_seqs + 1;
+    constexpr int KB = NW * kKW;
+    p.n_tiles = (int)(a.geo.total_kv / KB) + a.geo.num_seqs + 1;
     const int64_t blocks = (int64_t)p.n_tiles * a.geo.hkv;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_dkv_sym_kernel<T, D, DV, OUT_F32, NW>), dim3((unsigned)blocks), dim3(NW * 64), 0, st, p);
+    if constexpr (!OUT_F32) {
+        if (use_split(a, p.n_tiles)) {
+            hipLaunchKernelGGL((bwd_dkv_sym_kernel<T, D, DV, true, NW, true>),
+                               dim3((unsigned)a.dkv_plan.grid), dim3(NW * 64), 0, st, p);
+            const hipError_t e = hipGetLastError();
+            return e != hipSuccess ? e : launch_finish<T>(a, KB, 64, st);
+        }
+    }
+    hipLaunchKernelGGL((bwd_dkv_sym_kernel<T, D, DV, OUT_F32, NW, false>), dim3((unsigned)blocks), dim3(NW * 64), 0, st,
+                       p);
     return hipGetLastError();
 }
-
 
 }  // namespace
 
@@ -1237,6 +1380,84 @@ hipError_t launch_bwd_preprocess(int dtype, const Geometry& geo, const void* o, 
         hipLaunchKernelGGL(bwd_preprocess_kernel<F32>, grid, dim3(256), 0, st, (const float*)o, o_rs,
                            (const float*)dout, do_rs, delta, geo.total_q, geo.hq, geo.d);
     return hipGetLastError();
+}
+
+hipError_t launch_dkv_finish(int type_code, const BwdArgs& a, int kb, int qtl, hipStream_t st) {
+    const hipError_t e = hipGetLastError();   // the split launch's
+    if (e != hipSuccess) return e;
+    return type_code == BF16::code ? launch_finish<BF16>(a, kb, qtl, st) : launch_finish<F16>(a, kb, qtl, st);
+}
+
+// Small problems have fewer key blocks than the GPU has CUs, and a block's
+// stages run one after the other: at 1 x 2048 causal tokens, 32/8 heads, the
+// one-wave-per-SIMD kernel at D = 128 had 32 workgroups of 288 stages (450 us
+// of a 500 us backward). There the blocks' stages are cut into pieces, one
+// workgroup each, with fp32 partials added afterwards: about 1.6 us a stage
+// against 12 us to start a piece and write its partials, and 8 to 20 us to
+// add them. Backward before -> after, bf16 causal, 32/8 heads, D = 128:
+// 1 x 512 193 -> 58 us, 1 x 2048 501 -> 167, 1 x 4096 973 -> 490, 2 x 4096
+// 1149 -> 955, 5 x 4096 (320 pairs on 256 CUs) 2660 -> 2365; D = 64, 16/4 heads,
+// 1 x 2048 193 -> 70; D = 256, 16/4, 1 x 2048 612 -> 248. The line: the split
+// has to beat the unsplit grid's rounds by 10% by this count of stages, on
+// sequences of the average length; 3 x 4096 (192 pairs, 1.0x split) and
+// 8 x 4096 (512 pairs) stay unsplit.
+DkvPlan make_dkv_plan(const Geometry& g, int cus) {
+    DkvPlan plan;
+    if (!mfma_head_dim(g.d) || g.total_q <= 0 || g.total_kv <= 0 || g.num_seqs < 1) return plan;
+    // the kernel these problems run: keys per block, queries per stage,
+    // workgroups per CU, and whether unsplit blocks are taken in pairs
+    const bool wide = g.bias == nullptr && g.d != 64 && g.d != 160, sym = g.bias == nullptr && g.d == 64;
+    const int kb = wide && g.d <= 128 ? 256 : 128, qtl = wide || g.d > 128 ? 32 : 64;
+    const int64_t slots = (int64_t)cus * (sym ? 2 : 1);
+    const bool paired = wide && g.window <= 0;
+    const int64_t n_tiles = g.total_kv / kb + g.num_seqs + 1, max_grid = 3 * slots;
+    const int64_t part = 2 * g.total_kv * g.hkv * (int64_t)g.d * (int64_t)sizeof(float);   // one piece of every block
+    const int max_pieces = (int)std::min<int64_t>(kDkvMaxPieces, kDkvPartBytes / part);
+    if (n_tiles > 64 * kSplitChunks || n_tiles * g.hkv > max_grid || max_pieces < 2) return plan;
+    // stages of the blocks of a sequence of average length
+    const int64_t lq = (g.total_q + g.num_seqs - 1) / g.num_seqs, lk = (g.total_kv + g.num_seqs - 1) / g.num_seqs;
+    const int64_t coff = lk - lq, nb = (lk + kb - 1) / kb, heads = (int64_t)g.hkv * g.num_seqs;
+    int64_t n[64 * kSplitChunks + 1], n_max = 0, work = 0;
+    for (int64_t b = 0; b < nb; ++b) {
+        const int64_t k0 = b * kb, last = std::min(lk, k0 + kb) - 1;
+        const int64_t lo = g.causal ? std::max<int64_t>(0, k0 - coff) / qtl * qtl : 0;
+        const int64_t hi = g.window > 0 ? std::min(lq, last - coff + g.window) : lq;
+        n[b] = hi > lo ? (hi - lo + qtl - 1) / qtl * g.g : 0;
+        n_max = std::max(n_max, n[b]);
+        work += n[b] * heads;
+    }
+    int64_t unit = n_max;                       // the longest workgroup, unsplit
+    if (paired && nb > 1) {
+        unit = 0;
+        for (int64_t b = 0; b < nb; ++b) unit = std::max(unit, b == nb - 1 - b ? n[b] : n[b] + n[nb - 1 - b]);
+    }
+    const int64_t units = (paired ? (nb + 1) / 2 : nb) * heads;
+    const double cost = kDkvPieceCost * 32. / qtl;
+    // Unsplit, equal workgroups run in whole rounds; single causal blocks,
+    // heaviest first, fill the slots but for a tail.
+    const bool even = paired || !g.causal || g.window > 0;
+    const double unsplit = even || units <= slots ? (double)((units + slots - 1) / slots * unit)
+                                                  : std::max((double)unit, 1.1 * (double)work / (double)slots);
+    double best = 0.9 * unsplit;
+    for (int r = 1; r <= 3; ++r) {
+        if (n_tiles * g.hkv > r * slots) continue;
+        auto wgs = [&](int64_t c) {
+            int64_t x = 0;
+            for (int64_t b = 0; b < nb; ++b) x += std::max<int64_t>(1, (n[b] + c - 1) / c);
+            return x * heads;
+        };
+        int64_t c = std::max<int64_t>(kSplitMinPiece, (n_max + max_pieces - 1) / max_pieces);
+        while (c < n_max && wgs(c) > r * slots) ++c;
+        const double t = (r == 1 ? (double)c : (double)work / (double)slots + 0.5 * (double)c) + cost * r +
+                         cost * (double)wgs(c) / (double)slots;
+        if (c < n_max && t < best) {
+            best = t;
+            // (sequences longer than the average have more pieces)
+            plan.pieces = (int)std::min<int64_t>(max_pieces, (n_max + c - 1) / c * (g.num_seqs > 1 ? 2 : 1));
+            plan.grid = (int)(r * slots);
+        }
+    }
+    return plan;
 }
 
 hipError_t launch_zero_outside(const ZeroFill* fills, int n, int num_seqs, hipStream_t st) {

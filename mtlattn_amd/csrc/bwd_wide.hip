@@ -61,8 +61,11 @@ namespace {
 // The arithmetic is that of the other dK/dV kernels: P and dS rounded to T,
 // dS from the rounded P, masks as -inf logits (scale > 0, host-checked).
 // ---------------------------------------------------------------------------
-template <typename T, int D, int DV, int NKB, bool OUT_F32>
+// SPLIT (grids that leave CUs idle, make_dkv_plan): a workgroup takes one
+// piece of one key block's stages.
+template <typename T, int D, int DV, int NKB, bool OUT_F32, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
+    static_assert(!SPLIT || OUT_F32, "the pieces' partials are fp32");
     static_assert((D == 128 && NKB == 2) || (D == 256 && NKB == 1), "128-wide tiles: 64 keys per wave; 256-wide: 32");
     constexpr int NW = 4, KPW = 32 * NKB;               // waves, keys per wave
     constexpr int DC = (DV + 15) / 16, DB = (DV + 31) / 32;
@@ -78,9 +81,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
     const int l32 = lane & 31, hi = lane >> 5;
-    const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-    const int hk = L / p.n_tiles;
-    const int t = L - hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    SplitPiece pc{};
+    if constexpr (SPLIT) {
+        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+    } else {
+        const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
+        pc.hk = L / p.n_tiles;
+        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+    }
+    const int hk = pc.hk, t = pc.t;
     // Tiles are pairs of key blocks, block pi and block nb - 1 - pi of a
     // sequence (nb blocks): with causal masking a pair's work is the same
     // for every pair, so the in-order dispatch of workgroups keeps the CUs
@@ -88,7 +97,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
     // XCD's last sequence's heavy blocks running alone at the end).
     // Under a sliding window every block but a sequence's last few has the
     // same work, and pairs would not be: tiles are then single blocks.
-    const bool paired = p.window <= 0;
+    const bool paired = !SPLIT && p.window <= 0;
     const int TK = paired ? 2 * KB : KB;               // keys per tile
     const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, TK, t, p.total_kv);
     const int tb = tile_base(p.cu_kv, s, TK, p.total_kv);
@@ -111,6 +120,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
         const bool wave_active = kw < kv_len;
         const int wk_last = min(kv_len, kw + KPW) - 1;
 
+        const QWalk walk = query_walk(k0, KB, coff, q_len, kv_len, p.causal, p.window, QTL);
+        const int q_lo = walk.q_lo, n_q_tiles = walk.n_tiles;
+        int n_stages = n_q_tiles * p.g, st0 = 0;   // this workgroup's stages, the first of them
+        if constexpr (SPLIT) {
+            st0 = pc.st0;
+            n_stages = pc.n;
+        }
+
         // B operands of the S and dP products: K^T and V^T of both key blocks,
         // lane = key kw + 32 kb + l32, d = 16 kc + 8 hi + j (keys past the end
         // read the last key: masked; columns past DV are zero)
@@ -131,13 +148,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
         // direct loads
         wait_vmcnt<0>();
 
-        const int k_last_wg = min(kv_len, k0 + KB) - 1;
-        const int q_lo = p.causal ? max(0, k0 - coff) / QTL * QTL : 0;
-        const int q_hi = p.window > 0 ? min(q_len, k_last_wg - coff + p.window) : q_len;
-        const int n_q_tiles = q_hi > q_lo ? (q_hi - q_lo + QTL - 1) / QTL : 0;
-        const int n_stages = n_q_tiles * p.g;
-        const int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0);
         const int64_t cyc = (int64_t)n_q_tiles * QTL;        // rows of the walk's wrap
+        int qt_first = first_q_tile(q_lo, n_q_tiles, QTL, p.window > 0), hl_first = 0;
+        if constexpr (SPLIT) {   // the walk's position at stage st0
+            const int t0 = st0 / p.g;
+            hl_first = st0 - t0 * p.g;
+            qt_first -= t0 * QTL;
+            if (qt_first < q_lo) qt_first += (int)cyc;
+        }
 
         // Direct loads of a stage: the Q and dO tiles by all four waves (two
         // 1 KB loads of each per wave), and every wave's own copy of the lse and
@@ -150,10 +168,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
         constexpr int LQ = Stager::N;                        // loads per wave per tile
         static_assert(Stager::PER % NW == 0, "whole tile loads per wave");
         constexpr int NL = 2 * LQ + 2;                       // loads per wave per stage
-        int ld_st = 0, ld_hl = 0, ld_qt = qt_first, ld_slot = 0;
-        const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)hk * p.g * DV;
-        const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)hk * p.g * DV;
-        const int64_t l0 = (int64_t)(qr.start + qt_first) * p.hq + hk * p.g;
+        int ld_st = 0, ld_hl = hl_first, ld_qt = qt_first, ld_slot = 0;
+        const int h_first = hk * p.g + hl_first;
+        const uint16_t* ld_q = p.q + (int64_t)(qr.start + qt_first) * p.q_rs + (int64_t)h_first * DV;
+        const uint16_t* ld_do = p.dout + (int64_t)(qr.start + qt_first) * p.do_rs + (int64_t)h_first * DV;
+        const int64_t l0 = (int64_t)(qr.start + qt_first) * p.hq + h_first;
         const float* ld_l = p.lse + l0;
         const float* ld_d = p.delta + l0;
         const int wcol = 2 * TILE + w * 2 * LCOL;            // this wave's lse column in a slot (delta: + LCOL)
@@ -264,7 +283,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
         // P(j) (packed) and dP(j) - delta stay in registers into iteration
         // j + 1. The loads of stage j + AHEAD go out during phases A (Q),
         // B (dO) and C (lse and delta).
-        int c_hl = 0, c_qt = qt_first, c_slot = 0, p_slot = 0;
+        int c_hl = hl_first, c_qt = qt_first, c_slot = 0, p_slot = 0;
         u32x4_t pk[NKB][2];                      // P of the stage in flight, rounded to T (B operands of dV)
         f32x16_t pacc[NKB];                      // its dP - delta
         f32x16_t sacc[NKB];
@@ -585,20 +604,24 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
         wait_vmcnt<0>();
 
         if (wave_active) {
+            // (SPLIT: this piece's fp32 partials)
+            const int64_t row = (int64_t)p.hkv * DV;
+            void* dk = SPLIT ? p.part + part_offset(pc.z, 0, p.total_kv, row) : p.dk;
+            void* dv = SPLIT ? p.part + part_offset(pc.z, 1, p.total_kv, row) : p.dv;
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb) {
                 const int key = kw + 32 * kb + l32;
                 if (key >= kv_len) continue;
-                const int64_t off = (int64_t)(kr.start + key) * ((int64_t)p.hkv * DV) + (int64_t)hk * DV;
+                const int64_t off = (int64_t)(kr.start + key) * row + (int64_t)hk * DV;
 #pragma unroll
                 for (int db = 0; db < DB; ++db) {
 #pragma unroll
                     for (int rg = 0; rg < 4; ++rg) {
                         const int d = 32 * db + 8 * rg + 4 * hi;
                         if (DV % 32 != 0 && d >= DV) continue;
-                        store4<T, OUT_F32>(p.dv, off + d, accv[kb][db][4 * rg], accv[kb][db][4 * rg + 1],
+                        store4<T, OUT_F32>(dv, off + d, accv[kb][db][4 * rg], accv[kb][db][4 * rg + 1],
                                            accv[kb][db][4 * rg + 2], accv[kb][db][4 * rg + 3]);
-                        store4<T, OUT_F32>(p.dk, off + d, acck[kb][db][4 * rg] * p.scale,
+                        store4<T, OUT_F32>(dk, off + d, acck[kb][db][4 * rg] * p.scale,
                                            acck[kb][db][4 * rg + 1] * p.scale, acck[kb][db][4 * rg + 2] * p.scale,
                                            acck[kb][db][4 * rg + 3] * p.scale);
                     }
@@ -613,12 +636,21 @@ template <typename T, int D, int DV, bool OUT_F32>
 hipError_t launch_wide(const BwdArgs& a, hipStream_t st) {
     constexpr int NKB = D == 128 ? 2 : 1, KB = 4 * 32 * NKB;
     BwdKParams p = make_params(a);
-    // pairs of key blocks (single blocks under a sliding window)
-    const int tk = a.geo.window > 0 ? KB : 2 * KB;
+    const bool split = !OUT_F32 && use_split(a, a.geo.total_kv / KB + a.geo.num_seqs + 1);
+    // pairs of key blocks (single blocks under a sliding window, or split)
+    const int tk = a.geo.window > 0 || split ? KB : 2 * KB;
     p.n_tiles = (int)(a.geo.total_kv / tk) + a.geo.num_seqs + 1;
     const int64_t blocks = (int64_t)p.n_tiles * a.geo.hkv;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_dkv_wide_kernel<T, D, DV, NKB, OUT_F32>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+    if constexpr (!OUT_F32) {
+        if (split) {
+            hipLaunchKernelGGL((bwd_dkv_wide_kernel<T, D, DV, NKB, true, true>),
+                               dim3((unsigned)a.dkv_plan.grid), dim3(256), 0, st, p);
+            return launch_dkv_finish(T::code, a, KB, 32, st);
+        }
+    }
+    hipLaunchKernelGGL((bwd_dkv_wide_kernel<T, D, DV, NKB, OUT_F32, false>), dim3((unsigned)blocks), dim3(256), 0, st,
+                       p);
     return hipGetLastError();
 }
 

@@ -455,9 +455,17 @@ int f32_dq_splits(const mtlattn_problem* p) {
     return (int)std::max<int64_t>(ns, 1);
 }
 
-// fp32 partial bytes after delta: dQ's, then (in the same space, after the
-// dQ splits are summed) dK/dV's
+// Split of the 16-bit matrix-core dK/dV
+DkvPlan dkv_plan(const mtlattn_problem* p) {
+    if (!is16(p->dtype) || force_generic()) return DkvPlan{};
+    return make_dkv_plan(make_geo(p), device_cus());
+}
+
+// fp32 partial bytes after delta: 16-bit dK/dV's; or fp32 dQ's, then (in the
+// same space, after the dQ splits are summed) dK/dV's
 size_t bwd_part_bytes(const mtlattn_problem* p) {
+    if (is16(p->dtype))
+        return (size_t)dkv_part_floats(dkv_plan(p).pieces, p->total_kv, p->num_heads_kv, p->head_dim) * sizeof(float);
     const int64_t fq = f32_dq_part_floats(f32_dq_splits(p), p->total_q, p->num_heads_q, p->head_dim);
     const int64_t fk = f32_dkv_part_floats(f32_dkv_splits(p), p->total_kv, p->num_heads_kv, p->head_dim);
     return (size_t)std::max<int64_t>(fq, fk) * sizeof(float);
@@ -541,11 +549,14 @@ int mtlattn_bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride
 
 namespace {
 
-// mtlattn_bwd_dkv, with fp32 dK/dV partials for `splits` splits in `part`
-// (fp32 matrix-core path only; splits == 1: none)
+// mtlattn_bwd_dkv, with fp32 dK/dV partials in `part` (null: unsplit): for
+// `splits` splits on the fp32 matrix cores, for `plan` on the 16-bit ones,
+// where the pass that adds them also clears the rows of dq, dk and dv that no
+// sequence owns (*cleared)
 int bwd_dkv(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
             const void* v, int64_t v_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
-            const float* delta, void* dk, void* dv, int32_t dkv_dtype, void* stream, float* part, int splits) {
+            const float* delta, void* dk, void* dv, int32_t dkv_dtype, void* stream, float* part, int splits,
+            const DkvPlan& plan = DkvPlan{}, void* dq = nullptr, bool* cleared = nullptr) {
     int rc = check_problem(p);
     if (rc != MTLATTN_OK) return rc;
     if (dkv_dtype != MTLATTN_DTYPE_F32 && dkv_dtype != p->dtype)
@@ -559,8 +570,15 @@ int bwd_dkv(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const
     a.dv = dv;
     a.out_f32 = dkv_dtype == MTLATTN_DTYPE_F32 ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
-    if (bwd_mfma_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride))
+    if (bwd_mfma_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride)) {
+        if (part != nullptr && plan.pieces > 1 && ((uintptr_t)dk & 7u) == 0 && ((uintptr_t)dv & 7u) == 0) {
+            a.dq = dq;
+            a.dkv_part = part;
+            a.dkv_plan = plan;
+            a.cleared = cleared;
+        }
         return launch_status(launch_bwd_dkv_mfma(p->dtype, a, st), "dK/dV");
+    }
     if (bwd_f32_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride) &&
         ((uintptr_t)dk & 15u) == 0 && ((uintptr_t)dv & 15u) == 0) {
         a.f32_part = part;
@@ -595,6 +613,8 @@ int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
                     workspace_bytes, need);
     float* delta = (float*)workspace;
     int splits = f32_dkv_splits(p), dq_splits = f32_dq_splits(p);
+    const DkvPlan plan = dkv_plan(p);
+    bool cleared = false;
     float* part = nullptr;
     const size_t part_bytes = bwd_part_bytes(p);
     if (part_bytes > 0 && workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 &&
@@ -647,8 +667,8 @@ int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
         if (rc != MTLATTN_OK) return rc;
     }
     rc = bwd_dkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta, dk, dv,
-                 p->dtype, stream, part, splits);
-    if (rc != MTLATTN_OK) return rc;
+                 p->dtype, stream, part, splits, plan, dq, &cleared);
+    if (rc != MTLATTN_OK || cleared) return rc;
     // Rows outside every sequence take no part in the forward: zero gradient.
     hipStream_t st = (hipStream_t)stream;
     const int64_t es = elem_size(p->dtype);

@@ -36,6 +36,18 @@ struct FwdArgs {
     int f32_splits = 1;
 };
 
+// How the 16-bit dK/dV cuts its work (make_dkv_plan): pieces == 1: one
+// workgroup per key block or pair of key blocks; else at most `pieces` pieces
+// per key block on a grid of `grid` workgroups.
+struct DkvPlan {
+    int pieces = 1, grid = 0;
+};
+DkvPlan make_dkv_plan(const Geometry& g, int cus);
+constexpr int kDkvPartTail = 64;   // floats past the partials (the piece length)
+inline int64_t dkv_part_floats(int pieces, int64_t total_kv, int hkv, int d) {
+    return pieces > 1 ? (int64_t)pieces * 2 * total_kv * hkv * d + kDkvPartTail : 0;
+}
+
 struct BwdArgs {
     Geometry geo;
     const void* q; int64_t q_rs;
@@ -59,6 +71,13 @@ struct BwdArgs {
     // fixed order afterwards; dQ also takes o / delta_out (delta in-kernel)
     float* f32_part = nullptr;
     int f32_splits = 1;
+    // 16-bit dK/dV only: with dkv_plan.pieces > 1 a launch of dkv_plan.grid
+    // workgroups takes pieces of the key blocks' work, with fp32 partials in
+    // dkv_part (dkv_part_floats floats); the pass that adds them also clears
+    // the rows of dq, dk and dv that no sequence owns and says so
+    float* dkv_part = nullptr;
+    DkvPlan dkv_plan;
+    bool* cleared = nullptr;
 };
 
 struct DecodeArgs {
@@ -92,6 +111,10 @@ hipError_t launch_bwd_dkv_mfma(int dtype, const BwdArgs& a, hipStream_t st);
 // dK/dV without a bias at head dims 80-128, one wave per SIMD (bwd_wide.hip);
 // hipErrorNotSupported when the problem is not for it. type_code: BF16::code / F16::code.
 hipError_t launch_bwd_dkv_wide(int type_code, const BwdArgs& a, hipStream_t st);
+// Adds the partials of a split dK/dV launch (key blocks of kb keys, stages of
+// qtl queries) into dk / dv and clears the rows of dq, dk and dv that no
+// sequence owns.
+hipError_t launch_dkv_finish(int type_code, const BwdArgs& a, int kb, int qtl, hipStream_t st);
 hipError_t launch_bwd_dq_generic(int dtype, const BwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_dkv_generic(int dtype, const BwdArgs& a, hipStream_t st);
 // fp32 inputs on the fp32 matrix cores (f32_mfma_head_dim, 16-byte aligned

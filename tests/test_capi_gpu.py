@@ -255,6 +255,69 @@ def test_capi_fp32_split_dkv():
                dtype, floors)
 
 
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,causal,window,bias", [
+    ([700, 0, 131, 1, 300], [700, 5, 200, 33, 300], 8, 2, 128, torch.bfloat16, True, 0, None),
+    ([511], [513], 12, 12, 128, torch.float16, False, 0, None),
+    ([1024], [1024], 16, 1, 80, torch.bfloat16, True, 0, None),
+    ([513, 640], [900, 700], 16, 4, 96, torch.float16, True, 400, None),
+    ([640, 129], [640, 129], 8, 2, 64, torch.float16, True, 0, None),
+    ([300, 1500], [300, 1500], 16, 4, 64, torch.bfloat16, True, 500, None),
+    ([511], [511], 8, 2, 256, torch.bfloat16, True, 0, None),
+    ([400, 300], [400, 333], 8, 2, 160, torch.float16, True, 0, None),
+    ([600, 70], [600, 90], 8, 2, 128, torch.bfloat16, True, 250, "broadcast"),
+    ([600, 70], [600, 90], 8, 2, 64, torch.float16, False, 0, "head"),
+    ([450], [450], 8, 2, 256, torch.bfloat16, True, 0, "broadcast"),
+])
+def test_capi_split_dkv(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window, bias):
+    """16-bit dK/dV on grids that would leave CUs idle: with the queried
+    workspace the key blocks' stages are cut into pieces whose fp32 partials
+    are added afterwards; a delta-sized workspace runs unsplit. Every kernel
+    (one wave per SIMD at 128- and 256-wide tiles, D = 64, wave pairs, column
+    slices), tiles with remainders, a single token, an empty sequence, keys
+    that no query sees and rows outside every sequence; a workspace full of
+    NaN does not leak, and the result repeats bitwise. The two differ in the
+    order of fp32 sums before one rounding to the output type: at most one unit
+    in the last place (2^-7 relative in bf16, 2^-10 in fp16) plus 1e-5 RMS."""
+    print(f"\n[case] capi split dK/dV D={D} {dtype} {q_lens} window={window} bias={bias}", flush=True)
+    q, k, v, do, cq, ck = _case(q_lens, kv_lens, Hq, Hkv, D, dtype, seed=31)
+    g = torch.Generator().manual_seed(32)
+    q, do = (torch.cat([t, randn((3, Hq, D), dtype, g)]) for t in (q, do))
+    k, v = (torch.cat([t, randn((3, Hkv, D), dtype, g)]) for t in (k, v))
+    bd = None
+    if bias:
+        bd = torch.randn(q.shape[0], 1 if bias == "broadcast" else Hq, max(kv_lens), generator=g).cuda()
+    qd, kd, vd, dod, cqd, ckd = (t.cuda() for t in (q, k, v, do, cq, ck))
+    p = capi.problem_for(qd, kd, cqd, ckd, max(q_lens), 1.0 / math.sqrt(D), causal=causal, window=window, bias=bd)
+    out = torch.zeros_like(qd)
+    lse = torch.empty(qd.shape[0], Hq, dtype=torch.float32, device="cuda")
+    s = _stream()
+    capi.call("mtlattn_varlen_fwd", p, qd.data_ptr(), Hq * D, kd.data_ptr(), Hkv * D, vd.data_ptr(), Hkv * D,
+              out.data_ptr(), lse.data_ptr(), None, 0, s)
+    ws_n, delta_n = capi.lib().mtlattn_varlen_bwd_workspace_size(p), qd.shape[0] * Hq * 4
+    assert ws_n > delta_n, "expected the split dK/dV workspace for this small grid"
+    runs = []
+    for n in (ws_n, ws_n, delta_n):
+        ws = torch.full((n // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        dq, dk, dv = (torch.full_like(t, float("nan")) for t in (qd, kd, vd))
+        capi.call("mtlattn_varlen_bwd", p, qd.data_ptr(), Hq * D, kd.data_ptr(), Hkv * D, vd.data_ptr(), Hkv * D,
+                  out.data_ptr(), Hq * D, dod.data_ptr(), Hq * D, lse.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+                  dv.data_ptr(), ws.data_ptr(), n, s)
+        torch.cuda.synchronize()
+        runs.append([t.cpu() for t in (dq, dk, dv)])
+    for a, b in zip(runs[0], runs[1]):
+        assert torch.equal(a, b), "split dK/dV not bitwise repeatable"
+    nq, nk = int(cq[-1]), int(ck[-1])
+    for r in runs:
+        assert not r[0][nq:].any() and not r[1][nk:].any() and not r[2][nk:].any()
+    assert torch.equal(runs[0][0], runs[2][0])
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    for nm, a, b in (("dk", runs[0][1], runs[2][1]), ("dv", runs[0][2], runs[2][2])):
+        a, b = a.float(), b.float()
+        assert torch.isfinite(a).all(), nm
+        over = (a - b).abs() - ulp * b.abs() - 1e-5 * b.pow(2).mean().sqrt()
+        assert over.max().item() <= 0, f"{nm}: split and unsplit differ by more than a rounding ({over.max():.3e})"
+
+
 def test_capi_splitkv_and_workspace_errors():
     print("\n[case] capi split-KV decode bf16 + workspace check", flush=True)
     kv_lens, Hq, Hkv, D = [3000, 5000, 2048], 16, 2, 128
