@@ -104,7 +104,9 @@ int mtlattn_gpu_core_count(int device);
  * forward.
  *   out : contiguous [total_q, Hq, D], same dtype as q
  *   lse : NULL or fp32 [total_q, Hq] (rows with no allowed key get -inf)
- * Workspace: the split-KV partials of calls routed to decode; for fp32
+ * Workspace: the split-KV partials of calls routed to decode (few-query calls
+ * of fewer than 2048 keys a sequence run without one, one workgroup per
+ * sequence and kv head); for fp32
  * problems on the fp32 matrix-core kernels whose grid would leave CUs idle,
  * fp32 partials of 2-8 key splits (a smaller workspace runs them unsplit);
  * otherwise none.
@@ -271,7 +273,7 @@ int mtlattn_paged_decode(const mtlattn_problem* p,
 /* Number of split-KV work-item slots per (kv head, head group) the forward's
  * decode routing would use for `p` (0 = the call is not routed to split-KV).
  * The automatic path cuts each sequence's KV into fixed-length chunks (about
- * 18 work items per CU) rather than a fixed number of splits per sequence,
+ * 18 work items of one wave per CU, or 3 of one workgroup on short streams) rather than a fixed number of splits per sequence,
  * so ragged KV lengths stay balanced; with a window each sequence gets a
  * fixed number of equal splits of its window band instead (slots =
  * num_seqs * splits). Retunes src/ext.mm:372-388. */

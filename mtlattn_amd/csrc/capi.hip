@@ -168,10 +168,25 @@ struct PagedKV {
     int page_size;
 };
 
+// How a decode call cuts its KV (decode_plan, short_plan, paged_plan).
+struct DecodePlan {
+    int chunk = 0;    // > 0: fixed KV chunks of this many keys
+    int ns = 0;       // > 0: equal splits per sequence over the window band
+    int wg = 0;       // waves of one workgroup per item (0: one wave per item)
+    bool routed() const { return chunk > 0 || ns > 0; }
+    // whole sequences in one workgroup each: no partials
+    bool whole() const { return wg > 0 && chunk == 0 && ns == 1; }
+};
+
+size_t plan_bytes(const mtlattn_problem* p, const DecodePlan& plan) {
+    return plan.whole() ? 0 : splitkv_bytes(p, plan.ns, plan.chunk);
+}
+
 int run_splitkv(const mtlattn_problem* p, const void* q, int64_t qrs, const void* k, int64_t krs, const void* v,
-                int64_t vrs, void* out, float* lse, int ns, int chunk, void* ws, size_t ws_bytes, hipStream_t st,
+                int64_t vrs, void* out, float* lse, const DecodePlan& plan, void* ws, size_t ws_bytes, hipStream_t st,
                 const PagedKV* paged = nullptr) {
-    const size_t need = splitkv_bytes(p, ns, chunk);
+    const int ns = plan.ns, chunk = plan.chunk;
+    const size_t need = plan_bytes(p, plan);
     if (ws_bytes < need || (ws == nullptr && need > 0))
         return fail(MTLATTN_ERR_WORKSPACE, "mtlattn: split-KV workspace too small (%zu < %zu bytes)", ws_bytes,
                     need);
@@ -185,6 +200,7 @@ int run_splitkv(const mtlattn_problem* p, const void* q, int64_t qrs, const void
     a.num_splits = ns;
     a.chunk = chunk;
     a.max_q = p->max_seqlen_q;
+    a.wg = plan.wg;
     if (paged != nullptr) {
         a.block_table = paged->block_table;
         a.bt_stride = paged->bt_stride;
@@ -206,19 +222,24 @@ int run_splitkv(const mtlattn_problem* p, const void* q, int64_t qrs, const void
 // the work items and the workspace scale with the band, not the KV length.
 constexpr int64_t kItemsPerCu = 18;
 
-struct DecodePlan {
-    int chunk = 0;    // > 0: fixed KV chunks of this many keys
-    int ns = 0;       // > 0: equal splits per sequence over the window band
-    bool routed() const { return chunk > 0 || ns > 0; }
-};
+// One workgroup per item where the whole stream is short (below kWgBytes of K
+// and V, about 0.2 ms): chunks of at least 512 keys, 3 items per CU; above it
+// one wave per item, whose two tiles in flight stream up to 7% faster
+// (decode.hip; at 1.0 GB 206 against 211 us, at 0.4 GB 104 against 88).
+constexpr int64_t kWgBytes = 900ll << 20, kWgItemsPerCu = 3;
+
+// Work items when every sequence is one.
+int64_t decode_groups(const mtlattn_problem* p) {
+    const int g = p->num_heads_q / p->num_heads_kv;
+    return (int64_t)p->num_heads_kv * (g / decode_heads_per_group(g, p->max_seqlen_q));
+}
 
 // Chunk length (keys, a multiple of 256 in [256, 8192]) for `work` keys of
 // work per (kv head, head group).
-int64_t plan_chunk(const mtlattn_problem* p, int64_t work) {
-    const int g = p->num_heads_q / p->num_heads_kv;
-    const int64_t groups = (int64_t)p->num_heads_kv * (g / decode_heads_per_group(g, p->max_seqlen_q));
-    const int64_t items = (int64_t)device_cus() * kItemsPerCu;
-    int64_t c = (work * groups + items - 1) / items;
+int64_t plan_chunk(const mtlattn_problem* p, int64_t work, int64_t items_per_cu = kItemsPerCu) {
+    const int64_t items = (int64_t)device_cus() * items_per_cu;
+    int64_t c = (work * decode_groups(p) + items - 1) / items;
+    if (items_per_cu == kWgItemsPerCu && c < 512) c = 512;
     if (const char* e = std::getenv("MTLATTN_DECODE_CHUNK")) {   // tuning override (keys)
         const long v = std::strtol(e, nullptr, 10);
         if (v > 0) c = v;
@@ -237,17 +258,45 @@ int64_t band_keys(const mtlattn_problem* p, int64_t kv) {
     return kv < band ? kv : band;
 }
 
+// Fixed chunks of `work` keys in all, for one wave or one workgroup per item.
+void plan_chunks(const mtlattn_problem* p, int64_t work, DecodePlan& plan) {
+    if (work * decode_groups(p) * p->head_dim * 4 < kWgBytes) {
+        plan.chunk = (int)plan_chunk(p, work, kWgItemsPerCu);
+        plan.wg = plan.chunk >= 1024 ? 4 : 8;
+    } else {
+        plan.chunk = (int)plan_chunk(p, work);
+    }
+}
+
+bool decode_allowed(const mtlattn_problem* p) {
+    return check_problem(p) == MTLATTN_OK && p->total_q > 0 && splitkv_supported(p) &&
+           !env_set("MTLATTN_NO_SPLITKV") && !force_generic();
+}
+
+// Few-query calls that decode_plan leaves: one workgroup per whole sequence
+// (and kv head), which needs no workspace. Waves share a sequence's keys where
+// the flash forward's walk over them is serial: 64 sequences of 256 keys, 32/8
+// heads 29 -> 14 us, one of 1024 27 -> 14, 32 of 64 keys 7.6 -> 7.4.
+DecodePlan short_plan(const mtlattn_problem* p) {
+    DecodePlan plan;
+    if (!decode_allowed(p)) return plan;
+    plan.ns = 1;
+    plan.wg = decode_groups(p) * p->num_seqs > device_cus() ? 4 : 8;
+    return plan;
+}
+
 DecodePlan decode_plan(const mtlattn_problem* p) {
     DecodePlan plan;
-    if (check_problem(p) != MTLATTN_OK) return plan;
-    if (p->total_q <= 0 || env_set("MTLATTN_NO_SPLITKV") || force_generic() || !splitkv_supported(p)) return plan;
+    if (!decode_allowed(p)) return plan;
     const int64_t avg_kv = p->total_kv / (p->num_seqs > 0 ? p->num_seqs : 1);
     // keys a sequence's rows see on average (the window band at most)
     const int64_t band = (int64_t)p->window + p->max_seqlen_q - 1;
     const int64_t eff = p->window > 0 && avg_kv > band ? band : avg_kv;
-    if (eff < 2048) return plan;
+    // (few sequences: one workgroup per sequence would leave CUs idle; one of
+    // 2048 keys with 8 kv heads 23 us as a whole, 13 in chunks)
+    if (eff < (p->window <= 0 && decode_groups(p) * p->num_seqs <= 64 ? 1024 : 2048)) return plan;
     if (p->window <= 0) {
-        plan.chunk = (int)plan_chunk(p, p->total_kv);
+        plan_chunks(p, p->total_kv, plan);
     } else {
         // the splits must cover the longest band: W + q_len - 1 keys plus up
         // to 31 below its tile-aligned start
@@ -258,13 +307,18 @@ DecodePlan decode_plan(const mtlattn_problem* p) {
 }
 
 // Paged decode: the logical KV total is device data, p->total_kv bounds it.
-// Without a window, fixed chunks as on the contiguous path (slots for the
-// bound; chunks past a sequence's end exit at once); with one, equal splits
+// Without a window, whole sequences when they are short, else fixed chunks as
+// on the contiguous path (slots for the bound; chunks past a sequence's end exit at once); with one, equal splits
 // of the band sized for num_seqs bands of work.
 DecodePlan paged_plan(const mtlattn_problem* p, int64_t max_seqlen_kv) {
     DecodePlan plan;
     if (p->window <= 0) {
-        plan.chunk = (int)plan_chunk(p, p->total_kv > 0 ? p->total_kv : 1);
+        if (max_seqlen_kv <= 1024 || (max_seqlen_kv <= 2048 && decode_groups(p) * p->num_seqs > 64)) {
+            plan.ns = 1;
+            plan.wg = decode_groups(p) * p->num_seqs > device_cus() ? 4 : 8;
+        } else {
+            plan_chunks(p, p->total_kv > 0 ? p->total_kv : 1, plan);
+        }
         return plan;
     }
     const int64_t span = band_keys(p, max_seqlen_kv > 0 ? max_seqlen_kv : 1);
@@ -354,8 +408,8 @@ size_t fwd_part_bytes(const mtlattn_problem* p, int splits) {
 
 size_t mtlattn_varlen_fwd_workspace_size(const mtlattn_problem* p) {
     const DecodePlan plan = decode_plan(p);
-    if (plan.routed()) return splitkv_bytes(p, plan.ns, plan.chunk);
-    if (check_problem(p) != MTLATTN_OK) return 0;
+    if (plan.routed()) return plan_bytes(p, plan);
+    if (check_problem(p) != MTLATTN_OK || short_plan(p).routed()) return 0;
     return fwd_part_bytes(p, f32_fwd_splits(p));
 }
 
@@ -368,12 +422,15 @@ int mtlattn_varlen_fwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
     if (q == nullptr || out == nullptr || (p->total_kv > 0 && (k == nullptr || v == nullptr)))
         return fail(MTLATTN_ERR_INVALID, "mtlattn: null q/k/v/out pointer");
     hipStream_t st = (hipStream_t)stream;
-    const DecodePlan plan = decode_plan(p);
+    DecodePlan plan = decode_plan(p);
     const bool vec_ok = aligned16(q, q_row_stride, p->dtype) && aligned16(k, k_row_stride, p->dtype) &&
                         aligned16(v, v_row_stride, p->dtype) && ((uintptr_t)out & 15u) == 0;
+    // calls of fewer than 2048 keys a sequence run without a workspace too
+    if (!plan.routed() || (p->total_kv / p->num_seqs < 2048 && (workspace == nullptr || workspace_bytes < plan_bytes(p, plan))))
+        plan = short_plan(p);
     if (plan.routed() && vec_ok)
-        return run_splitkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, lse, plan.ns, plan.chunk,
-                           workspace, workspace_bytes, st);
+        return run_splitkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, lse, plan, workspace,
+                           workspace_bytes, st);
     FwdArgs a;
     a.geo = make_geo(p);
     a.q = q; a.q_rs = q_row_stride; a.k = k; a.k_rs = k_row_stride; a.v = v; a.v_rs = v_row_stride;
@@ -457,8 +514,9 @@ int f32_dq_splits(const mtlattn_problem* p) {
 
 // Split of the 16-bit matrix-core dK/dV
 DkvPlan dkv_plan(const mtlattn_problem* p) {
-    if (!is16(p->dtype) || force_generic()) return DkvPlan{};
-    return make_dkv_plan(make_geo(p), device_cus());
+    if (!is16(p->dtype)) return DkvPlan{};
+    const DkvPlan plan = make_dkv_plan(make_geo(p), device_cus());
+    return plan.pieces > 1 && force_generic() ? DkvPlan{} : plan;
 }
 
 // fp32 partial bytes after delta: 16-bit dK/dV's; or fp32 dQ's, then (in the
@@ -700,14 +758,16 @@ int mtlattn_attn_splitkv(const mtlattn_problem* p, const void* q, int64_t q_row_
     if (!aligned16(q, q_row_stride, p->dtype) || !aligned16(k, k_row_stride, p->dtype) ||
         !aligned16(v, v_row_stride, p->dtype) || ((uintptr_t)out & 15u) != 0)
         return fail(MTLATTN_ERR_UNSUPPORTED, "splitkv: q/k/v rows must be 16-byte aligned");
-    return run_splitkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, lse, num_splits, 0, workspace,
+    DecodePlan plan;
+    plan.ns = num_splits;
+    return run_splitkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, lse, plan, workspace,
                        workspace_bytes, (hipStream_t)stream);
 }
 
 size_t mtlattn_paged_decode_workspace_size(const mtlattn_problem* p, int64_t max_seqlen_kv) {
     if (check_problem(p) != MTLATTN_OK || !splitkv_supported(p)) return 0;
     const DecodePlan plan = paged_plan(p, max_seqlen_kv);
-    return splitkv_bytes(p, plan.ns, plan.chunk);
+    return plan_bytes(p, plan);
 }
 
 int mtlattn_paged_decode(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k_cache,
@@ -736,8 +796,8 @@ int mtlattn_paged_decode(const mtlattn_problem* p, const void* q, int64_t q_row_
         return fail(MTLATTN_ERR_UNSUPPORTED, "paged_decode: q/k/v rows must be 16-byte aligned");
     const DecodePlan plan = paged_plan(p, max_seqlen_kv);
     const PagedKV pk{block_table, block_table_stride, num_pages, page_size};
-    return run_splitkv(p, q, q_row_stride, k_cache, k_row_stride, v_cache, v_row_stride, out, lse, plan.ns,
-                       plan.chunk, workspace, workspace_bytes, (hipStream_t)stream, &pk);
+    return run_splitkv(p, q, q_row_stride, k_cache, k_row_stride, v_cache, v_row_stride, out, lse, plan, workspace,
+                       workspace_bytes, (hipStream_t)stream, &pk);
 }
 
 

@@ -339,6 +339,259 @@ __global__ __launch_bounds__(kDecWaves * 64) void decode_split_kernel(DecKParams
     }
 }
 
+// ---------------------------------------------------------------------------
+// Decode with the split inside the workgroup: one workgroup of NW waves per
+// work item (a sequence, or a KV chunk of it) and (kv head, head group). Wave
+// w takes the item's 32-key tiles w, w + NW, ...; the waves' unnormalised O,
+// row max and row sum meet in LDS. An item that is a whole sequence (chunk == 0
+// and ns == 1) writes its rows itself: one launch, no partials; else the
+// item's partial rows go to the combine kernel as above.
+//
+// Where the stream is short, the time is that of a few dependent loads: the
+// kernel above takes about 1 us per 32-key tile of a wave, whose items start
+// at 256 keys, plus the combine's launch; here a tile's latency is spread over
+// the NW waves (187 registers, so two waves per SIMD with one tile each in
+// flight) and short sequences need no second launch. Measured, bf16, D = 128,
+// one query per sequence, this kernel against what ran before: 16 sequences of
+// 1024 keys, 32/8 heads 37 -> 16 us; 64 of 2048 198 -> 102; one of 65536 (chunks)
+// 113 -> 63; 24 of 1024 to 8192 111 -> 101. On streams of a few hundred us and
+// more the kernel above, two tiles per wave in flight, is about 7% faster
+// (64 sequences of 8192 to 65536 keys, 64/8 heads: 1572 against 1713 us).
+// ---------------------------------------------------------------------------
+template <typename T, int D, bool BIAS, bool PAGED, int NW>
+__global__ __launch_bounds__(NW * 64) void decode_wg_kernel(DecKParams p, typename T::raw* __restrict__ out,
+                                                            float* __restrict__ lse_out) {
+    constexpr int KC = D / 32, DB = D / 16, VU = D / 64;
+    constexpr int OROW = D * 4 + 16;                 // bytes of an fp32 O row in LDS (padded: 16 rows, one column)
+    constexpr int REGION = 16 * OROW > D * kDecKT * 2 ? 16 * OROW : D * kDecKT * 2;   // per wave: V^T tile, then O
+    __shared__ __attribute__((aligned(16))) char smem[NW * REGION + NW * 32 * 4];
+    float* ml = reinterpret_cast<float*>(smem + NW * REGION);   // [NW][16] row max (log2), [NW][16] row sum
+
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n16 = lane & 15, lg = lane >> 4;
+    char* vt = smem + w * REGION;
+
+    int wid = blockIdx.x;
+    const int hk = wid % p.hkv; wid /= p.hkv;
+    const int hgi = wid % p.n_hg;
+    const int slot = wid / p.n_hg;
+    int s, ks, ke;
+    const bool has_keys = item_range(p, slot, s, ks, ke);
+    if (!has_keys && p.chunk > 0) return;
+    const SeqRange qr = seq_range(p.cu_q, s, p.total_q);
+    const SeqRange kr = seq_range(p.cu_kv, s, p.total_kv);
+    const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
+    if (q_len == 0) return;
+    const int coff = kv_len - q_len;
+
+    // (rows past the 16-row group, max_seqlen_q too small, are left untouched)
+    const int rows = min(p.hpb * q_len, 16);
+    const bool row_ok = n16 < rows;
+    const int hh = row_ok ? n16 / q_len : 0;
+    const int qi = row_ok ? n16 - hh * q_len : 0;
+    const int head = hk * p.g + hgi * p.hpb + hh;
+    const int64_t grow = qr.start + qi;
+
+    u32x4_t qf[KC];
+    {
+        const uint16_t* qp = p.q + grow * p.q_rs + (int64_t)head * D + 8 * lg;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) qf[kc] = ld16(qp + 32 * kc);
+    }
+    const int n_tiles = has_keys ? (ke - ks + kDecKT - 1) / kDecKT : 0;
+    const uint16_t* kbase = p.k + (PAGED ? 0 : (int64_t)kr.start * p.k_rs) + (int64_t)hk * D;
+    const uint16_t* vbase = p.v + (PAGED ? 0 : (int64_t)kr.start * p.v_rs) + (int64_t)hk * D;
+    const int* bt = PAGED ? p.block_table + (int64_t)s * p.bt_stride : nullptr;
+    auto page_row = [&](int key) -> int64_t {
+        const int col = min(key / p.page_size, (int)min(p.bt_stride, (int64_t)0x7fffffff) - 1);
+        const int pg = min(max(bt[col], 0), p.num_pages - 1);
+        return (int64_t)pg * p.page_size + key % p.page_size;
+    };
+    const float* brow = nullptr;
+    if (BIAS)
+        brow = p.bias + bias_row_offset(grow, s, qr.start, p.bias_qs, p.bias_ss, p.bias_rows) +
+               (int64_t)head * p.bias_hs;
+
+    u32x4_t ka[2][KC], vr[VU][4];
+    float bb[2][4];
+    auto load = [&](int kt) {
+        int64_t r0 = 0, r1 = 0;
+        if (PAGED) {
+            r0 = page_row(kt);
+            r1 = page_row(min(kt + 16, ke - 1));
+        }
+        auto row = [&](int key) -> int64_t {
+            if (!PAGED) return key;
+            return key < kt + 16 ? r0 + (key - kt) : r1 + (key - (kt + 16));
+        };
+        if (BIAS) {
+            if (p.bias_v4 && kt + kDecKT <= p.bias_cols) {
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) {
+                    const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(brow + kt + 16 * mb + 4 * lg);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bb[mb][r] = b4[r];
+                }
+            } else {
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = kt + 16 * mb + 4 * lg + r;
+                        const float b = brow[min(key, (int)p.bias_cols - 1)];
+                        bb[mb][r] = key < p.bias_cols ? b : 0.f;
+                    }
+            }
+        }
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+            const int key = min(kt + 16 * mb + n16, ke - 1);
+            const uint16_t* kp = kbase + row(key) * p.k_rs + 8 * lg;
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) ka[mb][kc] = ld16(kp + 32 * kc);
+        }
+#pragma unroll
+        for (int u = 0; u < VU; ++u) {
+            const int uid = lane + 64 * u;
+            const int dc = uid % (D / 8), kg = uid / (D / 8);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int key = min(kt + 4 * kg + i, ke - 1);
+                vr[u][i] = ld16(vbase + row(key) * p.v_rs + 8 * dc);
+            }
+        }
+    };
+
+    float m_run = kNegInf, l_run = 0.f;
+    f32x4_t oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    if (w < n_tiles) load(ks + w * kDecKT);
+    for (int it = w; it < n_tiles; it += NW) {
+        const int kt = ks + it * kDecKT;
+        f32x4_t sc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) {
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) sc[mb] = mfma16<T>(ka[mb][kc], qf[kc], sc[mb]);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < VU; ++u) {
+            const int uid = lane + 64 * u;
+            const int dc = uid % (D / 8), kg = uid / (D / 8);
+            u32x2_t tr[8];
+            transpose4x8(vr[u], tr);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) st8(vt + dec_tr_offset(8 * dc + i, kg), tr[i]);
+        }
+        float bt4[2][4];
+        if (BIAS) {
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bt4[mb][r] = bb[mb][r];
+        }
+        if (it + NW < n_tiles) load(kt + NW * kDecKT);
+
+        const bool need_mask = (kt + kDecKT > ke) || (p.causal && kt + kDecKT - 1 > coff) ||
+                               (p.window > 0 && kt < coff + q_len - p.window);
+        float mx = kNegInf;
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = kt + 16 * mb + 4 * lg + r;
+                bool ok = row_ok;
+                if (need_mask) {
+                    ok = ok && key < ke;
+                    if (p.causal) ok = ok && key <= qi + coff;
+                    if (p.window > 0) ok = ok && key > qi + coff - p.window;
+                }
+                float x = sc[mb][r] * p.scale_log2;
+                if (BIAS) x = fmaf(bt4[mb][r], kLog2e, x);
+                x = ok ? x : kNegInf;
+                sc[mb][r] = x;
+                mx = fmaxf(mx, x);
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = m_new == kNegInf ? 0.f : m_new;
+        const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
+        m_run = m_new;
+        float ls = 0.f;
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = __builtin_amdgcn_exp2f(sc[mb][r] - m_use);
+                ls += e;
+                sc[mb][r] = e;
+            }
+        }
+        l_run = l_run * corr + ls;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[db] *= corr;
+        const u32x4_t pf = u32x4_t{T::pack2(sc[0][0], sc[0][1]), T::pack2(sc[0][2], sc[0][3]),
+                                   T::pack2(sc[1][0], sc[1][1]), T::pack2(sc[1][2], sc[1][3])};
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            const int d = 16 * db + n16;
+            const u32x2_t x0 = ld8(vt + dec_tr_offset(d, lg));
+            const u32x2_t x1 = ld8(vt + dec_tr_offset(d, 4 + lg));
+            oacc[db] = mfma16<T>(u32x4_t{x0[0], x0[1], x1[0], x1[1]}, pf, oacc[db]);
+        }
+    }
+
+    // the wave's rows to LDS: O (lane: row n16, columns 16 db + 4 lg ..), max, sum
+    float lt = l_run + __shfl_xor(l_run, 16);
+    lt += __shfl_xor(lt, 32);
+    __builtin_amdgcn_wave_barrier();
+    if (row_ok) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            *reinterpret_cast<f32x4_t*>(vt + n16 * OROW + (16 * db + 4 * lg) * 4) = oacc[db];
+        if (lg == 0) {
+            ml[w * 16 + n16] = m_run;
+            ml[(NW + w) * 16 + n16] = lt;
+        }
+    }
+    __syncthreads();
+    const bool whole = p.chunk == 0 && p.ns == 1;
+    // one thread per row and 4 columns
+    for (int u = threadIdx.x; u < rows * (D / 4); u += NW * 64) {
+        const int n = u / (D / 4), d = 4 * (u - n * (D / 4));
+        float m = kNegInf;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) m = nan_max(ml[i * 16 + n], m);
+        const float m_use = m == kNegInf ? 0.f : m;
+        float l = 0.f;
+        f32x4_t o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const float wgt = __builtin_amdgcn_exp2f(ml[i * 16 + n] - m_use);
+            l += wgt * ml[(NW + i) * 16 + n];
+            o += wgt * *reinterpret_cast<const f32x4_t*>(smem + i * REGION + n * OROW + d * 4);
+        }
+        o *= !(l <= 0.f) ? 1.f / l : 0.f;
+        const float lse = !(l <= 0.f) ? m * kLn2 + logf(l) : kNegInf;
+        if (whole) {
+            const int h2 = n / q_len;
+            const int64_t rh = (int64_t)(qr.start + n - h2 * q_len) * p.hq + hk * p.g + hgi * p.hpb + h2;
+            st8(out + rh * D + d, u32x2_t{T::pack2(o[0], o[1]), T::pack2(o[2], o[3])});
+            if (lse_out != nullptr && d == 0) lse_out[rh] = lse;
+        } else {
+            const int64_t prow = ((int64_t)(hk * p.n_hg + hgi) * p.n_slots + slot) * 16 + n;
+            *reinterpret_cast<f32x4_t*>(p.o_part + prow * D + d) = o;
+            if (d == 0) p.lse_part[prow] = lse;
+        }
+    }
+}
+
 // One wave per (row, head): O = sum_i w_i O_i / sum_i w_i over the work items
 // of the row's sequence, w_i = exp(lse_i - max lse). Rows outside every
 // sequence, or beyond the 16-row group (max_seqlen_q too small), are left
@@ -422,6 +675,22 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecKParams p, typen
     if (lse_out != nullptr && lane == 0) lse_out[rh] = !(wsum <= 0.f) ? m + logf(wsum) : kNegInf;
 }
 
+template <typename T, int D, int NW>
+hipError_t launch_wg(const DecodeArgs& a, const DecKParams& p, bool paged, int64_t items, hipStream_t st) {
+    if (items > 0x7fffffff) return hipErrorInvalidValue;
+    if (items <= 0) return hipSuccess;
+    const dim3 grid((unsigned)items), block(NW * 64);
+    typename T::raw* out = (typename T::raw*)a.o;
+    if (p.bias != nullptr) {
+        if (paged) hipLaunchKernelGGL((decode_wg_kernel<T, D, true, true, NW>), grid, block, 0, st, p, out, a.lse);
+        else hipLaunchKernelGGL((decode_wg_kernel<T, D, true, false, NW>), grid, block, 0, st, p, out, a.lse);
+    } else {
+        if (paged) hipLaunchKernelGGL((decode_wg_kernel<T, D, false, true, NW>), grid, block, 0, st, p, out, a.lse);
+        else hipLaunchKernelGGL((decode_wg_kernel<T, D, false, false, NW>), grid, block, 0, st, p, out, a.lse);
+    }
+    return hipGetLastError();
+}
+
 template <typename T, int D>
 hipError_t launch_typed(const DecodeArgs& a, hipStream_t st) {
     const Geometry& g = a.geo;
@@ -460,7 +729,10 @@ hipError_t launch_typed(const DecodeArgs& a, hipStream_t st) {
     const int64_t waves = (int64_t)g.hkv * p.n_hg * p.n_slots;
     const int64_t blocks = (waves + kDecWaves - 1) / kDecWaves;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    if (blocks > 0) {
+    if (a.wg != 0) {
+        hipError_t e = a.wg == 8 ? launch_wg<T, D, 8>(a, p, paged, waves, st) : launch_wg<T, D, 4>(a, p, paged, waves, st);
+        if (e != hipSuccess || (p.chunk == 0 && p.ns == 1)) return e;
+    } else if (blocks > 0) {
         const dim3 grid((unsigned)blocks), block(kDecWaves * 64);
         if (p.bias != nullptr) {
             if (paged) hipLaunchKernelGGL((decode_split_kernel<T, D, true, true>), grid, block, 0, st, p);

@@ -92,6 +92,8 @@ struct DecodeArgs {
     int num_splits;               // equal splits per sequence (used when chunk == 0)
     int chunk;                    // > 0: fixed KV chunk length (multiple of 32)
     int max_q;                    // bound on q lengths; heads_per_group * max_q <= 16
+    int wg = 0;                   // 4 or 8: one workgroup of that many waves per item, not one wave;
+                                  // with chunk == 0 and num_splits == 1 it writes o and lse, no partials
     // paged KV: k / v are caches [num_pages, page_size, hkv, d] (row strides
     // k_rs / v_rs per token), logical key j of sequence s in page
     // block_table[s * bt_stride + j / page_size]; block_table == nullptr:

@@ -1,0 +1,79 @@
+"""The forward's work splits on small grids: one-workgroup decode (whole
+sequences, and chunks of a short stream), against the oracle."""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+import oracle
+from mtlattn_amd import capi
+from tests.helpers import LSE_TOL, REF_ATOL, cu_of, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(q_lens, kv_lens, Hq, Hkv, D, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    return (randn((sum(q_lens), Hq, D), dtype, g), randn((sum(kv_lens), Hkv, D), dtype, g),
+            randn((sum(kv_lens), Hkv, D), dtype, g))
+
+
+def _fwd(q, k, v, cq, ck, max_q, causal, window, bias, workspace):
+    """(out, lse, workspace bytes) of mtlattn_varlen_fwd on NaN-filled outputs,
+    with the queried workspace (NaN-filled) or none."""
+    Hq, D, Hkv = q.shape[1], q.shape[2], k.shape[1]
+    p = capi.problem_for(q, k, cq, ck, max_q, 1.0 / math.sqrt(D), causal=causal, window=window, bias=bias)
+    need = capi.lib().mtlattn_varlen_fwd_workspace_size(ctypes.byref(p))
+    n = need if workspace else 0
+    ws = torch.full((max(n // 4, 1),), float("nan"), dtype=torch.float32, device="cuda")
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((q.shape[0], Hq), float("nan"), dtype=torch.float32, device="cuda")
+    capi.call("mtlattn_varlen_fwd", p, q.data_ptr(), Hq * D, k.data_ptr(), Hkv * D, v.data_ptr(), Hkv * D,
+              out.data_ptr(), lse.data_ptr(), ws.data_ptr() if n else None, n, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return out.cpu(), lse.cpu(), need
+
+
+def _check(name, out, lse, ref, ref_lse, dtype):
+    fin = torch.isfinite(ref_lse)
+    assert torch.equal(torch.isfinite(lse), fin), f"{name}: LSE -inf pattern"
+    assert torch.isfinite(out.float()).all(), name
+    assert (out.float() - ref).abs().max().item() < REF_ATOL[dtype], name
+    assert (lse[fin] - ref_lse[fin]).abs().max().item() < LSE_TOL[dtype], name
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,causal,window,bias", [
+    ([1] * 9, [1, 31, 32, 33, 127, 128, 129, 0, 1000], 8, 2, 128, torch.bfloat16, True, 0, None),
+    ([1, 0, 4, 16, 7], [300, 50, 9, 16, 513], 16, 2, 128, torch.float16, True, 0, None),
+    ([3, 5], [260, 700], 12, 12, 64, torch.bfloat16, False, 0, None),
+    ([1] * 70, list(range(1, 281, 4)), 32, 8, 64, torch.float16, True, 0, None),       # more than one item per CU
+    ([1, 2, 1], [900, 1500, 40], 8, 8, 128, torch.bfloat16, True, 100, None),
+    ([2, 1], [700, 333], 16, 4, 128, torch.float16, True, 0, "head"),
+    ([1, 3], [530, 1200], 8, 2, 64, torch.bfloat16, True, 300, "broadcast"),
+    ([1], [1999], 8, 2, 128, torch.bfloat16, True, 0, None),                            # few sequences: chunks
+    ([2, 1], [5000, 2047], 16, 16, 128, torch.float16, True, 0, None),
+    ([1], [40000], 8, 2, 64, torch.bfloat16, True, 0, None),
+])
+def test_decode_workgroup(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window, bias):
+    """Few-query calls on one workgroup per item: key counts around a tile and
+    around the waves' share, empty sequences, rows with no key (more queries
+    than keys), head groups of several rows, windows, biases, chunked calls.
+    O and LSE against the oracle; a call without a workspace (whole sequences)
+    where fewer than 2048 keys a sequence allow one."""
+    print(f"\n[case] decode workgroup D={D} {dtype} {q_lens[:5]} {kv_lens[:9]} window={window} bias={bias}", flush=True)
+    q, k, v = _inputs(q_lens, kv_lens, Hq, Hkv, D, dtype, 3)
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    b = None
+    if bias:
+        b = torch.randn(sum(q_lens), 1 if bias == "broadcast" else Hq, max(kv_lens),
+                        generator=torch.Generator().manual_seed(4))
+    ref, ref_lse = oracle.varlen_forward(q, k, v, cq, ck, 1.0 / math.sqrt(D), causal, window, b)
+    dev = [t.cuda() for t in (q, k, v, cq, ck)]
+    bd = None if b is None else b.cuda()
+    for ws in (True, False):
+        if not ws and sum(kv_lens) // len(kv_lens) >= 2048:
+            continue
+        out, lse, need = _fwd(*dev, max(q_lens), causal, window, bd, ws)
+        _check(f"workspace={ws} ({need} bytes)", out, lse, ref, ref_lse, dtype)
