@@ -106,7 +106,8 @@ int mtlattn_gpu_core_count(int device);
  *   lse : NULL or fp32 [total_q, Hq] (rows with no allowed key get -inf)
  * Workspace: the split-KV partials of calls routed to decode (few-query calls
  * of fewer than 2048 keys a sequence run without one, one workgroup per
- * sequence and kv head); for fp32
+ * sequence and kv head); fp32 partials of O and the LSE for fp16/bf16 problems
+ * with few query rows against many keys (none needed: unsplit); for fp32
  * problems on the fp32 matrix-core kernels whose grid would leave CUs idle,
  * fp32 partials of 2-8 key splits (a smaller workspace runs them unsplit);
  * otherwise none.

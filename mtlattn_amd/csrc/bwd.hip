@@ -399,13 +399,13 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     const int pair = w & (NP - 1);
     SplitPiece pc{};
     if constexpr (SPLIT) {
-        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+        if (!dkv_piece<KB, QTL>(p, blockIdx.x, pc)) return;
     } else {
         const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-        pc.hk = L / p.n_tiles;
-        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+        pc.group = L / p.n_tiles;
+        pc.t = L - pc.group * p.n_tiles;                  // early key blocks (heavier when causal) first
     }
-    const int hk = pc.hk, t = pc.t;
+    const int hk = pc.group, t = pc.t;
     const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
     const int tb = tile_base(p.cu_kv, s, KB, p.total_kv);
     if (t < tb) return;
@@ -869,13 +869,13 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     const int l32 = lane & 31, hi = lane >> 5;
     SplitPiece pc{};
     if constexpr (SPLIT) {
-        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+        if (!dkv_piece<KB, QTL>(p, blockIdx.x, pc)) return;
     } else {
         const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-        pc.hk = L / p.n_tiles;
-        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+        pc.group = L / p.n_tiles;
+        pc.t = L - pc.group * p.n_tiles;                  // early key blocks (heavier when causal) first
     }
-    const int hk = pc.hk, t = pc.t;
+    const int hk = pc.group, t = pc.t;
     const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
     const int tb = tile_base(p.cu_kv, s, KB, p.total_kv);
     if (t < tb) return;
@@ -1446,7 +1446,7 @@ DkvPlan make_dkv_plan(const Geometry& g, int cus) {
             for (int64_t b = 0; b < nb; ++b) x += std::max<int64_t>(1, (n[b] + c - 1) / c);
             return x * heads;
         };
-        int64_t c = std::max<int64_t>(kSplitMinPiece, (n_max + max_pieces - 1) / max_pieces);
+        int64_t c = std::max<int64_t>(kDkvMinPiece, (n_max + max_pieces - 1) / max_pieces);
         while (c < n_max && wgs(c) > r * slots) ++c;
         const double t = (r == 1 ? (double)c : (double)work / (double)slots + 0.5 * (double)c) + cost * r +
                          cost * (double)wgs(c) / (double)slots;

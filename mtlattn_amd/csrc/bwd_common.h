@@ -43,99 +43,27 @@ __device__ inline QWalk query_walk(int k0, int kb, int coff, int q_len, int kv_l
     return QWalk{q_lo, q_hi > q_lo ? (q_hi - q_lo + qtl - 1) / qtl : 0};
 }
 
-// A split dK/dV launch cuts each key block's stages into pieces of `piece`
-// stages (the last one shorter), one workgroup each; pieces start at the same
-// distances from the top of the walk in every block, so workgroups that run
-// together read the same query tiles.
-__device__ inline int split_pieces(int n, int piece) { return max(1, (n + piece - 1) / piece); }
 // Offset of dK's (which = 0) or dV's (1) partial rows of piece z.
 __device__ inline int64_t part_offset(int z, int which, int64_t total_kv, int64_t row) {
     return (2 * (int64_t)z + which) * total_kv * row;
 }
 
-// The piece of workgroup `id` of a split launch: key tile t (KB keys, a
-// sequence's tiles as find_seq_for_tile numbers them) of kv head hk, its
-// piece z, stages [st0, st0 + n). Every wave finds it by itself from cu_seqlens: lane l holds
-// the stage counts of tiles l + 64 i, the piece length is the smallest whose
-// pieces fit the grid (and at least kSplitMinPiece stages, at most max_pieces
-// pieces per block), and the pieces are numbered by a scan over the lanes.
-// The host keeps n_tiles <= 64 kSplitChunks and n_tiles * hkv <= split_grid.
-constexpr int kSplitChunks = 4, kSplitMinPiece = 8;
-struct SplitPiece {
-    int t, hk, z, st0, n;
-};
+// The piece of workgroup `id` of a split dK/dV launch (find_piece): pieces of
+// the query stages of key tile t (KB keys) of kv head `group`. Pieces start at
+// the same distances from the top of the walk in every block, so workgroups
+// that run together read the same query tiles.
+constexpr int kDkvMinPiece = 8;
 template <int KB, int QTL>
-__device__ inline bool split_piece(const BwdKParams& p, int id, SplitPiece& out) {
-    const int lane = threadIdx.x & 63;
-    int n[kSplitChunks], n_max = 0;                  // stages per tile; -1: no such tile
-#pragma unroll
-    for (int i = 0; i < kSplitChunks; ++i) {
-        n[i] = -1;
-        const int t = lane + 64 * i;
-        if (64 * i >= p.n_tiles) continue;
-        if (t < p.n_tiles) {
-            const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
-            const SeqRange qr = seq_range(p.cu_q, s, p.total_q), kr = seq_range(p.cu_kv, s, p.total_kv);
-            const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
-            const int blk = t - tile_base(p.cu_kv, s, KB, p.total_kv);
-            if (blk >= 0 && blk * KB < kv_len)
-                n[i] = query_walk(blk * KB, KB, kv_len - q_len, q_len, kv_len, p.causal, p.window, QTL).n_tiles * p.g;
-        }
-        n_max = max(n_max, n[i]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) n_max = max(n_max, __shfl_xor(n_max, o));
-    // pieces of all tiles at piece length c
-    auto count = [&](int c) {
-        int x = 0;
-#pragma unroll
-        for (int i = 0; i < kSplitChunks; ++i)
-            if (64 * i < p.n_tiles && n[i] >= 0) x += split_pieces(n[i], c);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-        return __builtin_amdgcn_readfirstlane(x);
+__device__ inline bool dkv_piece(const BwdKParams& p, int id, SplitPiece& out) {
+    auto stages = [&](int t) {
+        const int s = find_seq_for_tile(p.cu_kv, p.num_seqs, KB, t, p.total_kv);
+        const SeqRange qr = seq_range(p.cu_q, s, p.total_q), kr = seq_range(p.cu_kv, s, p.total_kv);
+        const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
+        const int blk = t - tile_base(p.cu_kv, s, KB, p.total_kv);
+        if (blk < 0 || blk * KB >= kv_len) return -1;
+        return query_walk(blk * KB, KB, kv_len - q_len, q_len, kv_len, p.causal, p.window, QTL).n_tiles * p.g;
     };
-    const int fit = p.split_grid / p.hkv;
-    int c = max(kSplitMinPiece, (n_max + p.max_pieces - 1) / p.max_pieces), total = count(c);
-    if (total > fit) {
-        int lo = c, hi = max(c + 1, n_max);          // lo does not fit, hi (one piece per tile) does
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (count(mid) > fit) lo = mid; else hi = mid;
-        }
-        c = hi;
-        total = count(c);
-    }
-    c = __builtin_amdgcn_readfirstlane(c);
-    if (id == 0 && threadIdx.x == 0) *p.piece_out = c;
-    if (id >= total * p.hkv) return false;
-    const int L = xcd_remap(id, total * p.hkv);
-    out.hk = L / total;
-    int r = L - out.hk * total;
-#pragma unroll
-    for (int i = 0; i < kSplitChunks; ++i) {
-        if (64 * i >= p.n_tiles) break;
-        const int np = n[i] >= 0 ? split_pieces(n[i], c) : 0;
-        int sum = np;                                // inclusive scan
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(sum, o);
-            if (lane >= o) sum += y;
-        }
-        const unsigned long long past = __ballot(sum > r);
-        if (past != 0) {
-            const int l = __builtin_ctzll(past);
-            const int z = r - __builtin_amdgcn_readlane(sum - np, l);
-            const int m = __builtin_amdgcn_readlane(n[i], l);
-            out.t = 64 * i + l;
-            out.z = z;
-            out.st0 = z * c;
-            out.n = min(c, m - out.st0);
-            return true;
-        }
-        r -= __builtin_amdgcn_readlane(sum, 63);
-    }
-    return false;
+    return find_piece(stages, p.n_tiles, p.hkv, p.split_grid, kDkvMinPiece, p.max_pieces, p.piece_out, id, out);
 }
 
 // Sum of the 8 products of one 16-byte chunk of O and dO. The preprocess and

@@ -83,13 +83,13 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
     const int l32 = lane & 31, hi = lane >> 5;
     SplitPiece pc{};
     if constexpr (SPLIT) {
-        if (!split_piece<KB, QTL>(p, blockIdx.x, pc)) return;
+        if (!dkv_piece<KB, QTL>(p, blockIdx.x, pc)) return;
     } else {
         const int L = xcd_remap(blockIdx.x, p.n_tiles * p.hkv);
-        pc.hk = L / p.n_tiles;
-        pc.t = L - pc.hk * p.n_tiles;                  // early key blocks (heavier when causal) first
+        pc.group = L / p.n_tiles;
+        pc.t = L - pc.group * p.n_tiles;                  // early key blocks (heavier when causal) first
     }
-    const int hk = pc.hk, t = pc.t;
+    const int hk = pc.group, t = pc.t;
     // Tiles are pairs of key blocks, block pi and block nb - 1 - pi of a
     // sequence (nb blocks): with causal masking a pair's work is the same
     // for every pair, so the in-order dispatch of workgroups keeps the CUs

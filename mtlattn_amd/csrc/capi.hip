@@ -400,6 +400,15 @@ int f32_fwd_splits(const mtlattn_problem* p) {
     return ns >= 2 ? (int)ns : 1;
 }
 
+// Split of the 16-bit flash forward over its key tiles; its scratch fits the
+// no-allocation entry's, so that mtlattn_varlen_fwd_noalloc splits alike.
+FwdPlan fwd_plan(const mtlattn_problem* p) {
+    if (!is16(p->dtype)) return FwdPlan{};
+    const FwdPlan plan =
+        make_fwd_plan(make_geo(p), p->max_seqlen_q, device_cus(), (size_t)MTLATTN_NOALLOC_SCRATCH_BYTES);
+    return plan.grid > 0 && force_generic() ? FwdPlan{} : plan;
+}
+
 size_t fwd_part_bytes(const mtlattn_problem* p, int splits) {
     return (size_t)f32_fwd_part_floats(splits, p->total_q, p->num_heads_q, p->head_dim) * sizeof(float);
 }
@@ -410,6 +419,7 @@ size_t mtlattn_varlen_fwd_workspace_size(const mtlattn_problem* p) {
     const DecodePlan plan = decode_plan(p);
     if (plan.routed()) return plan_bytes(p, plan);
     if (check_problem(p) != MTLATTN_OK || short_plan(p).routed()) return 0;
+    if (is16(p->dtype)) return fwd_plan(p).bytes;
     return fwd_part_bytes(p, f32_fwd_splits(p));
 }
 
@@ -436,8 +446,16 @@ int mtlattn_varlen_fwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
     a.q = q; a.q_rs = q_row_stride; a.k = k; a.k_rs = k_row_stride; a.v = v; a.v_rs = v_row_stride;
     a.o = out; a.lse = lse;
     if (is16(p->dtype) && mfma_head_dim(p->head_dim) && vec_ok && tile_stride_ok(k_row_stride) &&
-        tile_stride_ok(v_row_stride) && !force_generic())
+        tile_stride_ok(v_row_stride) && !force_generic()) {
+        // (a workspace smaller than the size query asks for runs unsplit)
+        const FwdPlan split = fwd_plan(p);
+        if (split.grid > 0 && workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 &&
+            workspace_bytes >= split.bytes) {
+            a.plan = split;
+            a.split_ws = workspace;
+        }
         return launch_status(launch_fwd_mfma(p->dtype, a, st), "flash forward");
+    }
     if (p->dtype == MTLATTN_DTYPE_F32 && f32_mfma_head_dim(p->head_dim) && vec_ok && !force_generic()) {
         // split partials in the workspace when it holds them (the size query
         // counts them); a smaller workspace runs unsplit

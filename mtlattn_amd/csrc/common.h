@@ -547,4 +547,94 @@ __device__ inline int xcd_remap(int id, int n) {
     return (id & 7) * (n >> 3) + (id >> 3);
 }
 
+// ---------------------------------------------------------------------------
+// Split launches: on grids that would leave CUs idle, the sequential work of
+// each tile (its steps: key tiles of the forward, query stages of dK/dV) is
+// cut into pieces of `piece` steps, the last one shorter, one workgroup each.
+// ---------------------------------------------------------------------------
+__device__ inline int split_pieces(int n, int piece) { return max(1, (n + piece - 1) / piece); }
+
+struct SplitPiece {
+    int t, group, z, id;   // tile, head group, piece of the tile, number of the piece (all groups)
+    int st0, n;            // its steps [st0, st0 + n)
+    int pieces;            // of its tile
+};
+
+// The piece of workgroup `id` of a split launch, found by every wave from
+// steps(t), the steps of tile t (-1: no such tile): lane l holds tiles
+// l + 64 i, the piece length is the smallest (at least min_piece, at most
+// max_pieces pieces per tile) whose pieces fit `grid` workgroups, and the
+// pieces are numbered by a scan over the lanes, so that no workgroup between
+// them is empty (empty ones between the others left some shader engines with
+// two rounds of work: dK/dV at 1 x 2048 131 us with 240 pieces, 103 numbered
+// densely with more). Workgroup 0 writes the length for the pass that merges
+// the pieces. The host keeps n_tiles <= 64 kSplitChunks and
+// n_tiles * groups <= grid. About 1 us of each workgroup.
+constexpr int kSplitChunks = 4;
+template <typename F>
+__device__ inline bool find_piece(F steps, int n_tiles, int groups, int grid, int min_piece, int max_pieces,
+                                  int* piece_out, int id, SplitPiece& out) {
+    const int lane = threadIdx.x & 63;
+    int n[kSplitChunks], n_max = 0;
+#pragma unroll
+    for (int i = 0; i < kSplitChunks; ++i) {
+        n[i] = -1;
+        if (64 * i >= n_tiles) continue;
+        if (lane + 64 * i < n_tiles) n[i] = steps(lane + 64 * i);
+        n_max = max(n_max, n[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n_max = max(n_max, __shfl_xor(n_max, o));
+    // pieces of all tiles of a group at piece length c
+    auto count = [&](int c) {
+        int x = 0;
+#pragma unroll
+        for (int i = 0; i < kSplitChunks; ++i)
+            if (64 * i < n_tiles && n[i] >= 0) x += split_pieces(n[i], c);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+        return __builtin_amdgcn_readfirstlane(x);
+    };
+    const int fit = grid / groups;
+    int c = max(min_piece, (n_max + max_pieces - 1) / max_pieces), total = count(c);
+    if (total > fit) {
+        int lo = c, hi = max(c + 1, n_max);          // lo does not fit, hi (one piece per tile) does
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (count(mid) > fit) lo = mid; else hi = mid;
+        }
+        c = hi;
+        total = count(c);
+    }
+    c = __builtin_amdgcn_readfirstlane(c);
+    if (id == 0 && threadIdx.x == 0) *piece_out = c;
+    if (id >= total * groups) return false;
+    out.id = xcd_remap(id, total * groups);
+    out.group = out.id / total;
+    int r = out.id - out.group * total;
+#pragma unroll
+    for (int i = 0; i < kSplitChunks; ++i) {
+        if (64 * i >= n_tiles) break;
+        const int np = n[i] >= 0 ? split_pieces(n[i], c) : 0;
+        int sum = np;                                // inclusive scan
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(sum, o);
+            if (lane >= o) sum += y;
+        }
+        const unsigned long long past = __ballot(sum > r);
+        if (past != 0) {
+            const int l = __builtin_ctzll(past);
+            out.t = 64 * i + l;
+            out.z = r - __builtin_amdgcn_readlane(sum - np, l);
+            out.pieces = __builtin_amdgcn_readlane(np, l);
+            out.st0 = out.z * c;
+            out.n = min(c, __builtin_amdgcn_readlane(n[i], l) - out.st0);
+            return true;
+        }
+        r -= __builtin_amdgcn_readlane(sum, 63);
+    }
+    return false;
+}
+
 }  // namespace mtlattn

@@ -26,6 +26,7 @@
 //     sliding-window cost is O(W) (src/attn_mpp.metal:216-225).
 //   * Varlen tiles are numbered without a host sync (common.h), blocks are
 //     remapped so neighbouring query tiles of one (sequence, head) share an XCD.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -53,7 +54,37 @@ struct FwdKParams {
     int causal, window;
     int bias_v4;      // bias rows 16-byte aligned (pointer and strides)
     int col0;         // first output (and V) column of this launch
+    // SPLIT launches: workgroup grid, the piece length it works with, the
+    // number of each (head group, tile)'s first piece, and per piece its rows'
+    // normalised fp32 O and natural-log LSE (NW * 32 rows)
+    int split_grid;
+    int* piece_out; int* first;
+    float* part_o; float* part_lse;
 };
+
+// Key tiles [lo, lo + n KT) that the query rows q0 .. q0 + qt - 1 of a
+// sequence can see.
+struct KvTiles {
+    int lo, n;
+};
+template <int KT>
+__device__ inline KvTiles key_tiles(int q0, int qt, int q_len, int kv_len, int causal, int window) {
+    const int coff = kv_len - q_len;
+    const int q_last = min(q_len, q0 + qt) - 1;
+    const int hi = causal ? min(kv_len, q_last + coff + 1) : kv_len;
+    int lo = 0;
+    if (window > 0) {
+        lo = max(0, q0 + coff - window + 1);
+        lo = (lo / KT) * KT;
+    }
+    return KvTiles{lo, hi > lo ? (hi - lo + KT - 1) / KT : 0};
+}
+
+// Shortest piece of a split launch, in keys: below it the merge costs more
+// than the shorter walk saves (a 64-key tile takes about 1.2 us).
+constexpr int kFwdMinPieceKeys = 1024;
+// make_fwd_plan: the cost of starting and merging pieces, in 64-key tiles
+constexpr double kFwdSplitCost = 10.;
 
 // Softmax modes (SM). 0: no bias, scale > 0: the running max is taken over
 // raw scores and the scale folded into one FMA per element. 1: bias,
@@ -71,8 +102,13 @@ struct FwdKParams {
 // workgroup covers BROWS query rows; each key tile's bias block is staged in
 // the LDS ring with the K/V tiles (read from LDS by all waves of all heads)
 // instead of every wave loading its rows from global memory.
-template <typename T, int DK, int DV, int DVL, int DO, int SM, int BROWS = 0, int KT = kKT, int NW = kWaves, int NBUF = 3>
+// SPLIT (grids that leave CUs idle, make_fwd_plan): a workgroup takes one
+// piece of one tile's key tiles; pieces of tiles cut in several write their
+// rows' O and LSE as fp32 for fwd_merge_kernel.
+template <typename T, int DK, int DV, int DVL, int DO, int SM, int BROWS = 0, int KT = kKT, int NW = kWaves, int NBUF = 3,
+          bool SPLIT = false>
 __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKParams p) {
+    static_assert(!SPLIT || (SM == 0 && DO == DV), "split: no bias, all columns in one launch");
     static_assert(KT == 64 || ((KT == 32 || KT == 128) && BROWS == 0), "32- and 128-key tiles: no staged bias");
     constexpr int NKB = KT / 32;             // 32-key blocks per tile
     constexpr int NPC = KT / 16;             // 16-key P chunks per tile
@@ -95,9 +131,25 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
     const int l32 = lane & 31, hi = lane >> 5;
     const int QT = 32 * (NW / p.hpw);
-    const int L = xcd_remap(blockIdx.x, p.n_tiles * p.n_hg);
-    const int hg = L / p.n_tiles;
-    const int t = p.n_tiles - 1 - (L - hg * p.n_tiles);   // late (heavier) tiles first
+    SplitPiece pc{};
+    if constexpr (SPLIT) {
+        auto tiles = [&](int t) {
+            const int s = find_seq_for_tile(p.cu_q, p.num_seqs, QT, t, p.total_q);
+            const SeqRange qr = seq_range(p.cu_q, s, p.total_q), kr = seq_range(p.cu_kv, s, p.total_kv);
+            const int q0 = (t - tile_base(p.cu_q, s, QT, p.total_q)) * QT;
+            if (q0 < 0 || q0 >= qr.end - qr.start) return -1;
+            return key_tiles<KT>(q0, QT, qr.end - qr.start, kr.end - kr.start, p.causal, p.window).n;
+        };
+        if (!find_piece(tiles, p.n_tiles, p.n_hg, p.split_grid, kFwdMinPieceKeys / KT, 0x7fffffff, p.piece_out,
+                        blockIdx.x, pc))
+            return;
+        if (pc.z == 0 && threadIdx.x == 0) p.first[pc.group * p.n_tiles + pc.t] = pc.id;
+    } else {
+        const int L = xcd_remap(blockIdx.x, p.n_tiles * p.n_hg);
+        pc.group = L / p.n_tiles;
+        pc.t = p.n_tiles - 1 - (L - pc.group * p.n_tiles);   // late (heavier) tiles first
+    }
+    const int hg = pc.group, t = pc.t;
     const int s = find_seq_for_tile(p.cu_q, p.num_seqs, QT, t, p.total_q);
     const int tb = tile_base(p.cu_q, s, QT, p.total_q);
     if (t < tb) return;
@@ -129,15 +181,10 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
         wait_vmcnt<0>();
     }
 
-    // Key range of the whole workgroup.
-    const int q_last_wg = min(q_len, q0 + QT) - 1;
-    const int kv_hi = p.causal ? min(kv_len, q_last_wg + coff + 1) : kv_len;
-    int kv_lo = 0;
-    if (p.window > 0) {
-        kv_lo = max(0, q0 + coff - p.window + 1);
-        kv_lo = (kv_lo / KT) * KT;
-    }
-    const int n_kv_tiles = kv_hi > kv_lo ? (kv_hi - kv_lo + KT - 1) / KT : 0;
+    // Key tiles of the whole workgroup.
+    const KvTiles kts = key_tiles<KT>(q0, QT, q_len, kv_len, p.causal, p.window);
+    const int kv_lo = SPLIT ? kts.lo + pc.st0 * KT : kts.lo;
+    const int n_kv_tiles = SPLIT ? pc.n : kts.n;
 
     const uint16_t* kbase = p.k + (int64_t)kr.start * p.k_rs + (int64_t)hk * DV;
     const uint16_t* vbase = p.v + (int64_t)kr.start * p.v_rs + (int64_t)hk * DV + p.col0;
@@ -454,6 +501,24 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
     const float lt = pair_sum(l_run);
     if (wave_active && qrow < q_len) {
         const float inv = !(lt <= 0.f) ? 1.f / lt : 0.f;
+        if constexpr (SPLIT) {
+            if (pc.pieces > 1) {
+                const int64_t row = (int64_t)pc.id * (NW * 32) + w * 32 + l32;
+                float* op = p.part_o + row * DV;
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int rg = 0; rg < 4; ++rg) {
+                        const int d = 32 * db + 8 * rg + 4 * hi;
+                        if (DO % 32 != 0 && d >= DO) continue;
+                        *reinterpret_cast<f32x4_t*>(op + d) =
+                            f32x4_t{oacc[db][4 * rg + 0], oacc[db][4 * rg + 1], oacc[db][4 * rg + 2],
+                                    oacc[db][4 * rg + 3]} * inv;
+                    }
+                if (hi == 0) p.part_lse[row] = !(lt <= 0.f) ? m_run * kLn2 + logf(lt) : kNegInf;
+                return;
+            }
+        }
         uint16_t* op = p.o + (int64_t)(qr.start + qrow) * ((int64_t)p.hq * DV) + (int64_t)head * DV + p.col0;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
@@ -470,6 +535,64 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
     }
 }
 
+// Merges the pieces of the tiles that a split launch cut: one wave per row of
+// a piece's NW * 32 (a query row of one head), lanes over the head dim,
+// O = sum_z w_z O_z / sum_z w_z with w_z = exp(lse_z - max lse) in piece
+// order, and the row's LSE. Bound by the partials' bytes.
+template <typename T, int DV, int KT>
+__global__ __launch_bounds__(256) void fwd_merge_kernel(FwdKParams p, int nw) {
+    constexpr int NJ = (DV + 63) / 64;
+    const int lane = threadIdx.x & 63;
+    const int rows = 32 * nw, wph = nw / p.hpw, QT = 32 * wph;
+    const int tile = blockIdx.x;                                 // (head group, tile)
+    const int hg = tile / p.n_tiles, t = tile - hg * p.n_tiles;
+    const int s = find_seq_for_tile(p.cu_q, p.num_seqs, QT, t, p.total_q);
+    const SeqRange qr = seq_range(p.cu_q, s, p.total_q), kr = seq_range(p.cu_kv, s, p.total_kv);
+    const int q_len = qr.end - qr.start;
+    const int q0 = (t - tile_base(p.cu_q, s, QT, p.total_q)) * QT;
+    if (q0 < 0 || q0 >= q_len) return;
+    const int pieces =
+        split_pieces(key_tiles<KT>(q0, QT, q_len, kr.end - kr.start, p.causal, p.window).n, *p.piece_out);
+    if (pieces == 1) return;
+    const int64_t first = p.first[tile];
+    for (int rr = blockIdx.y * 4 + (threadIdx.x >> 6); rr < rows; rr += 4 * gridDim.y) {
+        const int w = rr >> 5;
+        const int qrow = q0 + 32 * (w % wph) + (rr & 31);
+        if (qrow >= q_len) continue;
+        const int64_t rh = (int64_t)(qr.start + qrow) * p.hq + hg * p.hpw + w / wph;
+        // (NaN-preserving: a row whose pieces are all NaN must not look empty)
+        float m = kNegInf;
+        for (int z = lane; z < pieces; z += 64) m = nan_max(p.part_lse[(first + z) * rows + rr], m);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = nan_max(m, __shfl_xor(m, o));
+        float acc[NJ], wsum = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[j] = 0.f;
+        if (m != kNegInf) {
+#pragma unroll 4
+            for (int z = 0; z < pieces; ++z) {
+                const int64_t row = (first + z) * rows + rr;
+                const float l = p.part_lse[row];
+                const float wgt = l == kNegInf ? 0.f : __expf(l - m);
+                wsum += wgt;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const int d = lane + 64 * j;
+                    const float o = DV % 64 == 0 || d < DV ? p.part_o[row * DV + d] : 0.f;
+                    acc[j] += l == kNegInf ? 0.f : wgt * o;
+                }
+            }
+        }
+        const float inv = !(wsum <= 0.f) ? 1.f / wsum : 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int d = lane + 64 * j;
+            if (DV % 64 == 0 || d < DV) p.o[rh * DV + d] = T::from_float(acc[j] * inv);
+        }
+        if (p.lse != nullptr && lane == 0) p.lse[rh] = !(wsum <= 0.f) ? m + logf(wsum) : kNegInf;
+    }
+}
+
 int gcd_int(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
 
 // CUs of the current device (cached per device; 256 if unknown)
@@ -483,6 +606,38 @@ int device_cus() {
         cache[dev] = n;
     }
     return cache[dev];
+}
+
+// The split variant of each head dim: the same tiles as its unsplit kernel on
+// small grids (4-wave workgroups, two per CU, at D = 64 and 128).
+template <int DK, int DV>
+struct SplitCfg {
+    static constexpr int NW = DV == 64 || DV == 128 ? 4 : kWaves;
+    static constexpr int KT = NW == 4 ? 64 : DK == 128 ? 128 : DV <= 192 ? 64 : 32;
+    static constexpr int NBUF = DV == 256 ? 3 : 2;
+};
+
+template <typename T, int DK, int DV>
+hipError_t launch_split(const FwdArgs& a, FwdKParams p, hipStream_t st) {
+    using C = SplitCfg<DK, DV>;
+    const FwdPlan& plan = a.plan;
+    p.hpw = plan.hpw;
+    p.n_tiles = plan.n_tiles;
+    p.n_hg = a.geo.hq / plan.hpw;
+    p.split_grid = plan.grid;
+    p.col0 = 0;
+    p.piece_out = (int*)a.split_ws;
+    p.first = p.piece_out + 64;
+    const size_t ints = ((size_t)p.n_tiles * p.n_hg + 64 + 63) / 64 * 64;
+    p.part_o = (float*)a.split_ws + ints;
+    p.part_lse = p.part_o + (size_t)plan.grid * C::NW * 32 * DV;
+    hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 0, 0, C::KT, C::NW, C::NBUF, true>), dim3((unsigned)plan.grid),
+                       dim3(C::NW * 64), 0, st, p);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((fwd_merge_kernel<T, DV, C::KT>), dim3((unsigned)(p.n_tiles * p.n_hg), 8), dim3(256), 0, st, p,
+                       C::NW);
+    return hipGetLastError();
 }
 
 template <typename T, int DK, int DV, int DVL, int DO>
@@ -506,6 +661,7 @@ hipError_t launch_typed(const FwdArgs& a, hipStream_t st) {
     p.causal = g.causal; p.window = g.window > 0 ? g.window : 0;
     p.bias_v4 = g.bias != nullptr && ((uintptr_t)g.bias % 16 == 0) && g.bias_qs % 4 == 0 && g.bias_hs % 4 == 0 &&
                 (g.bias_ss < 0 || g.bias_ss % 4 == 0);
+    if (a.plan.grid > 0 && a.split_ws != nullptr) return launch_split<T, DK, DV>(a, p, st);
     const int64_t blocks = (int64_t)p.n_tiles * p.n_hg;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
@@ -624,6 +780,71 @@ hipError_t launch_dims(const FwdArgs& a, hipStream_t st) {
         case 256: return launch_typed<T, 256, 256, 128, 128>(a, st);
         default: return hipErrorInvalidValue;
     }
+}
+
+// A chunk of a long prompt, or a few queries against a long cache, has few
+// row tiles that each walk thousands of keys one after the other: there the
+// tiles' keys are cut into pieces of at least 1024, one workgroup each, which
+// fp32 partials of O and the LSE merge. Forward before -> after, bf16 causal,
+// 32/8 heads, D = 128: 512 queries against 8192 keys 148 -> 88 us, 32 against
+// 16384 383 -> 40, 2 x 512 against 8192 to 32768 419 -> 308, 1024 against
+// 32768 771 -> 520 (1.06 PFLOP/s); 8 x 17 against 3000 76 -> 39. The line: the
+// split has to save 15% of the walk by this count of key tiles on sequences of
+// the average length, with kFwdSplitCost for the pieces' start and the merge's
+// launch (at 1 x 1500 causal, 384 unsplit workgroups, it lost, 45 -> 56 us).
+FwdPlan make_fwd_plan(const Geometry& g, int max_q, int cus, size_t max_bytes) {
+    FwdPlan none, plan;
+    if (!mfma_head_dim(g.d) || g.bias != nullptr || !(g.scale > 0.f) || g.total_q <= 0 || g.total_kv <= 0) return none;
+    const int nw = g.d == 64 || g.d == 128 ? 4 : kWaves;
+    const int kt = nw == 4 ? 64 : g.d < 128 ? 128 : g.d == 160 ? 64 : 32, min_piece = kFwdMinPieceKeys / kt;
+    const int64_t lq = (g.total_q + g.num_seqs - 1) / g.num_seqs, lk = (g.total_kv + g.num_seqs - 1) / g.num_seqs;
+    if (lk <= kFwdMinPieceKeys) return none;
+    // heads per workgroup: more where a sequence's rows fill few waves
+    int hpw = gcd_int(g.g, nw == 4 ? (max_q > 0 && max_q <= 32 ? 4 : 2) : kWaves);
+    const int qt = 32 * (nw / hpw), rows = 32 * nw;
+    plan.nw = nw;
+    plan.hpw = hpw;
+    const int64_t n_tiles = g.total_q / qt + g.num_seqs + 1, n_hg = g.hq / hpw;
+    if (n_tiles > 64 * kSplitChunks) return none;
+    plan.n_tiles = (int)n_tiles;
+    // key tiles of the row tiles of a sequence of average length
+    const int64_t nt = (lq + qt - 1) / qt, coff = lk - lq, units = nt * g.num_seqs * n_hg;
+    int64_t n[64 * kSplitChunks + 1], n_max = 0, work = 0;
+    for (int64_t i = 0; i < nt; ++i) {
+        const int64_t last = std::min(lq, (i + 1) * qt) - 1;
+        const int64_t hi = g.causal ? std::min(lk, last + coff + 1) : lk;
+        const int64_t lo = g.window > 0 ? std::max<int64_t>(0, i * qt + coff - g.window + 1) / kt * kt : 0;
+        n[i] = hi > lo ? (hi - lo + kt - 1) / kt : 0;
+        n_max = std::max(n_max, n[i]);
+        work += n[i] * g.num_seqs * n_hg;
+    }
+    // time in key tiles: two 4-wave workgroups on a CU take 1.5x as long as one
+    const double pair = nw == 4 ? 1.5 : 1.;
+    const int64_t slots = (int64_t)cus * (nw == 4 ? 2 : 1);
+    const double unsplit = units <= cus ? (double)n_max
+                                        : std::max(pair * (double)n_max, 1.1 * pair * (double)work / (double)slots);
+    double best = 0.85 * unsplit;
+    const int64_t ints = (n_tiles * n_hg + 64 + 63) / 64 * 64;
+    for (int64_t full = cus; full <= slots; full += cus) {
+        // (as many workgroups as the scratch holds)
+        const int64_t grid = std::min(full, ((int64_t)(max_bytes / sizeof(float)) - ints) / (rows * (g.d + 1)) / 8 * 8);
+        if (n_tiles * n_hg > grid) continue;
+        const size_t bytes = (size_t)(ints + grid * rows * (g.d + 1)) * sizeof(float);
+        auto wgs = [&](int64_t c) {
+            int64_t x = 0;
+            for (int64_t i = 0; i < nt; ++i) x += std::max<int64_t>(1, (n[i] + c - 1) / c);
+            return x * g.num_seqs * n_hg;
+        };
+        int64_t c = min_piece;
+        while (c < n_max && wgs(c) > grid) ++c;
+        const double t = (double)c * (wgs(c) <= cus ? 1. : pair) + kFwdSplitCost * 64. / kt;
+        if (c < n_max && t < best) {
+            best = t;
+            plan.grid = (int)grid;
+            plan.bytes = bytes;
+        }
+    }
+    return plan.grid > 0 ? plan : none;
 }
 
 hipError_t launch_fwd_mfma(int dtype, const FwdArgs& a, hipStream_t st) {

@@ -22,6 +22,15 @@ struct Geometry {
     int64_t bias_rows = 0;        // rows per sequence block when bias_ss >= 0
 };
 
+// How the 16-bit flash forward cuts its work (make_fwd_plan): grid == 0: one
+// workgroup per tile of query rows; else `grid` workgroups take pieces of the
+// tiles' key tiles, merged afterwards.
+struct FwdPlan {
+    int grid = 0, nw = 0, hpw = 0, n_tiles = 0;   // waves and heads per workgroup, row tiles
+    size_t bytes = 0;                             // workspace
+};
+FwdPlan make_fwd_plan(const Geometry& g, int max_q, int cus, size_t max_bytes);
+
 struct FwdArgs {
     Geometry geo;
     const void* q; int64_t q_rs;
@@ -34,6 +43,9 @@ struct FwdArgs {
     // their LSEs in f32_part (f32_fwd_part_floats floats), then merged
     float* f32_part = nullptr;
     int f32_splits = 1;
+    // 16-bit flash forward only: split as plan says, with plan.bytes of scratch
+    FwdPlan plan;
+    void* split_ws = nullptr;
 };
 
 // How the 16-bit dK/dV cuts its work (make_dkv_plan): pieces == 1: one

@@ -1,5 +1,6 @@
 """The forward's work splits on small grids: one-workgroup decode (whole
-sequences, and chunks of a short stream), against the oracle."""
+sequences, and chunks of a short stream) and the flash forward's key pieces,
+against the oracle and against the unsplit flash forward."""
 
 import ctypes
 import math
@@ -77,3 +78,34 @@ def test_decode_workgroup(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window, bi
             continue
         out, lse, need = _fwd(*dev, max(q_lens), causal, window, bd, ws)
         _check(f"workspace={ws} ({need} bytes)", out, lse, ref, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,causal,window", [
+    ([512, 130], [4096, 9000], 8, 2, 128, torch.bfloat16, True, 0),
+    ([32], [6000], 16, 2, 128, torch.float16, True, 0),
+    ([17, 0, 65], [3000, 5, 5000], 8, 8, 64, torch.bfloat16, True, 0),
+    ([100], [5001], 12, 12, 64, torch.float16, False, 0),
+    ([257], [4100], 8, 2, 128, torch.bfloat16, True, 2100),
+    ([70, 40], [4097, 3071], 8, 2, 80, torch.float16, True, 0),
+    ([60], [5000], 8, 8, 96, torch.bfloat16, False, 0),
+    ([90], [3500], 8, 2, 160, torch.bfloat16, True, 0),
+    ([1, 65], [4000, 2999], 8, 2, 256, torch.float16, True, 0),
+])
+def test_forward_key_pieces(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window):
+    """The flash forward on row tiles too few for the GPU cuts their keys into
+    pieces (with the queried workspace) and merges them; without a workspace it
+    runs unsplit. Row and key remainders, an empty sequence, keys below one
+    piece, a window, every head dim's kernel; NaN in the workspace and trailing
+    rows that no sequence owns stay out; equal on a second call, bitwise."""
+    print(f"\n[case] forward key pieces D={D} {dtype} {q_lens} {kv_lens} window={window}", flush=True)
+    q, k, v = _inputs(q_lens, kv_lens, Hq, Hkv, D, dtype, 5)
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    ref, ref_lse = oracle.varlen_forward(q, k, v, cq, ck, 1.0 / math.sqrt(D), causal, window)
+    n = q.shape[0]
+    dev = [torch.cat([q, q[:3]]).cuda(), torch.cat([k, k[:3]]).cuda(), torch.cat([v, v[:3]]).cuda(), cq.cuda(), ck.cuda()]
+    runs = [_fwd(*dev, max(q_lens), causal, window, None, ws) for ws in (True, True, False)]
+    assert runs[0][2] > 0, "expected a split workspace for this small grid"
+    for out, lse, _ in runs:
+        _check("pieces", out[:n], lse[:n], ref, ref_lse, dtype)
+        assert out[n:].isnan().all() and lse[n:].isnan().all(), "rows outside every sequence were written"
+    assert torch.equal(runs[0][0][:n], runs[1][0][:n]) and torch.equal(runs[0][1][:n], runs[1][1][:n])
