@@ -176,6 +176,26 @@ int mtlattn_varlen_bwd(const mtlattn_problem* p,
                        void* stream);
 
 /*
+ * The backward above with row strides (elements) for dq and for dk and dv, so
+ * that the gradients of a packed qkv or kv tensor are written in place. No
+ * counterpart in the reference (its wrappers stack the three). fp16/bf16 on
+ * the matrix-core kernels with 8-byte aligned rows; otherwise
+ * MTLATTN_ERR_UNSUPPORTED before anything is launched. Same workspace,
+ * kernels and values as mtlattn_varlen_bwd.
+ */
+int mtlattn_varlen_bwd_strided(const mtlattn_problem* p,
+                               const void* q, int64_t q_row_stride,
+                               const void* k, int64_t k_row_stride,
+                               const void* v, int64_t v_row_stride,
+                               const void* out, int64_t out_row_stride,
+                               const void* dout, int64_t dout_row_stride,
+                               const float* lse,
+                               void* dq, int64_t dq_row_stride,
+                               void* dk, void* dv, int64_t dkv_row_stride,
+                               void* workspace, size_t workspace_bytes,
+                               void* stream);
+
+/*
  * delta[row, h] = sum_d dout[row, h, d] * out[row, h, d] in fp32.
  * Replaces the torch reduction at src/ext.mm:518 / bwd_delta_impl
  * (src/attention.metal:724-733). delta: fp32 [total_q, Hq].

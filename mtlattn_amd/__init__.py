@@ -70,6 +70,45 @@ class _VarlenAttnFn(torch.autograd.Function):
         return (*grads, None, None, None, None, None, None, None)
 
 
+class _QkvPackedAttnFn(torch.autograd.Function):
+    """Autograd node for a packed qkv [M, 3, H, D]: its gradient is written in
+    place by the backward kernels, not stacked from three tensors."""
+
+    @staticmethod
+    def forward(ctx, qkv, cu, max_q, scale, causal, window):
+        q, k, v = qkv.unbind(dim=1)
+        lse = torch.empty((q.shape[0], q.shape[1]), dtype=torch.float32, device=q.device)
+        out = _C.varlen_attention(q, k, v, cu, cu, max_q, scale, causal, window, lse)
+        ctx.save_for_backward(qkv, out, lse, cu)
+        ctx.args = (scale, causal, window)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        qkv, out, lse, cu = ctx.saved_tensors
+        d = _C.varlen_attention_bwd_qkvpacked(qkv, out, dout.contiguous(), lse, cu, *ctx.args)
+        return d, None, None, None, None, None
+
+
+class _KvPackedAttnFn(torch.autograd.Function):
+    """Autograd node for q and a packed kv [Mkv, 2, Hkv, D] (as above)."""
+
+    @staticmethod
+    def forward(ctx, q, kv, cu_q, cu_kv, max_q, scale, causal, window):
+        k, v = kv.unbind(dim=1)
+        lse = torch.empty((q.shape[0], q.shape[1]), dtype=torch.float32, device=q.device)
+        out = _C.varlen_attention(q, k, v, cu_q, cu_kv, max_q, scale, causal, window, lse)
+        ctx.save_for_backward(q, kv, out, lse, cu_q, cu_kv)
+        ctx.args = (scale, causal, window)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        q, kv, out, lse, cu_q, cu_kv = ctx.saved_tensors
+        dq, dkv = _C.varlen_attention_bwd_kvpacked(q, kv, out, dout.contiguous(), lse, cu_q, cu_kv, *ctx.args)
+        return dq, dkv, None, None, None, None, None, None
+
+
 def _prep_bias(attn_bias):
     """Bring an additive mask to the kernel contract (reference:
     mtlattn/__init__.py:49-63): fp32, 3-D, unit stride on the key dim. A 4-D
@@ -126,9 +165,13 @@ def flash_attn_varlen_qkvpacked_func(qkv, cu_seqlens, max_seqlen, softmax_scale=
                                      causal=False, window=0, **kwargs):
     """flash_attn-style entry, qkv: [M, 3, H, D] (reference:
     mtlattn/__init__.py:104-110). Differentiable; q/k/v are row-strided views."""
+    window = _window_from_kwargs(window, kwargs)
+    if torch.is_grad_enabled() and qkv.requires_grad:
+        scale = 1.0 / math.sqrt(qkv.shape[-1]) if softmax_scale is None else softmax_scale
+        return _QkvPackedAttnFn.apply(qkv, cu_seqlens.int(), int(max_seqlen), float(scale), bool(causal), int(window))
     q, k, v = qkv.unbind(dim=1)
     return varlen_attention(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, softmax_scale,
-                            causal=causal, window=_window_from_kwargs(window, kwargs))
+                            causal=causal, window=window)
 
 
 def flash_attn_varlen_kvpacked_func(q, kv, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
@@ -136,9 +179,14 @@ def flash_attn_varlen_kvpacked_func(q, kv, cu_seqlens_q, cu_seqlens_k, max_seqle
                                     **kwargs):
     """flash_attn-style entry, q: [Mq, H, D], kv: [Mkv, 2, Hkv, D] (reference:
     mtlattn/__init__.py:113-120). Differentiable."""
+    window = _window_from_kwargs(window, kwargs)
+    if torch.is_grad_enabled() and (q.requires_grad or kv.requires_grad):
+        scale = 1.0 / math.sqrt(q.shape[-1]) if softmax_scale is None else softmax_scale
+        return _KvPackedAttnFn.apply(q, kv, cu_seqlens_q.int(), cu_seqlens_k.int(), int(max_seqlen_q), float(scale),
+                                     bool(causal), int(window))
     k, v = kv.unbind(dim=1)
     return varlen_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_scale,
-                            causal=causal, window=_window_from_kwargs(window, kwargs))
+                            causal=causal, window=window)
 
 
 def paged_decode(q, k_cache, v_cache, cu_seqlens_q, cu_seqlens_kv, block_table, max_seqlen_q,

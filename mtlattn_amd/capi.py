@@ -56,6 +56,8 @@ SIGNATURES = {
     "mtlattn_varlen_bwd_workspace_size": (_sz, [_P]),
     "mtlattn_varlen_bwd": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp,
                                           _vp, _vp, _vp, _vp, _sz, _vp]),
+    "mtlattn_varlen_bwd_strided": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp,
+                                                  _vp, _i64, _vp, _vp, _i64, _vp, _sz, _vp]),
     "mtlattn_bwd_preprocess": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _vp]),
     "mtlattn_bwd_dq": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _vp]),
     "mtlattn_bwd_dkv": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i32,

@@ -323,7 +323,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void bwd_dq_kernel(BwdKParams p) {
     }
 
     if (wave_active && row_ok) {
-        const int64_t off = grow * ((int64_t)p.hq * DV) + (int64_t)head * DV + C0;
+        const int64_t off = grow * p.dq_rs + (int64_t)head * DV + C0;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_dkv_kernel(BwdKParams p) {
     }
 
     if (pair_active && key_ok) {
-        const int64_t row = (int64_t)p.hkv * DV;
+        const int64_t row = SPLIT ? (int64_t)p.hkv * DV : p.dkv_rs;
         const int64_t off = (int64_t)(kr.start + key) * row + (int64_t)hk * DV + c0;
         void* dst = role_a ? p.dv : p.dk;
         if constexpr (SPLIT) dst = p.part + part_offset(pc.z, role_a ? 1 : 0, p.total_kv, row);
@@ -1091,7 +1091,7 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     }
 
     if (wave_active && key_ok) {
-        const int64_t row = (int64_t)p.hkv * DV;
+        const int64_t row = SPLIT ? (int64_t)p.hkv * DV : p.dkv_rs;
         const int64_t off = (int64_t)(kr.start + key) * row + (int64_t)hk * DV;
         void* dk = SPLIT ? p.part + part_offset(pc.z, 0, p.total_kv, row) : p.dk;
         void* dv = SPLIT ? p.part + part_offset(pc.z, 1, p.total_kv, row) : p.dv;
@@ -1110,15 +1110,17 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void bwd_dkv_sym_kernel(BwdKP
     }
 }
 
-// Zero the rows of a [total_rows, row_halves] tensor of 16-bit halves outside
-// [first, last), with all threads of grid x.
-__device__ inline void zero_outside(uint16_t* ptr, int64_t row_halves, int64_t total_rows, int64_t first, int64_t last) {
+// Zero the rows of a [total_rows, row_halves] tensor of 16-bit halves (row
+// stride rs) outside [first, last), with all threads of grid x.
+__device__ inline void zero_outside(uint16_t* ptr, int64_t row_halves, int64_t rs, int64_t total_rows, int64_t first,
+                                    int64_t last) {
     first = first < 0 ? 0 : (first > total_rows ? total_rows : first);
     last = last < first ? first : (last > total_rows ? total_rows : last);
-    const int64_t head_end = first * row_halves, tail_begin = last * row_halves, end = total_rows * row_halves;
-    const int64_t n = head_end + (end - tail_begin);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        ptr[i < head_end ? i : tail_begin + (i - head_end)] = 0;
+    const int64_t n = (first + (total_rows - last)) * row_halves;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t r = i / row_halves;
+        ptr[(r < first ? r : last + (r - first)) * rs + (i - r * row_halves)] = 0;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1131,14 +1133,14 @@ struct FinishKParams {
     const float* part;
     uint16_t* dq; uint16_t* dk; uint16_t* dv;
     const int* cu_q; const int* cu_kv;
-    int64_t total_q, total_kv, dq_row;
+    int64_t total_q, total_kv, dq_row, dq_rs, dkv_rs;
     const int* piece;              // the piece length the split launch worked with
     int num_seqs, row, g, causal, window, kb, qtl;
 };
 template <typename T>
 __global__ __launch_bounds__(256) void dkv_finish_kernel(FinishKParams p) {
     if (blockIdx.y == 1) {
-        zero_outside(p.dq, p.dq_row, p.total_q, p.cu_q[0], p.cu_q[p.num_seqs]);
+        zero_outside(p.dq, p.dq_row, p.dq_rs, p.total_q, p.cu_q[0], p.cu_q[p.num_seqs]);
         return;
     }
     const uint32_t units = (uint32_t)p.row / 4;                  // 4-column units of a row
@@ -1169,8 +1171,9 @@ __global__ __launch_bounds__(256) void dkv_finish_kernel(FinishKParams p) {
             for (int e = 0; e < 4; ++e) { k4[e] += a[e]; v4[e] += b[e]; }
         }
     }
-    store4<T, false>(p.dk, off, k4[0], k4[1], k4[2], k4[3]);
-    store4<T, false>(p.dv, off, v4[0], v4[1], v4[2], v4[3]);
+    const int64_t dst = r * p.dkv_rs + (off - (int64_t)r * p.row);
+    store4<T, false>(p.dk, dst, k4[0], k4[1], k4[2], k4[3]);
+    store4<T, false>(p.dv, dst, v4[0], v4[1], v4[2], v4[3]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1222,7 +1225,7 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const typename T::r
 // launch covers up to three tensors (blockIdx.y picks the job).
 struct ZeroJob {
     uint16_t* ptr;
-    int64_t row_halves, total_rows;
+    int64_t row_halves, rs, total_rows;
     const int* cu;
 };
 struct ZeroJobs {
@@ -1231,7 +1234,7 @@ struct ZeroJobs {
 };
 __global__ __launch_bounds__(256) void zero_outside_kernel(ZeroJobs jobs) {
     const ZeroJob& j = jobs.job[blockIdx.y];
-    zero_outside(j.ptr, j.row_halves, j.total_rows, j.cu[0], j.cu[jobs.num_seqs]);
+    zero_outside(j.ptr, j.row_halves, j.rs, j.total_rows, j.cu[0], j.cu[jobs.num_seqs]);
 }
 
 int gcd_int(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
@@ -1286,7 +1289,9 @@ hipError_t launch_finish(const BwdArgs& a, int kb, int qtl, hipStream_t st) {
     p.dq_row = (int64_t)g.hq * g.d;
     p.num_seqs = g.num_seqs; p.row = g.hkv * g.d; p.g = g.g;
     p.causal = g.causal; p.window = g.window > 0 ? g.window : 0;
-    p.kb = kb; p.qtl = qtl; p.piece = make_params(a).piece_out;
+    const BwdKParams b = make_params(a);
+    p.dq_rs = b.dq_rs; p.dkv_rs = b.dkv_rs;
+    p.kb = kb; p.qtl = qtl; p.piece = b.piece_out;
     const int64_t blocks = (g.total_kv * (p.row / 4) + 255) / 256;   // (make_dkv_plan bounds the partials)
     hipLaunchKernelGGL(dkv_finish_kernel<T>, dim3((unsigned)blocks, 2), dim3(256), 0, st, p);
     const hipError_t e = hipGetLastError();
@@ -1466,7 +1471,9 @@ hipError_t launch_zero_outside(const ZeroFill* fills, int n, int num_seqs, hipSt
     int used = 0;
     for (int i = 0; i < n && i < 3; ++i) {
         if (fills[i].total_rows <= 0 || fills[i].row_bytes <= 0) continue;
-        jobs.job[used++] = ZeroJob{(uint16_t*)fills[i].ptr, fills[i].row_bytes / 2, fills[i].total_rows, fills[i].cu};
+        jobs.job[used++] = ZeroJob{(uint16_t*)fills[i].ptr, fills[i].row_bytes / 2,
+                                   (fills[i].stride_bytes > 0 ? fills[i].stride_bytes : fills[i].row_bytes) / 2,
+                                   fills[i].total_rows, fills[i].cu};
     }
     if (used == 0) return hipSuccess;
     hipLaunchKernelGGL(zero_outside_kernel, dim3(64, used), dim3(256), 0, st, jobs);

@@ -12,6 +12,7 @@ struct BwdKParams {
     const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* dout;
     const float* lse; const float* delta;
     void* dq; void* dk; void* dv;
+    int64_t dq_rs, dkv_rs;             // their row strides
     const int* cu_q; const int* cu_kv;
     const float* bias;
     int64_t q_rs, k_rs, v_rs, do_rs;
@@ -124,6 +125,8 @@ BwdKParams make_params(const BwdArgs& a) {
     p.dout = (const uint16_t*)a.dout;
     p.lse = a.lse; p.delta = a.delta;
     p.dq = a.dq; p.dk = a.dk; p.dv = a.dv;
+    p.dq_rs = a.dq_rs > 0 ? a.dq_rs : (int64_t)g.hq * g.d;
+    p.dkv_rs = a.dkv_rs > 0 ? a.dkv_rs : (int64_t)g.hkv * g.d;
     p.cu_q = g.cu_q; p.cu_kv = g.cu_kv; p.bias = g.bias;
     p.q_rs = a.q_rs; p.k_rs = a.k_rs; p.v_rs = a.v_rs; p.do_rs = a.do_rs;
     p.bias_qs = g.bias_qs; p.bias_hs = g.bias_hs; p.bias_cols = g.bias_cols;

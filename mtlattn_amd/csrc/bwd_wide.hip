@@ -605,7 +605,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
 
         if (wave_active) {
             // (SPLIT: this piece's fp32 partials)
-            const int64_t row = (int64_t)p.hkv * DV;
+            const int64_t row = SPLIT ? (int64_t)p.hkv * DV : p.dkv_rs;
             void* dk = SPLIT ? p.part + part_offset(pc.z, 0, p.total_kv, row) : p.dk;
             void* dv = SPLIT ? p.part + part_offset(pc.z, 1, p.total_kv, row) : p.dv;
 #pragma unroll

@@ -599,10 +599,12 @@ bool bwd_f32_ok(const mtlattn_problem* p, const void* q, int64_t qrs, const void
 
 }  // namespace
 
-int mtlattn_bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k,
-                   int64_t k_row_stride, const void* v, int64_t v_row_stride, const void* dout,
-                   int64_t dout_row_stride, const float* lse, const float* delta, void* dq, int32_t dq_dtype,
-                   void* stream) {
+namespace {
+
+// mtlattn_bwd_dq with dq's row stride (16-bit matrix-core path only; 0: contiguous)
+int bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
+           const void* v, int64_t v_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
+           const float* delta, void* dq, int32_t dq_dtype, void* stream, int64_t dq_rs) {
     int rc = check_problem(p);
     if (rc != MTLATTN_OK) return rc;
     if (dq_dtype != MTLATTN_DTYPE_F32 && dq_dtype != p->dtype)
@@ -613,6 +615,7 @@ int mtlattn_bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride
         return fail(MTLATTN_ERR_INVALID, "mtlattn: null pointer argument");
     BwdArgs a = make_bwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta);
     a.dq = dq;
+    a.dq_rs = dq_rs;
     a.out_f32 = dq_dtype == MTLATTN_DTYPE_F32 ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     if (bwd_mfma_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride))
@@ -621,6 +624,16 @@ int mtlattn_bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride
         ((uintptr_t)dq & 15u) == 0)
         return launch_status(launch_bwd_dq_f32mfma(a, st), "fp32 dQ");
     return launch_status(launch_bwd_dq_generic(p->dtype, a, st), "generic dQ");
+}
+
+}  // namespace
+
+int mtlattn_bwd_dq(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k,
+                   int64_t k_row_stride, const void* v, int64_t v_row_stride, const void* dout,
+                   int64_t dout_row_stride, const float* lse, const float* delta, void* dq, int32_t dq_dtype,
+                   void* stream) {
+    return bwd_dq(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta, dq,
+                  dq_dtype, stream, 0);
 }
 
 namespace {
@@ -632,7 +645,8 @@ namespace {
 int bwd_dkv(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
             const void* v, int64_t v_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
             const float* delta, void* dk, void* dv, int32_t dkv_dtype, void* stream, float* part, int splits,
-            const DkvPlan& plan = DkvPlan{}, void* dq = nullptr, bool* cleared = nullptr) {
+            const DkvPlan& plan = DkvPlan{}, void* dq = nullptr, bool* cleared = nullptr, int64_t dq_rs = 0,
+            int64_t dkv_rs = 0) {
     int rc = check_problem(p);
     if (rc != MTLATTN_OK) return rc;
     if (dkv_dtype != MTLATTN_DTYPE_F32 && dkv_dtype != p->dtype)
@@ -647,6 +661,8 @@ int bwd_dkv(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const
     a.out_f32 = dkv_dtype == MTLATTN_DTYPE_F32 ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     if (bwd_mfma_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride)) {
+        a.dq_rs = dq_rs;
+        a.dkv_rs = dkv_rs;
         if (part != nullptr && plan.pieces > 1 && ((uintptr_t)dk & 7u) == 0 && ((uintptr_t)dv & 7u) == 0) {
             a.dq = dq;
             a.dkv_part = part;
@@ -674,10 +690,14 @@ int mtlattn_bwd_dkv(const mtlattn_problem* p, const void* q, int64_t q_row_strid
                    dkv_dtype, stream, nullptr, 1);
 }
 
-int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k,
-                       int64_t k_row_stride, const void* v, int64_t v_row_stride, const void* out,
-                       int64_t out_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
-                       void* dq, void* dk, void* dv, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+
+// mtlattn_varlen_bwd with the row strides of dq and of dk / dv (0: contiguous;
+// others on the 16-bit matrix-core path only)
+int varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride,
+               const void* v, int64_t v_row_stride, const void* out, int64_t out_row_stride, const void* dout,
+               int64_t dout_row_stride, const float* lse, void* dq, int64_t dq_rs, void* dk, void* dv, int64_t dkv_rs,
+               void* workspace, size_t workspace_bytes, void* stream) {
     int rc = check_problem(p);
     if (rc != MTLATTN_OK) return rc;
     // delta is required; the fp32 dK/dV partials after it are used when the
@@ -715,6 +735,7 @@ int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
             return fail(MTLATTN_ERR_INVALID, "mtlattn: null pointer argument");
         BwdArgs a = make_bwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta);
         a.dq = dq;
+        a.dq_rs = dq_rs;
         a.o = out;
         a.o_rs = out_row_stride;
         a.delta_out = delta;
@@ -738,21 +759,51 @@ int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_st
     } else if (p->total_q > 0) {
         rc = mtlattn_bwd_preprocess(p, out, out_row_stride, dout, dout_row_stride, delta, stream);
         if (rc != MTLATTN_OK) return rc;
-        rc = mtlattn_bwd_dq(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse,
-                            delta, dq, p->dtype, stream);
+        rc = bwd_dq(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta, dq,
+                    p->dtype, stream, dq_rs);
         if (rc != MTLATTN_OK) return rc;
     }
     rc = bwd_dkv(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta, dk, dv,
-                 p->dtype, stream, part, splits, plan, dq, &cleared);
+                 p->dtype, stream, part, splits, plan, dq, &cleared, dq_rs, dkv_rs);
     if (rc != MTLATTN_OK || cleared) return rc;
     // Rows outside every sequence take no part in the forward: zero gradient.
     hipStream_t st = (hipStream_t)stream;
     const int64_t es = elem_size(p->dtype);
     const int64_t qrow = (int64_t)p->num_heads_q * p->head_dim * es, krow = (int64_t)p->num_heads_kv * p->head_dim * es;
-    const ZeroFill fills[3] = {{dq, qrow, p->total_q, p->cu_seqlens_q},
-                               {dk, krow, p->total_kv, p->cu_seqlens_kv},
-                               {dv, krow, p->total_kv, p->cu_seqlens_kv}};
+    const ZeroFill fills[3] = {{dq, qrow, p->total_q, p->cu_seqlens_q, dq_rs * es},
+                               {dk, krow, p->total_kv, p->cu_seqlens_kv, dkv_rs * es},
+                               {dv, krow, p->total_kv, p->cu_seqlens_kv, dkv_rs * es}};
     return launch_status(launch_zero_outside(fills, 3, p->num_seqs, st), "gradient tail fill");
+}
+
+}  // namespace
+
+int mtlattn_varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k,
+                       int64_t k_row_stride, const void* v, int64_t v_row_stride, const void* out,
+                       int64_t out_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
+                       void* dq, void* dk, void* dv, void* workspace, size_t workspace_bytes, void* stream) {
+    return varlen_bwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, out_row_stride, dout, dout_row_stride,
+                      lse, dq, 0, dk, dv, 0, workspace, workspace_bytes, stream);
+}
+
+int mtlattn_varlen_bwd_strided(const mtlattn_problem* p, const void* q, int64_t q_row_stride, const void* k,
+                               int64_t k_row_stride, const void* v, int64_t v_row_stride, const void* out,
+                               int64_t out_row_stride, const void* dout, int64_t dout_row_stride, const float* lse,
+                               void* dq, int64_t dq_row_stride, void* dk, void* dv, int64_t dkv_row_stride,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+    int rc = check_problem(p);
+    if (rc != MTLATTN_OK) return rc;
+    const int64_t qrow = (int64_t)p->num_heads_q * p->head_dim, krow = (int64_t)p->num_heads_kv * p->head_dim;
+    if (dq_row_stride < qrow || dkv_row_stride < krow)
+        return fail(MTLATTN_ERR_INVALID, "mtlattn: gradient row strides must cover a row");
+    // the kernels store 8 bytes a lane
+    if (!bwd_mfma_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride) ||
+        ((uintptr_t)dq & 7u) != 0 || ((uintptr_t)dk & 7u) != 0 || ((uintptr_t)dv & 7u) != 0 || dq_row_stride % 4 != 0 ||
+        dkv_row_stride % 4 != 0)
+        return fail(MTLATTN_ERR_UNSUPPORTED, "mtlattn: strided gradients need the 16-bit matrix-core kernels and "
+                                             "8-byte aligned rows");
+    return varlen_bwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, out_row_stride, dout, dout_row_stride,
+                      lse, dq, dq_row_stride, dk, dv, dkv_row_stride, workspace, workspace_bytes, stream);
 }
 
 size_t mtlattn_attn_splitkv_workspace_size(const mtlattn_problem* p, int32_t num_splits) {

@@ -68,9 +68,12 @@ struct BwdArgs {
     const void* dout; int64_t do_rs;
     const float* lse;             // [total_q, hq]
     const float* delta;           // [total_q, hq]
-    void* dq;                     // contiguous [total_q, hq, d]
-    void* dk;                     // contiguous [total_kv, hkv, d]
+    void* dq;                     // [total_q, hq, d]
+    void* dk;                     // [total_kv, hkv, d]
     void* dv;
+    // 16-bit matrix-core kernels only: row strides of dq and of dk / dv
+    // (0: contiguous)
+    int64_t dq_rs = 0, dkv_rs = 0;
     int out_f32;                  // 1: dq/dk/dv are fp32, 0: input dtype
     // dQ only: with delta_out set, the dQ kernel computes delta = rowsum(dO * O)
     // itself from o (the forward's output) and writes it to delta_out for the
@@ -136,11 +139,13 @@ hipError_t launch_bwd_dkv_generic(int dtype, const BwdArgs& a, hipStream_t st);
 hipError_t launch_fwd_f32mfma(const FwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_dq_f32mfma(const BwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_dkv_f32mfma(const BwdArgs& a, hipStream_t st);
-// Rows of a [total_rows, row_bytes] tensor outside [cu[0], cu[num_seqs]).
+// Rows of a [total_rows, row_bytes] tensor (row stride stride_bytes, 0:
+// contiguous) outside [cu[0], cu[num_seqs]).
 struct ZeroFill {
     void* ptr;
     int64_t row_bytes, total_rows;
     const int* cu;
+    int64_t stride_bytes = 0;
 };
 // Zeroes those rows of up to three tensors in one launch.
 hipError_t launch_zero_outside(const ZeroFill* fills, int n, int num_seqs, hipStream_t st);

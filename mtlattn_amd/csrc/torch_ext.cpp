@@ -169,11 +169,13 @@ at::Tensor varlen_attention(const at::Tensor& q, const at::Tensor& k, const at::
     return out;
 }
 
-// _C.varlen_attention_bwd (src/ext.mm:502-594).
-std::tuple<at::Tensor, at::Tensor, at::Tensor> varlen_attention_bwd(
-    const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& dout,
-    const at::Tensor& lse, const at::Tensor& cu_seqlens_q, const at::Tensor& cu_seqlens_kv, double scale,
-    bool causal, int64_t window, c10::optional<at::Tensor> attn_bias) {
+// The backward into dQ, dK and dV: [M, H, D] tensors or slices of one packed
+// tensor (heads contiguous, any row stride, dK's and dV's the same). False,
+// with nothing launched, where the kernels only write contiguous gradients.
+bool backward_into(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
+                   const at::Tensor& dout, const at::Tensor& lse, const at::Tensor& cu_seqlens_q,
+                   const at::Tensor& cu_seqlens_kv, double scale, bool causal, int64_t window,
+                   const c10::optional<at::Tensor>& attn_bias, at::Tensor dQ, at::Tensor dK, at::Tensor dV) {
     check_qkv(q, k, v);
     check_cu(cu_seqlens_q, cu_seqlens_kv, q);
     TORCH_CHECK(o.sizes() == q.sizes() && dout.sizes() == q.sizes(), "mtlattn: o/dout must match q's shape");
@@ -185,19 +187,73 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> varlen_attention_bwd(
                 "mtlattn: lse must be a contiguous fp32 [total_q, H] GPU tensor");
     const c10::OptionalDeviceGuard guard(q.device());
     auto cu_q = cu_seqlens_q.contiguous(), cu_kv = cu_seqlens_kv.contiguous();
-    auto dQ = at::empty({q.size(0), q.size(1), q.size(2)}, q.options());
-    auto dK = at::empty({k.size(0), k.size(1), k.size(2)}, k.options());
-    auto dV = at::empty({v.size(0), v.size(1), v.size(2)}, v.options());
     mtlattn_problem p = make_problem(q, k, cu_q, cu_kv, q.size(0), scale, causal, window);
     at::Tensor bias_keep;
     fill_bias(p, attn_bias, q, bias_keep);
     const size_t ws_bytes = mtlattn_varlen_bwd_workspace_size(&p);
     at::Tensor ws = workspace((int64_t)ws_bytes, q);
+    if (!(dQ.is_contiguous() && dK.is_contiguous() && dV.is_contiguous())) {
+        const int rc = mtlattn_varlen_bwd_strided(
+            &p, q.data_ptr(), row_stride(q), k.data_ptr(), row_stride(k), v.data_ptr(), row_stride(v), o.data_ptr(),
+            row_stride(o), dout.data_ptr(), row_stride(dout), lse.data_ptr<float>(), dQ.data_ptr(), row_stride(dQ),
+            dK.data_ptr(), dV.data_ptr(), row_stride(dK), ws.data_ptr(), ws_bytes, current_stream(q));
+        if (rc == MTLATTN_ERR_UNSUPPORTED) return false;
+        check_rc(rc);
+        return true;
+    }
     check_rc(mtlattn_varlen_bwd(&p, q.data_ptr(), row_stride(q), k.data_ptr(), row_stride(k), v.data_ptr(),
                                 row_stride(v), o.data_ptr(), row_stride(o), dout.data_ptr(), row_stride(dout),
                                 lse.data_ptr<float>(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), ws.data_ptr(),
                                 ws_bytes, current_stream(q)));
+    return true;
+}
+
+// _C.varlen_attention_bwd (src/ext.mm:502-594).
+std::tuple<at::Tensor, at::Tensor, at::Tensor> varlen_attention_bwd(
+    const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& dout,
+    const at::Tensor& lse, const at::Tensor& cu_seqlens_q, const at::Tensor& cu_seqlens_kv, double scale,
+    bool causal, int64_t window, c10::optional<at::Tensor> attn_bias) {
+    check_qkv(q, k, v);
+    const c10::OptionalDeviceGuard guard(q.device());
+    auto dQ = at::empty({q.size(0), q.size(1), q.size(2)}, q.options());
+    auto dK = at::empty({k.size(0), k.size(1), k.size(2)}, k.options());
+    auto dV = at::empty({v.size(0), v.size(1), v.size(2)}, v.options());
+    backward_into(q, k, v, o, dout, lse, cu_seqlens_q, cu_seqlens_kv, scale, causal, window, attn_bias, dQ, dK, dV);
     return {dQ, dK, dV};
+}
+
+// The gradient of a packed qkv [M, 3, H, D], or dq and the gradient of a
+// packed kv [Mkv, 2, Hkv, D], written in place (no counterpart in the
+// reference, whose wrappers stack the views' gradients).
+at::Tensor varlen_attention_bwd_qkvpacked(const at::Tensor& qkv, const at::Tensor& o, const at::Tensor& dout,
+                                          const at::Tensor& lse, const at::Tensor& cu_seqlens, double scale,
+                                          bool causal, int64_t window) {
+    TORCH_CHECK(qkv.dim() == 4 && qkv.size(1) == 3, "mtlattn: qkv must be [M, 3, H, D]");
+    const c10::OptionalDeviceGuard guard(qkv.device());
+    const auto q = qkv.select(1, 0), k = qkv.select(1, 1), v = qkv.select(1, 2);
+    auto d = at::empty(qkv.sizes(), qkv.options());
+    if (backward_into(q, k, v, o, dout, lse, cu_seqlens, cu_seqlens, scale, causal, window, c10::nullopt,
+                      d.select(1, 0), d.select(1, 1), d.select(1, 2)))
+        return d;
+    const auto g = varlen_attention_bwd(q, k, v, o, dout, lse, cu_seqlens, cu_seqlens, scale, causal, window,
+                                        c10::nullopt);
+    return at::stack({std::get<0>(g), std::get<1>(g), std::get<2>(g)}, 1);
+}
+
+std::tuple<at::Tensor, at::Tensor> varlen_attention_bwd_kvpacked(
+    const at::Tensor& q, const at::Tensor& kv, const at::Tensor& o, const at::Tensor& dout, const at::Tensor& lse,
+    const at::Tensor& cu_seqlens_q, const at::Tensor& cu_seqlens_kv, double scale, bool causal, int64_t window) {
+    TORCH_CHECK(kv.dim() == 4 && kv.size(1) == 2, "mtlattn: kv must be [Mkv, 2, Hkv, D]");
+    const c10::OptionalDeviceGuard guard(q.device());
+    const auto k = kv.select(1, 0), v = kv.select(1, 1);
+    auto dQ = at::empty({q.size(0), q.size(1), q.size(2)}, q.options());
+    auto d = at::empty(kv.sizes(), kv.options());
+    if (backward_into(q, k, v, o, dout, lse, cu_seqlens_q, cu_seqlens_kv, scale, causal, window, c10::nullopt, dQ,
+                      d.select(1, 0), d.select(1, 1)))
+        return {dQ, d};
+    const auto g = varlen_attention_bwd(q, k, v, o, dout, lse, cu_seqlens_q, cu_seqlens_kv, scale, causal, window,
+                                        c10::nullopt);
+    return {std::get<0>(g), at::stack({std::get<1>(g), std::get<2>(g)}, 1)};
 }
 
 // _C.attn_splitkv (src/ext.mm:716-773). `window` and `attn_bias` (after the
@@ -439,4 +495,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("k"), py::arg("v"), py::arg("o"), py::arg("dout"), py::arg("lse"), py::arg("cu_seqlens_q"),
           py::arg("cu_seqlens_kv"), py::arg("scale"), py::arg("causal") = false, py::arg("window") = 0,
           py::arg("attn_bias") = c10::nullopt);
+    m.def("varlen_attention_bwd_qkvpacked", &varlen_attention_bwd_qkvpacked, "Backward into a packed qkv gradient",
+          py::arg("qkv"), py::arg("o"), py::arg("dout"), py::arg("lse"), py::arg("cu_seqlens"), py::arg("scale"),
+          py::arg("causal") = false, py::arg("window") = 0);
+    m.def("varlen_attention_bwd_kvpacked", &varlen_attention_bwd_kvpacked, "Backward into dq and a packed kv gradient",
+          py::arg("q"), py::arg("kv"), py::arg("o"), py::arg("dout"), py::arg("lse"), py::arg("cu_seqlens_q"),
+          py::arg("cu_seqlens_kv"), py::arg("scale"), py::arg("causal") = false, py::arg("window") = 0);
 }
