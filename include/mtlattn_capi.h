@@ -146,6 +146,26 @@ int mtlattn_varlen_fwd_noalloc(const mtlattn_problem* p,
                                void* stream);
 
 /*
+ * Dense forward for the SDPA adapter: q [B, Hq, Nq, D], k / v [B, Hkv, Nkv, D]
+ * read in place through element strides of their B, H and N dims (D contiguous),
+ * out contiguous [B, Hq, Nq, D]. No counterpart in the reference, whose adapter
+ * copies all four into packed rows (mtlattn/__init__.py:162-181). `p` gives
+ * dtype, num_seqs (= B), the head counts, head_dim, scale, causal and a bias
+ * with bias_seq_local; its cu_seqlens, token totals and window are not read.
+ * lens: NULL, or device int32 [B] (Nq == Nkv): tokens past lens[b] (clamped to
+ * [0, Nq]) are padding -- not attended, their output rows 0. fp16/bf16,
+ * D in {64, 80, 88, 96, 128}, scale > 0, 16-byte aligned rows, and shapes that
+ * mtlattn_varlen_fwd runs on its unsplit flash kernels; otherwise
+ * MTLATTN_ERR_UNSUPPORTED with nothing launched (pack the rows and call
+ * mtlattn_varlen_fwd). Same values as that. No workspace.
+ */
+int mtlattn_dense_fwd(const mtlattn_problem* p, int32_t Nq, int32_t Nkv,
+                      const void* q, int64_t q_batch_stride, int64_t q_head_stride, int64_t q_row_stride,
+                      const void* k, int64_t k_batch_stride, int64_t k_head_stride, int64_t k_row_stride,
+                      const void* v, int64_t v_batch_stride, int64_t v_head_stride, int64_t v_row_stride,
+                      const int32_t* lens, void* out, void* stream);
+
+/*
  * Backward: (dq, dk, dv) of the forward above given dout and the forward's
  * out and lse. dk/dv of a kv head are summed over its Hq/Hkv query heads
  * inside the kernels (no atomics; bitwise run-to-run deterministic).

@@ -248,6 +248,14 @@ def _sdpa_mask_to_bias(attn_mask, B, Hq, Nq, Nkv):
     return m
 
 
+def _dense(query, key, value, scale, causal, lens=None, bias=None):
+    """The dense forward in place -- no packed copies of q, k, v and the output
+    -- or None where the kernels need packed rows or gradients are wanted."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (query, key, value)):
+        return None
+    return _C.dense_attention(query, key, value, float(scale), bool(causal), lens, bias)
+
+
 def sdpa(query, key, value, attn_mask=None, dropout_p=0.0, is_causal=False, scale=None):
     """Dense [B, H, N, D] attention through the varlen kernel (reference:
     mtlattn/__init__.py:162-181): equal-length batches become trivial
@@ -257,13 +265,17 @@ def sdpa(query, key, value, attn_mask=None, dropout_p=0.0, is_causal=False, scal
     Hkv, Nkv = key.shape[1], key.shape[2]
     if scale is None:
         scale = 1.0 / math.sqrt(D)
+    bias = None if attn_mask is None else _sdpa_mask_to_bias(attn_mask, B, Hq, Nq, Nkv)
+    if bias is None or not bias.requires_grad:
+        out = _dense(query, key, value, scale, is_causal, bias=bias)
+        if out is not None:
+            return out
     q = query.transpose(1, 2).contiguous().view(B * Nq, Hq, D)
     k = key.transpose(1, 2).contiguous().view(B * Nkv, Hkv, D)
     v = value.transpose(1, 2).contiguous().view(B * Nkv, Hkv, D)
     dev = query.device
     cu_q = torch.arange(0, (B + 1) * Nq, Nq, dtype=torch.int32, device=dev)
     cu_kv = torch.arange(0, (B + 1) * Nkv, Nkv, dtype=torch.int32, device=dev)
-    bias = None if attn_mask is None else _sdpa_mask_to_bias(attn_mask, B, Hq, Nq, Nkv)
     out = varlen_attention(q, k, v, cu_q, cu_kv, Nq, scale, causal=is_causal, attn_bias=bias)
     return out.view(B, Nq, Hq, D).transpose(1, 2).contiguous()
 
@@ -345,6 +357,9 @@ def _try_padding_varlen(query, key, value, attn_mask, is_causal, scale):
     ok, lens = _padding_decision(attn_mask, B, Hq, Nq, Nkv)
     if not ok:
         return None
+    out = _dense(query, key, value, scale, is_causal, lens)
+    if out is not None:
+        return out
     # pack, attend, unpack on the device: no lengths on the host, no
     # per-batch copies (rows past cu[B] belong to no sequence)
     qp, cu = _C.pack_padded(query, lens)

@@ -53,6 +53,8 @@ SIGNATURES = {
     "mtlattn_varlen_fwd_workspace_size": (_sz, [_P]),
     "mtlattn_varlen_fwd": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _sz, _vp]),
     "mtlattn_varlen_fwd_noalloc": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp]),
+    "mtlattn_dense_fwd": (ctypes.c_int, [_P, _i32, _i32, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _i64,
+                                         _i64, _vp, _vp, _vp]),
     "mtlattn_varlen_bwd_workspace_size": (_sz, [_P]),
     "mtlattn_varlen_bwd": (ctypes.c_int, [_P, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp,
                                           _vp, _vp, _vp, _vp, _sz, _vp]),

@@ -493,6 +493,49 @@ int mtlattn_varlen_fwd_noalloc(const mtlattn_problem* p, const void* q, int64_t 
     return mtlattn_varlen_fwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, out, lse, ws, need, stream);
 }
 
+int mtlattn_dense_fwd(const mtlattn_problem* p, int32_t Nq, int32_t Nkv, const void* q, int64_t q_batch_stride,
+                      int64_t q_head_stride, int64_t q_row_stride, const void* k, int64_t k_batch_stride,
+                      int64_t k_head_stride, int64_t k_row_stride, const void* v, int64_t v_batch_stride,
+                      int64_t v_head_stride, int64_t v_row_stride, const int32_t* lens, void* out, void* stream) {
+    if (p == nullptr) return fail(MTLATTN_ERR_INVALID, "mtlattn: null problem descriptor");
+    if (Nq < 0 || Nkv < 0 || (lens != nullptr && Nq != Nkv))
+        return fail(MTLATTN_ERR_INVALID, "mtlattn: dense_fwd: bad sequence lengths");
+    static const int32_t kNoCu = 0;       // (check_problem wants the pointers; they are not read)
+    mtlattn_problem d = *p;
+    d.cu_seqlens_q = d.cu_seqlens_kv = &kNoCu;
+    d.total_q = (int64_t)d.num_seqs * Nq;
+    d.total_kv = (int64_t)d.num_seqs * Nkv;
+    d.max_seqlen_q = Nq;
+    d.window = 0;
+    int rc = check_problem(&d);
+    if (rc != MTLATTN_OK) return rc;
+    if (d.total_q == 0) return ok();
+    if (q == nullptr || k == nullptr || v == nullptr || out == nullptr)
+        return fail(MTLATTN_ERR_INVALID, "mtlattn: null q/k/v/out pointer");
+    if (!is16(d.dtype) || !dense_head_dim(d.head_dim) || !(d.scale > 0.f) || Nkv == 0 ||
+        (d.bias != nullptr && d.bias_kv_cols > 0 && d.bias_seq_local == 0))
+        return fail(MTLATTN_ERR_UNSUPPORTED, "mtlattn: dense_fwd: unsupported type, head dim or scale");
+    const int64_t strides[9] = {q_batch_stride, q_head_stride, q_row_stride, k_batch_stride, k_head_stride,
+                                k_row_stride,   v_batch_stride, v_head_stride, v_row_stride};
+    for (const int64_t s : strides)
+        if (s < 0 || s % 8 != 0) return fail(MTLATTN_ERR_UNSUPPORTED, "mtlattn: dense_fwd: rows must be 16-byte aligned");
+    if (((uintptr_t)q & 15u) || ((uintptr_t)k & 15u) || ((uintptr_t)v & 15u) || ((uintptr_t)out & 15u) ||
+        !tile_stride_ok(k_row_stride) || !tile_stride_ok(v_row_stride))
+        return fail(MTLATTN_ERR_UNSUPPORTED, "mtlattn: dense_fwd: rows must be 16-byte aligned");
+    if (force_generic() || decode_allowed(&d) || fwd_plan(&d).grid > 0)
+        return fail(MTLATTN_ERR_UNSUPPORTED, "mtlattn: dense_fwd: a shape for the split kernels");
+    DenseArgs a;
+    a.geo = make_geo(&d);
+    a.q = q; a.q_bs = q_batch_stride; a.q_hs = q_head_stride; a.q_rs = q_row_stride;
+    a.k = k; a.k_bs = k_batch_stride; a.k_hs = k_head_stride; a.k_rs = k_row_stride;
+    a.v = v; a.v_bs = v_batch_stride; a.v_hs = v_head_stride; a.v_rs = v_row_stride;
+    a.o = out;
+    a.lens = lens;
+    a.nq = Nq;
+    a.nkv = Nkv;
+    return launch_status(launch_fwd_dense(d.dtype, a, (hipStream_t)stream), "dense forward");
+}
+
 namespace {
 
 size_t bwd_delta_bytes(const mtlattn_problem* p) { return (size_t)p->total_q * (size_t)p->num_heads_q * sizeof(float); }

@@ -60,6 +60,12 @@ struct FwdKParams {
     int split_grid;
     int* piece_out; int* first;
     float* part_o; float* part_lse;
+    // DENSE launches: [B, H, N, D] tensors by batch, head and row strides (q_rs,
+    // k_rs, v_rs above), nq / nkv tokens a batch of which the first lens[b] are
+    // attended (null: all); tps row tiles per batch
+    int64_t q_bs, q_hs, k_bs, k_hs, v_bs, v_hs, o_bs, o_hs, o_rs;
+    const int* lens;
+    int nq, nkv, tps;
 };
 
 // Key tiles [lo, lo + n KT) that the query rows q0 .. q0 + qt - 1 of a
@@ -105,9 +111,13 @@ constexpr double kFwdSplitCost = 10.;
 // SPLIT (grids that leave CUs idle, make_fwd_plan): a workgroup takes one
 // piece of one tile's key tiles; pieces of tiles cut in several write their
 // rows' O and LSE as fp32 for fwd_merge_kernel.
+// DENSE: the tensors are [B, H, N, D] with their own strides instead of packed
+// rows (the SDPA adapter's layout, read and written in place); query rows past
+// a batch's length are written as 0.
 template <typename T, int DK, int DV, int DVL, int DO, int SM, int BROWS = 0, int KT = kKT, int NW = kWaves, int NBUF = 3,
-          bool SPLIT = false>
+          bool SPLIT = false, bool DENSE = false>
 __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKParams p) {
+    static_assert(!DENSE || (!SPLIT && SM != 2 && DO == DV), "dense: one launch, scale > 0");
     static_assert(!SPLIT || (SM == 0 && DO == DV), "split: no bias, all columns in one launch");
     static_assert(KT == 64 || ((KT == 32 || KT == 128) && BROWS == 0), "32- and 128-key tiles: no staged bias");
     constexpr int NKB = KT / 32;             // 32-key blocks per tile
@@ -150,19 +160,52 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
         pc.t = p.n_tiles - 1 - (L - pc.group * p.n_tiles);   // late (heavier) tiles first
     }
     const int hg = pc.group, t = pc.t;
-    const int s = find_seq_for_tile(p.cu_q, p.num_seqs, QT, t, p.total_q);
-    const int tb = tile_base(p.cu_q, s, QT, p.total_q);
-    if (t < tb) return;
-    const SeqRange qr = seq_range(p.cu_q, s, p.total_q);
-    const SeqRange kr = seq_range(p.cu_kv, s, p.total_kv);
-    const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
-    const int q0 = (t - tb) * QT;
-    if (q0 >= q_len) return;
+    int s, q0, q_len, kv_len;
+    SeqRange qr{0, 0}, kr{0, 0};
+    if constexpr (DENSE) {
+        s = t / p.tps;
+        q0 = (t - s * p.tps) * QT;
+        q_len = p.lens != nullptr ? min(max(p.lens[s], 0), p.nq) : p.nq;
+        kv_len = p.lens != nullptr ? min(q_len, p.nkv) : p.nkv;
+    } else {
+        s = find_seq_for_tile(p.cu_q, p.num_seqs, QT, t, p.total_q);
+        const int tb = tile_base(p.cu_q, s, QT, p.total_q);
+        if (t < tb) return;
+        qr = seq_range(p.cu_q, s, p.total_q);
+        kr = seq_range(p.cu_kv, s, p.total_kv);
+        q_len = qr.end - qr.start;
+        kv_len = kr.end - kr.start;
+        q0 = (t - tb) * QT;
+        if (q0 >= q_len) return;
+    }
 
     const int wph = NW / p.hpw;
     const int head = hg * p.hpw + w / wph;
     const int hk = head / p.g;
     const int qa = q0 + 32 * (w % wph);          // first query row of this wave (seq-local)
+    // element offsets of the sequence's first row and of a head
+    const uint16_t* qseq = p.q + (DENSE ? s * p.q_bs + head * p.q_hs : (int64_t)qr.start * p.q_rs + (int64_t)head * DV);
+    uint16_t* oseq = p.o + (DENSE ? s * p.o_bs + head * p.o_hs
+                                  : (int64_t)qr.start * ((int64_t)p.hq * DV) + (int64_t)head * DV);
+    const int64_t o_rs = DENSE ? p.o_rs : (int64_t)p.hq * DV;
+    if constexpr (DENSE) {
+        // padded query rows (past the batch's length): zeros
+        const int row = qa + l32;
+        if (row >= q_len && row < p.nq) {
+            uint16_t* op = oseq + row * o_rs;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int rg = 0; rg < 4; ++rg) {
+                    const int d = 32 * db + 8 * rg + 4 * hi;
+                    if (DO % 32 != 0 && d >= DO) continue;
+                    st8(op + d, u32x2_t{0u, 0u});
+                }
+        }
+        if (q0 >= q_len) return;
+        // settle the stores: the key loop's waits count only its direct loads
+        wait_vmcnt<0>();
+    }
     const int coff = kv_len - q_len;
     const bool wave_active = qa < q_len;
     const int wq_last = min(q_len, qa + 32) - 1;
@@ -172,7 +215,7 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
     u32x4_t qf[DC];
     {
         const int row = min(qa + l32, q_len - 1);
-        const uint16_t* qp = p.q + (int64_t)(qr.start + row) * p.q_rs + (int64_t)head * DV + 8 * hi;
+        const uint16_t* qp = qseq + (int64_t)row * p.q_rs + 8 * hi;
 #pragma unroll
         for (int kc = 0; kc < DC; ++kc)
             qf[kc] = (DV % 16 == 0 || 16 * kc + 8 * hi < DV) ? ld16(qp + 16 * kc) : u32x4_t{};
@@ -186,8 +229,8 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
     const int kv_lo = SPLIT ? kts.lo + pc.st0 * KT : kts.lo;
     const int n_kv_tiles = SPLIT ? pc.n : kts.n;
 
-    const uint16_t* kbase = p.k + (int64_t)kr.start * p.k_rs + (int64_t)hk * DV;
-    const uint16_t* vbase = p.v + (int64_t)kr.start * p.v_rs + (int64_t)hk * DV + p.col0;
+    const uint16_t* kbase = p.k + (DENSE ? s * p.k_bs + hk * p.k_hs : (int64_t)kr.start * p.k_rs + (int64_t)hk * DV);
+    const uint16_t* vbase = p.v + (DENSE ? s * p.v_bs + hk * p.v_hs : (int64_t)kr.start * p.v_rs + (int64_t)hk * DV) + p.col0;
     // The NW waves stage each tile straight from HBM into LDS (K then V).
     TileStager<DK, KT, NW, DV> kst;
     TileStager<DVL, KT, NW, DO> vst;
@@ -519,7 +562,7 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
                 return;
             }
         }
-        uint16_t* op = p.o + (int64_t)(qr.start + qrow) * ((int64_t)p.hq * DV) + (int64_t)head * DV + p.col0;
+        uint16_t* op = oseq + (int64_t)qrow * o_rs + p.col0;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -530,7 +573,7 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
                                     T::pack2(oacc[db][4 * rg + 2] * inv, oacc[db][4 * rg + 3] * inv)});
             }
         }
-        if (p.lse != nullptr && hi == 0)
+        if (!DENSE && p.lse != nullptr && hi == 0)
             p.lse[(int64_t)(qr.start + qrow) * p.hq + head] = !(lt <= 0.f) ? m_run * kLn2 + logf(lt) : kNegInf;
     }
 }
@@ -637,6 +680,70 @@ hipError_t launch_split(const FwdArgs& a, FwdKParams p, hipStream_t st) {
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((fwd_merge_kernel<T, DV, C::KT>), dim3((unsigned)(p.n_tiles * p.n_hg), 8), dim3(256), 0, st, p,
                        C::NW);
+    return hipGetLastError();
+}
+
+// Dense launches follow launch_typed's choices of workgroup and tile (the
+// same values, bitwise). The packed path's copies and small launches around the
+// kernel cost as much as it: 2 x 2048 causal, 32/8 heads, D = 128, 93 us of
+// kernel in 144 us of call, now 87; 8 x 1536 padded, 16 heads, D = 64, 132 -> 68;
+// 3 x 228, 32/8 heads, 40 -> 10.
+template <typename T, int DK, int DV>
+hipError_t launch_dense_typed(const DenseArgs& a, hipStream_t st) {
+    const Geometry& g = a.geo;
+    FwdKParams p{};
+    p.q = (const uint16_t*)a.q; p.k = (const uint16_t*)a.k; p.v = (const uint16_t*)a.v; p.o = (uint16_t*)a.o;
+    p.q_bs = a.q_bs; p.q_hs = a.q_hs; p.q_rs = a.q_rs;
+    p.k_bs = a.k_bs; p.k_hs = a.k_hs; p.k_rs = a.k_rs;
+    p.v_bs = a.v_bs; p.v_hs = a.v_hs; p.v_rs = a.v_rs;
+    p.o_rs = g.d; p.o_hs = (int64_t)a.nq * g.d; p.o_bs = p.o_hs * g.hq;
+    p.lens = a.lens; p.nq = a.nq; p.nkv = a.nkv;
+    p.bias = g.bias;
+    p.bias_qs = g.bias_qs; p.bias_hs = g.bias_hs; p.bias_cols = g.bias_cols;
+    p.bias_ss = g.bias_ss; p.bias_rows = g.bias_rows;
+    p.num_seqs = g.num_seqs; p.hq = g.hq; p.g = g.g;
+    p.scale = g.scale; p.scale_log2 = g.scale * kLog2e;
+    p.causal = g.causal;
+    p.bias_v4 = g.bias != nullptr && ((uintptr_t)g.bias % 16 == 0) && g.bias_qs % 4 == 0 && g.bias_hs % 4 == 0 &&
+                (g.bias_ss < 0 || g.bias_ss % 4 == 0);
+    auto grid = [&](int nw, int hpw) {
+        p.hpw = hpw;
+        const int qt = 32 * (nw / hpw);
+        p.tps = (a.nq + qt - 1) / qt;
+        p.n_tiles = g.num_seqs * p.tps;
+        p.n_hg = g.hq / hpw;
+        return (int64_t)p.n_tiles * p.n_hg;
+    };
+    const int hpw = gcd_int(g.g, kWaves), QT = 32 * (kWaves / hpw);
+    if ((int64_t)g.num_seqs * ((a.nq + 31) / 32) * g.hq > 0x7fffffff) return hipErrorInvalidValue;
+    if (g.bias == nullptr) {
+        if ((DV == 128 || (DV == 64 && p.causal)) &&
+            (g.total_q / QT) * (g.hq / hpw) <= 2 * (int64_t)device_cus()) {
+            if constexpr (DV == 64 || DV == 128) {
+                const int64_t blocks = grid(4, gcd_int(g.g, 2));
+                hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 0, 0, 64, 4, 2, false, true>),
+                                   dim3((unsigned)blocks), dim3(256), 0, st, p);
+                return hipGetLastError();
+            }
+        }
+        const int64_t blocks = grid(kWaves, hpw);
+        hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 0, 0, DK == 128 ? 128 : 64, kWaves, DK == 128 ? 2 : 3,
+                                            false, true>),
+                           dim3((unsigned)blocks), dim3(kThreads), 0, st, p);
+        return hipGetLastError();
+    }
+    const int64_t blocks = grid(kWaves, hpw);
+    const bool staged = g.bias_hs == 0 && p.bias_v4 && g.bias_cols >= 4 && g.bias_cols % 4 == 0 &&
+                        ((int64_t)QT * g.bias_qs + g.bias_cols) * 4 < ((int64_t)1 << 32);
+    if (staged && QT == 32)
+        hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 1, 32, kKT, kWaves, 3, false, true>),
+                           dim3((unsigned)blocks), dim3(kThreads), 0, st, p);
+    else if (staged && QT == 64)
+        hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 1, 64, kKT, kWaves, 3, false, true>),
+                           dim3((unsigned)blocks), dim3(kThreads), 0, st, p);
+    else
+        hipLaunchKernelGGL((fwd_mfma_kernel<T, DK, DV, DK, DV, 1, 0, kKT, kWaves, 3, false, true>),
+                           dim3((unsigned)blocks), dim3(kThreads), 0, st, p);
     return hipGetLastError();
 }
 
@@ -850,6 +957,23 @@ FwdPlan make_fwd_plan(const Geometry& g, int max_q, int cus, size_t max_bytes) {
 hipError_t launch_fwd_mfma(int dtype, const FwdArgs& a, hipStream_t st) {
     if (dtype == MTLATTN_DTYPE_BF16) return launch_dims<BF16>(a, st);
     if (dtype == MTLATTN_DTYPE_F16) return launch_dims<F16>(a, st);
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_fwd_dense(int dtype, const DenseArgs& a, hipStream_t st) {
+    auto dims = [&](auto t) {
+        using T = decltype(t);
+        switch (a.geo.d) {
+            case 64: return launch_dense_typed<T, 64, 64>(a, st);
+            case 80: return launch_dense_typed<T, 128, 80>(a, st);
+            case 88: return launch_dense_typed<T, 128, 88>(a, st);
+            case 96: return launch_dense_typed<T, 128, 96>(a, st);
+            case 128: return launch_dense_typed<T, 128, 128>(a, st);
+            default: return hipErrorInvalidValue;
+        }
+    };
+    if (dtype == MTLATTN_DTYPE_BF16) return dims(BF16{});
+    if (dtype == MTLATTN_DTYPE_F16) return dims(F16{});
     return hipErrorInvalidValue;
 }
 

@@ -48,6 +48,22 @@ struct FwdArgs {
     void* split_ws = nullptr;
 };
 
+// Dense forward: [B, H, N, D] tensors by strides (elements; the head dim
+// contiguous), o contiguous. geo: num_seqs = B, total_q = B * nq, hq, hkv, g, d,
+// scale, causal and a bias by sequence and local row; no cu_seqlens. lens
+// (nullable, nq == nkv): the first lens[b] tokens of batch b attend, the other
+// query rows are written as 0.
+struct DenseArgs {
+    Geometry geo;
+    const void* q; int64_t q_bs, q_hs, q_rs;
+    const void* k; int64_t k_bs, k_hs, k_rs;
+    const void* v; int64_t v_bs, v_hs, v_rs;
+    void* o;
+    const int* lens;
+    int nq, nkv;
+};
+inline bool dense_head_dim(int d) { return d == 64 || d == 80 || d == 88 || d == 96 || d == 128; }
+
 // How the 16-bit dK/dV cuts its work (make_dkv_plan): pieces == 1: one
 // workgroup per key block or pair of key blocks; else at most `pieces` pieces
 // per key block on a grid of `grid` workgroups.
@@ -120,6 +136,7 @@ struct DecodeArgs {
 
 // Launchers return hipSuccess or the launch error. `dtype` is MTLATTN_DTYPE_*.
 hipError_t launch_fwd_mfma(int dtype, const FwdArgs& a, hipStream_t st);
+hipError_t launch_fwd_dense(int dtype, const DenseArgs& a, hipStream_t st);
 hipError_t launch_fwd_generic(int dtype, const FwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_preprocess(int dtype, const Geometry& geo, const void* o, int64_t o_rs,
                                  const void* dout, int64_t do_rs, float* delta, hipStream_t st);

@@ -169,6 +169,48 @@ at::Tensor varlen_attention(const at::Tensor& q, const at::Tensor& k, const at::
     return out;
 }
 
+// _C.dense_attention: the SDPA adapter's [B, H, N, D] forward in place (no
+// reference counterpart). None where the kernels need packed rows.
+c10::optional<at::Tensor> dense_attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double scale,
+                                          bool causal, c10::optional<at::Tensor> lens,
+                                          c10::optional<at::Tensor> attn_bias) {
+    const auto B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Hkv = k.size(1), Nkv = k.size(2);
+    if (!q.is_cuda() || k.get_device() != q.get_device() || v.get_device() != q.get_device() ||
+        k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || v.sizes() != k.sizes() ||
+        k.size(0) != B || k.size(3) != D || Hkv == 0 || H % Hkv != 0)
+        return c10::nullopt;
+    for (const auto& t : {q, k, v})
+        if (D > 1 && t.stride(3) != 1) return c10::nullopt;
+    if (q.scalar_type() != at::kHalf && q.scalar_type() != at::kBFloat16) return c10::nullopt;
+    const c10::OptionalDeviceGuard guard(q.device());
+    mtlattn_problem p;
+    std::memset(&p, 0, sizeof(p));
+    p.dtype = dtype_code(q.scalar_type());
+    p.num_seqs = (int32_t)B;
+    p.num_heads_q = (int32_t)H;
+    p.num_heads_kv = (int32_t)Hkv;
+    p.head_dim = (int32_t)D;
+    p.scale = (float)scale;
+    p.causal = causal ? 1 : 0;
+    at::Tensor bias_keep, lens_keep;
+    if (defined(attn_bias) && attn_bias->dim() != 4) return c10::nullopt;
+    fill_bias(p, attn_bias, q, bias_keep);
+    if (lens.has_value()) {
+        lens_keep = lens->contiguous();
+        TORCH_CHECK(lens_keep.is_cuda() && lens_keep.scalar_type() == at::kInt && lens_keep.numel() == B,
+                    "mtlattn: lens must be an int32 [B] GPU tensor");
+    }
+    auto out = at::empty({B, H, N, D}, q.options());
+    const int rc = mtlattn_dense_fwd(&p, (int32_t)N, (int32_t)Nkv, q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
+                                     k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0),
+                                     v.stride(1), v.stride(2),
+                                     lens_keep.defined() ? lens_keep.data_ptr<int32_t>() : nullptr, out.data_ptr(),
+                                     current_stream(q));
+    if (rc == MTLATTN_ERR_UNSUPPORTED) return c10::nullopt;
+    check_rc(rc);
+    return out;
+}
+
 // The backward into dQ, dK and dV: [M, H, D] tensors or slices of one packed
 // tensor (heads contiguous, any row stride, dK's and dV's the same). False,
 // with nothing launched, where the kernels only write contiguous gradients.
@@ -501,4 +543,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("varlen_attention_bwd_kvpacked", &varlen_attention_bwd_kvpacked, "Backward into dq and a packed kv gradient",
           py::arg("q"), py::arg("kv"), py::arg("o"), py::arg("dout"), py::arg("lse"), py::arg("cu_seqlens_q"),
           py::arg("cu_seqlens_kv"), py::arg("scale"), py::arg("causal") = false, py::arg("window") = 0);
+    m.def("dense_attention", &dense_attention, "dense [B,H,N,D] forward in place, or None (pack the rows)",
+          py::arg("q"), py::arg("k"), py::arg("v"), py::arg("scale"), py::arg("causal") = false,
+          py::arg("lens") = c10::nullopt, py::arg("attn_bias") = c10::nullopt);
 }

@@ -1,0 +1,92 @@
+"""The SDPA adapter's dense forward, in place through strides, against the
+packed path on the same inputs (the same kernels on packed copies)."""
+
+import pytest
+import torch
+
+from tests.helpers import randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _tensor(layout, B, H, N, D, dtype, g):
+    if layout == "bhnd":
+        return randn((B, H, N, D), dtype, g).cuda()
+    if layout == "bnhd":                      # a projection's [B, N, H, D], transposed
+        return randn((B, N, H, D), dtype, g).cuda().transpose(1, 2)
+    if layout == "slice":                     # rows and heads inside a wider tensor
+        return randn((B, H, N + 3, D + 16), dtype, g).cuda()[:, :, 2:N + 2, 8:D + 8]
+    return randn((1, H, N, D), dtype, g).cuda().expand(B, H, N, D)    # "shared": one batch for all
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Nq,Nkv,D,dtype,layout,mask,causal", [
+    (2, 8, 2, 300, 300, 128, torch.bfloat16, "bhnd", None, True),
+    (3, 4, 4, 257, 257, 64, torch.float16, "bnhd", None, False),
+    (1, 16, 4, 1025, 1025, 64, torch.bfloat16, "bnhd", None, True),
+    (2, 4, 4, 33, 129, 80, torch.float16, "slice", None, False),
+    (2, 8, 8, 100, 700, 128, torch.float16, "shared", None, True),
+    (2, 4, 2, 64, 64, 96, torch.bfloat16, "bhnd", None, True),
+    (2, 4, 4, 70, 70, 88, torch.bfloat16, "bnhd", "bool", False),
+    (2, 8, 1, 130, 128, 128, torch.bfloat16, "bnhd", "float", False),
+    (2, 8, 2, 130, 131, 64, torch.float16, "bhnd", "heads", False),
+    (40, 16, 16, 512, 512, 128, torch.bfloat16, "bhnd", None, False),   # beyond the small-grid kernels
+])
+def test_dense_matches_packed(monkeypatch, B, Hq, Hkv, Nq, Nkv, D, dtype, layout, mask, causal):
+    import mtlattn_amd as mt
+    print(f"\n[case] dense {layout} {B}x{Hq}/{Hkv} {Nq}x{Nkv} D={D} {dtype} mask={mask} causal={causal}", flush=True)
+    g = torch.Generator().manual_seed(2)
+    q = _tensor("bnhd" if layout == "shared" else layout, B, Hq, Nq, D, dtype, g)
+    k, v = (_tensor(layout, B, Hkv, Nkv, D, dtype, g) for _ in range(2))
+    m = None
+    if mask == "bool":
+        m = torch.rand(B, 1, Nq, Nkv, generator=g).cuda() < 0.6
+        m[..., 0] = True
+    elif mask == "float":
+        m = torch.randn(Nq, Nkv, generator=g).cuda()
+    elif mask == "heads":
+        m = torch.randn(B, Hq, Nq, Nkv, generator=g).cuda()
+    with torch.no_grad():
+        assert mt._dense(q, k, v, 0.1, causal,
+                         bias=None if m is None else mt._sdpa_mask_to_bias(m, B, Hq, Nq, Nkv)) is not None
+        out = mt.sdpa(q, k, v, m, is_causal=causal)
+        monkeypatch.setattr(mt, "_dense", lambda *a, **kw: None)
+        ref = mt.sdpa(q, k, v, m, is_causal=causal)
+    assert out.is_contiguous() and out.shape == ref.shape
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,dtype,layout,causal", [
+    (4, 8, 8, 257, 64, torch.bfloat16, "bhnd", False),
+    (5, 8, 2, 300, 128, torch.float16, "bnhd", True),
+    (3, 4, 4, 64, 80, torch.bfloat16, "slice", False),
+])
+def test_dense_padding_matches_packed(monkeypatch, B, Hq, Hkv, N, D, dtype, layout, causal):
+    """Key-padding lengths (0, 1, a tile's edge, all): padded query rows are 0."""
+    import mtlattn_amd as mt
+    print(f"\n[case] dense padding {layout} {B}x{Hq}/{Hkv}x{N} D={D} {dtype} causal={causal}", flush=True)
+    g = torch.Generator().manual_seed(4)
+    q = _tensor(layout, B, Hq, N, D, dtype, g)
+    k, v = (_tensor(layout, B, Hkv, N, D, dtype, g) for _ in range(2))
+    lens = torch.tensor([N, 0, 1, 32, N - 1][:B], device="cuda")
+    m = (torch.arange(N, device="cuda")[None] < lens[:, None])[:, None, None, :]
+    assert mt._dense(q, k, v, 0.1, causal, lens.int()) is not None
+    out = mt._try_padding_varlen(q, k, v, m, causal, 0.1)
+    monkeypatch.setattr(mt, "_dense", lambda *a, **kw: None)
+    ref = mt._try_padding_varlen(q, k, v, m, causal, 0.1)
+    assert torch.equal(out, ref)
+    for b in range(B):
+        assert not out[b, :, lens[b]:].any()
+
+
+def test_dense_refusals():
+    """Calls the dense kernels do not take go through the packed path."""
+    import mtlattn_amd as mt
+    x = lambda *s, dt=torch.bfloat16: torch.randn(s, device="cuda").to(dt)   # noqa: E731
+    q = x(2, 4, 64, 128)
+    assert mt._dense(q, q, q, 0.1, False) is not None
+    for a, kw in (((q.float(),) * 3, {}), ((x(2, 4, 64, 72),) * 3, {}), ((x(2, 4, 64, 256),) * 3, {}),
+                  ((x(2, 4, 8, 128),) * 3, {}), ((x(2, 4, 64, 136)[..., 1:129],) * 3, {}),
+                  ((x(2, 4, 128, 64).transpose(2, 3),) * 3, {}), ((q, q, x(2, 4, 65, 128)), {}),
+                  ((q.clone().requires_grad_(), q, q), {})):
+        assert mt._dense(*a, 0.1, False, **kw) is None, [tuple(t.shape) for t in a]
+    assert mt._dense(q, q, q, -0.1, False) is None
