@@ -1400,21 +1400,18 @@ hipError_t launch_dkv_finish(int type_code, const BwdArgs& a, int kb, int qtl, h
 // workgroup each, with fp32 partials added afterwards: about 1.6 us a stage
 // against 12 us to start a piece and write its partials, and 8 to 20 us to
 // add them. Backward before -> after, bf16 causal, 32/8 heads, D = 128:
-// 1 x 512 193 -> 58 us, 1 x 2048 501 -> 167, 1 x 4096 973 -> 490, 2 x 4096
-// 1149 -> 955, 5 x 4096 (320 pairs on 256 CUs) 2660 -> 2365; D = 64, 16/4 heads,
-// 1 x 2048 193 -> 70; D = 256, 16/4, 1 x 2048 612 -> 248. The line: the split
-// has to beat the unsplit grid's rounds by 10% by this count of stages, on
-// sequences of the average length; 3 x 4096 (192 pairs, 1.0x split) and
-// 8 x 4096 (512 pairs) stay unsplit.
+// 1 x 512 193 -> 58 us, 1 x 2048 501 -> 167, 1 x 4096 973 -> 484; D = 64, 16/4
+// heads, 1 x 2048 193 -> 72; D = 256, 16/4, 1 x 2048 613 -> 244. The line: the
+// split has to beat the unsplit grid by 10% by this count of stages, on
+// sequences of the average length.
 DkvPlan make_dkv_plan(const Geometry& g, int cus) {
     DkvPlan plan;
     if (!mfma_head_dim(g.d) || g.total_q <= 0 || g.total_kv <= 0 || g.num_seqs < 1) return plan;
-    // the kernel these problems run: keys per block, queries per stage,
-    // workgroups per CU, and whether unsplit blocks are taken in pairs
+    // the kernel these problems run: keys per block, queries per stage and
+    // workgroups per CU
     const bool wide = g.bias == nullptr && g.d != 64 && g.d != 160, sym = g.bias == nullptr && g.d == 64;
     const int kb = wide && g.d <= 128 ? 256 : 128, qtl = wide || g.d > 128 ? 32 : 64;
     const int64_t slots = (int64_t)cus * (sym ? 2 : 1);
-    const bool paired = wide && g.window <= 0;
     const int64_t n_tiles = g.total_kv / kb + g.num_seqs + 1, max_grid = 3 * slots;
     const int64_t part = 2 * g.total_kv * g.hkv * (int64_t)g.d * (int64_t)sizeof(float);   // one piece of every block
     const int max_pieces = (int)std::min<int64_t>(kDkvMaxPieces, kDkvPartBytes / part);
@@ -1431,18 +1428,13 @@ DkvPlan make_dkv_plan(const Geometry& g, int cus) {
         n_max = std::max(n_max, n[b]);
         work += n[b] * heads;
     }
-    int64_t unit = n_max;                       // the longest workgroup, unsplit
-    if (paired && nb > 1) {
-        unit = 0;
-        for (int64_t b = 0; b < nb; ++b) unit = std::max(unit, b == nb - 1 - b ? n[b] : n[b] + n[nb - 1 - b]);
-    }
-    const int64_t units = (paired ? (nb + 1) / 2 : nb) * heads;
+    const int64_t units = nb * heads;
     const double cost = kDkvPieceCost * 32. / qtl;
-    // Unsplit, equal workgroups run in whole rounds; single causal blocks,
-    // heaviest first, fill the slots but for a tail.
-    const bool even = paired || !g.causal || g.window > 0;
-    const double unsplit = even || units <= slots ? (double)((units + slots - 1) / slots * unit)
-                                                  : std::max((double)unit, 1.1 * (double)work / (double)slots);
+    // Unsplit, equal blocks run in whole rounds; causal ones, heaviest first,
+    // fill the slots but for a tail.
+    const bool even = !g.causal || g.window > 0;
+    const double unsplit = even || units <= slots ? (double)((units + slots - 1) / slots * n_max)
+                                                  : std::max((double)n_max, 1.1 * (double)work / (double)slots);
     double best = 0.9 * unsplit;
     for (int r = 1; r <= 3; ++r) {
         if (n_tiles * g.hkv > r * slots) continue;

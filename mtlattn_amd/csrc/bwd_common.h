@@ -21,6 +21,7 @@ struct BwdKParams {
     int num_seqs, hq, hkv, g, hpw, n_tiles, n_hg;
     float scale, scale_log2;
     int causal, window;
+    int seq_group;    // one-wave-per-SIMD dK/dV: sequences dispatched together
     int bias_v4;      // bias rows 16-byte aligned (pointer and strides)
     int bias_b32;     // 64 bias rows plus a row's columns span < 2^32 bytes (32-bit buffer offsets)
     const uint16_t* o; int64_t o_rs;   // forward output (dQ with delta_w)
@@ -134,7 +135,7 @@ BwdKParams make_params(const BwdArgs& a) {
     p.total_q = g.total_q; p.total_kv = g.total_kv;
     p.num_seqs = g.num_seqs; p.hq = g.hq; p.hkv = g.hkv; p.g = g.g;
     p.hpw = 1;
-    p.n_tiles = 0; p.n_hg = 0;
+    p.n_tiles = 0; p.n_hg = 0; p.seq_group = g.num_seqs;
     p.scale = g.scale; p.scale_log2 = g.scale * kLog2e;
     p.causal = g.causal; p.window = g.window > 0 ? g.window : 0;
     p.bias_b32 = g.bias != nullptr && (64 * g.bias_qs + g.bias_cols) * 4 < ((int64_t)1 << 32);

@@ -257,7 +257,7 @@ def test_capi_fp32_split_dkv():
 
 @pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,causal,window,bias", [
     ([700, 0, 131, 1, 300], [700, 5, 200, 33, 300], 8, 2, 128, torch.bfloat16, True, 0, None),
-    ([511], [513], 12, 12, 128, torch.float16, False, 0, None),
+    ([1023], [1025], 12, 12, 128, torch.float16, False, 0, None),
     ([1024], [1024], 16, 1, 80, torch.bfloat16, True, 0, None),
     ([513, 640], [900, 700], 16, 4, 96, torch.float16, True, 400, None),
     ([640, 129], [640, 129], 8, 2, 64, torch.float16, True, 0, None),
@@ -339,3 +339,45 @@ def test_capi_splitkv_and_workspace_errors():
     ro, rl = oracle.varlen_forward(q, k, v, cq, ck, scale, True)
     _check("capi-splitkv", [("out", out.cpu(), ro)], torch.bfloat16)
     assert (lse.cpu() - rl).abs().max().item() < LSE_TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,D,causal", [
+    ([700, 1, 0, 256, 257, 511, 3000], 16, 8, 128, True),       # whole kv heads per XCD
+    ([900, 40, 1300], 12, 12, 128, True),                       # one list for all heads
+    ([64] * 66 + [300], 8, 8, 80, True),                        # more sequences than lanes: natural order
+    ([600, 1500] * 10, 8, 8, 128, True),                        # sequences in two halves
+    ([513, 130], 4, 4, 256, True),
+    ([513, 700, 30], 8, 2, 96, False),
+])
+def test_capi_dkv_block_order(lens, Hq, Hkv, D, causal):
+    """The order in which the one-wave-per-SIMD dK/dV takes its key blocks (all
+    sequences' heavy blocks first under causal masking) covers every block of
+    every kv head exactly once: unsplit gradients on NaN-filled outputs against
+    the oracle's, by the RMS error of each sequence (a block left out or taken
+    twice is an error of order 1 in its rows; the roundings of P, dS and the
+    output to bf16 are 2^-9 each, the suite's bound is 8e-3)."""
+    print(f"\\n[case] capi dK/dV block order {lens[:4]} {Hq}/{Hkv} D={D}", flush=True)
+    dtype = torch.bfloat16
+    q, k, v, do, cq, ck = _case(lens, lens, Hq, Hkv, D, dtype, seed=41)
+    qd, kd, vd, dod, cqd, ckd = (t.cuda() for t in (q, k, v, do, cq, ck))
+    scale = 1.0 / math.sqrt(D)
+    p = capi.problem_for(qd, kd, cqd, ckd, max(lens), scale, causal=causal)
+    out = torch.empty_like(qd)
+    lse = torch.empty(qd.shape[0], Hq, dtype=torch.float32, device="cuda")
+    s = _stream()
+    capi.call("mtlattn_varlen_fwd", p, qd.data_ptr(), Hq * D, kd.data_ptr(), Hkv * D, vd.data_ptr(), Hkv * D,
+              out.data_ptr(), lse.data_ptr(), None, 0, s)
+    ws = torch.empty(qd.shape[0] * Hq, dtype=torch.float32, device="cuda")     # delta only: unsplit
+    dq, dk, dv = (torch.full_like(t, float("nan")) for t in (qd, kd, vd))
+    capi.call("mtlattn_varlen_bwd", p, qd.data_ptr(), Hq * D, kd.data_ptr(), Hkv * D, vd.data_ptr(), Hkv * D,
+              out.data_ptr(), Hq * D, dod.data_ptr(), Hq * D, lse.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+              dv.data_ptr(), ws.data_ptr(), ws.numel() * 4, s)
+    torch.cuda.synchronize()
+    _, _, rq, rk, rv = oracle.varlen_forward_backward(q, k, v, do, cq, ck, scale, causal)
+    for nm, a, r in (("dq", dq, rq), ("dk", dk, rk), ("dv", dv, rv)):
+        a = a.cpu().float()
+        assert torch.isfinite(a).all(), nm
+        for i, (b, e) in enumerate(zip(cq[:-1].tolist(), cq[1:].tolist())):
+            err, ref = (a[b:e] - r[b:e]).norm().item(), r[b:e].norm().item()
+            # (a single token's dS cancels to rounding noise: absolute there)
+            assert err <= 8e-3 * ref + 1e-4 * (e - b) ** 0.5, (nm, i, err, ref)
