@@ -772,6 +772,14 @@ int varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, co
                                 bwd_f32_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout,
                                            dout_row_stride) &&
                                 aligned16(out, out_row_stride, p->dtype) && ((uintptr_t)dq & 15u) == 0;
+    // fp32: dQ's (where it computes delta) and dK/dV's partials, each added by
+    // a pass that also clears the rows no sequence owns
+    const bool f32_split = part != nullptr && p->total_q > 0 && p->total_kv > 0 &&
+                           bwd_f32_ok(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride) &&
+                           (((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) & 15u) == 0;
+    if (!is16(p->dtype) && !f32_split) part = nullptr;
+    if (!fuse_delta_f32 || part == nullptr) dq_splits = 1;
+    if (part == nullptr) splits = 1;
     if (fuse_delta) {
         if (q == nullptr || out == nullptr || dout == nullptr || lse == nullptr || dq == nullptr ||
             (p->total_kv > 0 && (k == nullptr || v == nullptr)))
@@ -796,8 +804,11 @@ int varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, co
         a.o_rs = out_row_stride;
         a.delta_out = delta;
         a.f32_part = part;
-        a.f32_splits = part != nullptr ? dq_splits : 1;
+        a.f32_splits = dq_splits;
         rc = launch_status(launch_bwd_dq_f32mfma(a, (hipStream_t)stream), "fp32 dQ");
+        if (rc == MTLATTN_OK && dq_splits > 1)
+            rc = launch_status(launch_f32_bwd_finish(a, part, dq_splits, true, false, (hipStream_t)stream),
+                               "fp32 dQ split sum");
         if (rc != MTLATTN_OK) return rc;
     } else if (p->total_q > 0) {
         rc = mtlattn_bwd_preprocess(p, out, out_row_stride, dout, dout_row_stride, delta, stream);
@@ -811,6 +822,13 @@ int varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, co
     if (rc != MTLATTN_OK || cleared) return rc;
     // Rows outside every sequence take no part in the forward: zero gradient.
     hipStream_t st = (hipStream_t)stream;
+    if (f32_split) {
+        BwdArgs a = make_bwd(p, q, q_row_stride, k, k_row_stride, v, v_row_stride, dout, dout_row_stride, lse, delta);
+        a.dq = dq;
+        a.dk = dk;
+        a.dv = dv;
+        return launch_status(launch_f32_bwd_finish(a, part, splits, dq_splits == 1, true, st), "fp32 dK/dV split sum");
+    }
     const int64_t es = elem_size(p->dtype);
     const int64_t qrow = (int64_t)p->num_heads_q * p->head_dim * es, krow = (int64_t)p->num_heads_kv * p->head_dim * es;
     const ZeroFill fills[3] = {{dq, qrow, p->total_q, p->cu_seqlens_q, dq_rs * es},

@@ -32,6 +32,8 @@
 // one barrier per tile. Row-major tiles use rows of DP + 4 floats (16-byte
 // reads of 16 consecutive rows land in 16 distinct groups of 4 banks),
 // transposed tiles DP rows of 36 floats.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -216,6 +218,7 @@ __device__ inline Tiling tiling(const int* cu, const int* cu_other, int num_seqs
 // workgroup's key tiles over blockIdx.z; f32_fwd_combine_kernel merges the
 // splits' normalised O and LSE.
 // ---------------------------------------------------------------------------
+constexpr int kMaxSplits = 8;   // of every fp32 split (capi.hip)
 template <int DP>
 __global__ __launch_bounds__(256, DP <= 96 ? 2 : 1) void f32_fwd_kernel(F32Params p) {
     constexpr int HD = DP / 2, NB = DP / 32, SR = DP + 4;
@@ -353,23 +356,31 @@ __global__ __launch_bounds__(256) void f32_fwd_combine_kernel(const float* __res
     r1 = r1 < r0 ? r0 : (r1 > total_q ? total_q : r1);
     if (row < r0 || row >= r1) return;
     const float* lp = part + (int64_t)nsplit * plane * d;
+    // every split's LSE and partial in flight together (loads past the last
+    // split repeat it): one after the other, the up to 8 loads' latencies were
+    // most of the pass
+    float lz[kMaxSplits];
+    f32x4_t oz[kMaxSplits];
+#pragma unroll
+    for (int z = 0; z < kMaxSplits; ++z) {
+        const int64_t zr = min(z, nsplit - 1) * plane + rh;
+        lz[z] = lp[zr];
+        oz[z] = ld4(part + zr * d + 4 * c4);
+    }
     // max over the splits that keeps a NaN LSE (a NaN logit in the split):
     // fmaxf would drop it and the row would look empty
     float mx = kNegInf;
-    for (int z = 0; z < nsplit; ++z) {
-        const float lz = lp[z * plane + rh];
-        mx = nan_max(lz, mx);
-        if (mx != mx) break;
-    }
+#pragma unroll
+    for (int z = 0; z < kMaxSplits; ++z) mx = nan_max(lz[z], mx);
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     float sum = 0.f;
     if (mx != kNegInf) {
-        for (int z = 0; z < nsplit; ++z) {
-            const float lz = lp[z * plane + rh];
-            if (lz == kNegInf) continue;
-            const float wz = exp_fp32(lz - mx);
+#pragma unroll
+        for (int z = 0; z < kMaxSplits; ++z) {
+            if (z >= nsplit || lz[z] == kNegInf) continue;
+            const float wz = exp_fp32(lz[z] - mx);
             sum += wz;
-            acc += wz * ld4(part + (z * plane + rh) * d + 4 * c4);
+            acc += wz * oz[z];
         }
     }
     const float inv = !(sum <= 0.f) ? 1.f / sum : 0.f;
@@ -380,7 +391,7 @@ __global__ __launch_bounds__(256) void f32_fwd_combine_kernel(const float* __res
 // ---------------------------------------------------------------------------
 // dQ = scale * dS.K with dS = P * (dP - delta), dP = dO.V^T. Grids with fewer
 // workgroups than the GPU holds split each workgroup's key tiles over
-// blockIdx.z; f32_split_sum_kernel adds the splits in order.
+// blockIdx.z; f32_bwd_finish_kernel adds the splits in order.
 // ---------------------------------------------------------------------------
 template <int DP>
 __global__ __launch_bounds__(256, 1) void f32_dq_kernel(F32Params p) {
@@ -495,7 +506,7 @@ __global__ __launch_bounds__(256, 1) void f32_dq_kernel(F32Params p) {
 // dV = P^T.dO, dK = scale * dS^T.Q, summed over the g query heads of the kv
 // head in a fixed order (no atomics). Grids with fewer workgroups than the
 // GPU holds split the (head, query tile) iterations of each workgroup over
-// blockIdx.z; f32_split_sum_kernel then adds the splits in order z = 0, 1,
+// blockIdx.z; f32_bwd_finish_kernel then adds the splits in order z = 0, 1,
 // ... (deterministic for a given split count).
 // ---------------------------------------------------------------------------
 template <int DP>
@@ -624,24 +635,56 @@ __global__ __launch_bounds__(256, 1) void f32_dkv_kernel(F32Params p) {
     }
 }
 
-// Sum of the splits' partials in order z = 0, 1, ...: out0 = scale0 * sum_z
-// part[z][0], and with out1, out1 = sum_z part[z][1]; a split holds nout
-// arrays of n4 float4 elements (d % 4 == 0).
-__global__ __launch_bounds__(256) void f32_split_sum_kernel(const float* __restrict__ part, int nsplit, int64_t n4,
-                                                            float scale0, float* __restrict__ out0,
-                                                            float* __restrict__ out1) {
+// Sum over the splits, in order z = 0, 1, ..., of element i (float4) of
+// partials whose splits lie `stride` float4 elements apart; all loads in flight
+// together (loads past the last split repeat it and are not added).
+__device__ inline f32x4_t split_sum(const f32x4_t* src, int nsplit, int64_t stride) {
+    f32x4_t x[kMaxSplits];
+#pragma unroll
+    for (int z = 0; z < kMaxSplits; ++z) x[z] = src[min(z, nsplit - 1) * stride];
+    f32x4_t a = x[0];
+#pragma unroll
+    for (int z = 1; z < kMaxSplits; ++z)
+        if (z < nsplit) a += x[z];
+    return a;
+}
+
+// dq, or dk and dv, from their splits' partials, and the rows that no sequence
+// owns cleared; one float4 a thread, grid y = job.
+// With all of an element's loads in flight a pass takes about 3 us where 8
+// dependent loads took 5.6, and the clearing needs no launch of its own.
+struct F32Finish {
+    const float* part;                          // null: the tensor is written, only clear
+    float* out0; float* out1;                   // dq; or dk, dv
+    const int* cu;
+    int64_t total;
+    int row4, nsplit;                           // row in float4 elements
+};
+struct F32FinishJobs {
+    F32Finish job[2];
+    int num_seqs;
+    float scale;
+};
+__global__ __launch_bounds__(256) void f32_bwd_finish_kernel(F32FinishJobs jobs) {
+    const F32Finish& p = jobs.job[blockIdx.y];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t n4 = p.total * p.row4;
     if (i >= n4) return;
-    const int64_t stride = (out1 != nullptr ? 2 : 1) * n4;   // float4 elements per split
-    const f32x4_t* src = reinterpret_cast<const f32x4_t*>(part);
-    f32x4_t a = src[i];
-    for (int z = 1; z < nsplit; ++z) a += src[z * stride + i];
-    reinterpret_cast<f32x4_t*>(out0)[i] = a * scale0;
-    if (out1 != nullptr) {
-        f32x4_t b = src[n4 + i];
-        for (int z = 1; z < nsplit; ++z) b += src[z * stride + n4 + i];
-        reinterpret_cast<f32x4_t*>(out1)[i] = b;
+    const int64_t row = i / p.row4;
+    int64_t r0 = p.cu[0], r1 = p.cu[jobs.num_seqs];
+    r0 = r0 < 0 ? 0 : (r0 > p.total ? p.total : r0);
+    r1 = r1 < r0 ? r0 : (r1 > p.total ? p.total : r1);
+    const bool own = row >= r0 && row < r1;
+    if (own && p.part == nullptr) return;
+    f32x4_t x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+    if (own) {
+        const f32x4_t* src = reinterpret_cast<const f32x4_t*>(p.part) + i;
+        const int64_t stride = (p.out1 != nullptr ? 2 : 1) * n4;
+        x0 = split_sum(src, p.nsplit, stride) * jobs.scale;
+        if (p.out1 != nullptr) x1 = split_sum(src + n4, p.nsplit, stride);
     }
+    reinterpret_cast<f32x4_t*>(p.out0)[i] = x0;
+    if (p.out1 != nullptr) reinterpret_cast<f32x4_t*>(p.out1)[i] = x1;
 }
 
 F32Params make_params(const Geometry& g) {
@@ -704,11 +747,7 @@ hipError_t launch_bwd_dq_f32mfma(const BwdArgs& a, hipStream_t st) {
     p.nsplit = splits;
     hipError_t e = launch(p, a.geo.total_q, a.geo.hq, st, f32_dq_kernel<32>, f32_dq_kernel<64>, f32_dq_kernel<96>,
                           f32_dq_kernel<128>, splits);
-    if (e != hipSuccess || splits == 1 || a.geo.total_q <= 0) return e;
-    const int64_t n4 = a.geo.total_q * a.geo.hq * a.geo.d / 4;
-    hipLaunchKernelGGL(f32_split_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, p.part, splits,
-                       n4, p.scale, p.dq, nullptr);
-    return hipGetLastError();
+    return e;
 }
 
 hipError_t launch_bwd_dkv_f32mfma(const BwdArgs& a, hipStream_t st) {
@@ -721,10 +760,34 @@ hipError_t launch_bwd_dkv_f32mfma(const BwdArgs& a, hipStream_t st) {
     p.nsplit = splits;
     hipError_t e = launch(p, a.geo.total_kv, a.geo.hkv, st, f32_dkv_kernel<32>, f32_dkv_kernel<64>,
                           f32_dkv_kernel<96>, f32_dkv_kernel<128>, splits);
-    if (e != hipSuccess || splits == 1 || a.geo.total_kv <= 0) return e;
-    const int64_t n4 = a.geo.total_kv * a.geo.hkv * a.geo.d / 4;
-    hipLaunchKernelGGL(f32_split_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, p.part, splits,
-                       n4, p.scale, p.dk, p.dv);
+    return e;
+}
+
+hipError_t launch_f32_bwd_finish(const BwdArgs& a, const float* part, int splits, bool dq, bool dkv, hipStream_t st) {
+    const Geometry& g = a.geo;
+    if (splits > kMaxSplits) return hipErrorInvalidValue;
+    F32FinishJobs jobs{};
+    jobs.num_seqs = g.num_seqs;
+    jobs.scale = g.scale;
+    int n = 0;
+    int64_t most = 0;
+    // (with both, dq has no partials)
+    if (dq) {
+        jobs.job[n] = F32Finish{dkv || splits == 1 ? nullptr : part, (float*)a.dq, nullptr, g.cu_q, g.total_q,
+                                g.hq * g.d / 4, splits};
+        most = std::max(most, jobs.job[n].total * jobs.job[n].row4);
+        ++n;
+    }
+    if (dkv) {
+        jobs.job[n] = F32Finish{splits == 1 ? nullptr : part, (float*)a.dk, (float*)a.dv, g.cu_kv, g.total_kv,
+                                g.hkv * g.d / 4, splits};
+        most = std::max(most, jobs.job[n].total * jobs.job[n].row4);
+        ++n;
+    }
+    const int64_t blocks = (most + 255) / 256;
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    if (n == 0 || blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(f32_bwd_finish_kernel, dim3((unsigned)blocks, (unsigned)n), dim3(256), 0, st, jobs);
     return hipGetLastError();
 }
 

@@ -98,8 +98,8 @@ struct BwdArgs {
     float* delta_out = nullptr;
     // fp32 matrix-core dQ and dK/dV only: f32_splits > 1 splits each
     // workgroup's work over that many workgroups, with fp32 partials in
-    // f32_part (f32_dq_part_floats / f32_dkv_part_floats floats) summed in a
-    // fixed order afterwards; dQ also takes o / delta_out (delta in-kernel)
+    // f32_part (f32_dq_part_floats / f32_dkv_part_floats floats), which
+    // launch_f32_bwd_finish adds in a fixed order; dQ also takes o / delta_out (delta in-kernel)
     float* f32_part = nullptr;
     int f32_splits = 1;
     // 16-bit dK/dV only: with dkv_plan.pieces > 1 a launch of dkv_plan.grid
@@ -156,6 +156,10 @@ hipError_t launch_bwd_dkv_generic(int dtype, const BwdArgs& a, hipStream_t st);
 hipError_t launch_fwd_f32mfma(const FwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_dq_f32mfma(const BwdArgs& a, hipStream_t st);
 hipError_t launch_bwd_dkv_f32mfma(const BwdArgs& a, hipStream_t st);
+// The splits' partials of dq, or of dk and dv, added into them (splits 1:
+// already written), and their rows that no sequence owns cleared. With both,
+// dq is only cleared.
+hipError_t launch_f32_bwd_finish(const BwdArgs& a, const float* part, int splits, bool dq, bool dkv, hipStream_t st);
 // Rows of a [total_rows, row_bytes] tensor (row stride stride_bytes, 0:
 // contiguous) outside [cu[0], cu[num_seqs]).
 struct ZeroFill {
