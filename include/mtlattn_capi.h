@@ -127,8 +127,8 @@ int mtlattn_varlen_fwd(const mtlattn_problem* p,
  * memory -- code under HIP graph capture, tight serving (decode) loops,
  * harnesses that forbid allocation. Same routing, kernels and results as
  * mtlattn_varlen_fwd (bitwise); the split-KV partials of calls routed to
- * decode, and the fp32 key-split partials (sized to fit it), live in a
- * static device array of MTLATTN_NOALLOC_SCRATCH_BYTES per
+ * decode, and the key-split partials of fp32 and 16-bit forwards on small
+ * grids (sized to fit it), live in a static device array of MTLATTN_NOALLOC_SCRATCH_BYTES per
  * GPU, set up on the first call on each GPU (do that call outside capture)
  * and held until the process ends. Calls whose partials would exceed it
  * (mtlattn_varlen_fwd_workspace_size(p) > MTLATTN_NOALLOC_SCRATCH_BYTES)
