@@ -299,13 +299,62 @@ def _basic_ok(query, key, value, dropout_p, min_seqlen):
     return query.shape[2] >= min_seqlen
 
 
-# The padding path's one host decision -- a device reduction read back to the
-# host -- is made once per mask tensor and reused while that tensor is alive
-# and unmodified (same object, version counter, storage, shape and strides):
-# a model passes the same mask to every layer's attention call, so a forward
-# pass waits on the device once for it, not once per layer. Entries go when
-# their mask is freed.
+# The padding path needs one host decision about the mask, which its content
+# decides: a device reduction read back to the host. It is kept per mask tensor
+# while that tensor is alive, because a model passes the same mask to every
+# layer's attention call, together with a copy of the content it was made from
+# (a broadcast dim once). A kept "padding" is compared with the mask on every
+# call, whatever wrote to it (the version counter misses .data, other kernels
+# on the same memory and graph replays, and an inference-mode tensor has none);
+# the answer travels to the host while the attention is already launched, so
+# the GPU does not wait for it. A kept "not padding" only leaves the call to
+# the additive-bias path, right for any mask, and is not compared. Masks whose
+# content takes more than _PAD_COPY_BYTES are decided on every call.
 _PAD_DECISIONS = {}
+_PAD_COPY_BYTES = 16 << 20
+
+
+class _Answer:
+    """A device bool on its way to the host; bool() waits for it."""
+
+    def __init__(self, flag):
+        self._host, self._event = flag, None
+        if flag.is_cuda:
+            with torch.cuda.device(flag.device):
+                self._host = torch.empty((), dtype=torch.bool, pin_memory=True)
+                self._host.copy_(flag, non_blocking=True)
+                self._event = torch.cuda.Event()
+                self._event.record()
+
+    def __bool__(self):
+        if self._event is not None:
+            self._event.synchronize()
+        return bool(self._host)
+
+
+def _mask_content(attn_mask):
+    """The mask with its broadcast (stride 0) dims narrowed to one entry."""
+    return attn_mask.detach()[tuple(slice(0, 1) if st == 0 else slice(None) for st in attn_mask.stride())]
+
+
+def _mask_signature(attn_mask, B, Hq, Nq, Nkv):
+    version = None if attn_mask.is_inference() else attn_mask._version
+    return (version, attn_mask.data_ptr(), tuple(attn_mask.shape), tuple(attn_mask.stride()), attn_mask.dtype,
+            B, Hq, Nq, Nkv)
+
+
+def _kept_decision(attn_mask, B, Hq, Nq, Nkv):
+    """(ok, lens, holds) of the decision kept for this mask, or None. `holds` is
+    true when it still stands; asking it may wait for the device."""
+    hit = _PAD_DECISIONS.get(id(attn_mask))
+    if hit is None or hit[0]() is not attn_mask or hit[1] != _mask_signature(attn_mask, B, Hq, Nq, Nkv):
+        return None
+    _, _, ok, lens, content = hit
+    # (under graph capture nothing can be read back: a decision made before it
+    # goes into the graph, as its launches do)
+    if not ok or (attn_mask.is_cuda and torch.cuda.is_current_stream_capturing()):
+        return ok, lens, True
+    return ok, lens, _Answer((_mask_content(attn_mask) == content).all())
 
 
 def _padding_decision(attn_mask, B, Hq, Nq, Nkv):
@@ -313,15 +362,17 @@ def _padding_decision(attn_mask, B, Hq, Nq, Nkv):
     depends only on (batch, key) with the kept keys a prefix (and, for a float
     mask, adds exactly 0 to them); lens = kept keys per batch (int32, on the
     mask's device), or None when the mask does not broadcast to that shape.
-    Cached per mask tensor (see _PAD_DECISIONS)."""
-    sig = (attn_mask._version, attn_mask.data_ptr(), tuple(attn_mask.shape), tuple(attn_mask.stride()),
-           B, Hq, Nq, Nkv)
-    hit = _PAD_DECISIONS.get(id(attn_mask))
-    if hit is not None and hit[0]() is attn_mask and hit[1] == sig:
-        return hit[2], hit[3]
-    keep0 = attn_mask if attn_mask.dtype == torch.bool else attn_mask > -1e30
+    Kept per mask tensor (see _PAD_DECISIONS)."""
+    kept = _kept_decision(attn_mask, B, Hq, Nq, Nkv)
+    if kept is not None and kept[2]:
+        return kept[:2]
+    content = _mask_content(attn_mask)
+    small = content.numel() * content.element_size() <= _PAD_COPY_BYTES
+    if small:
+        content = content.clone()
+    keep0 = content if content.dtype == torch.bool else content > -1e30
     try:
-        keep = keep0.expand(B, Hq, Nq, Nkv)
+        keep = keep0.expand(attn_mask.shape).expand(B, Hq, Nq, Nkv)
     except RuntimeError:
         return False, None
     kv_keep = keep[:, 0, 0, :]
@@ -331,13 +382,17 @@ def _padding_decision(attn_mask, B, Hq, Nq, Nkv):
     # broadcast shape, not the expanded [B, H, N, N]
     ok = torch.logical_and((keep0 == kv_keep[:, None, None, :]).all(),
                            (kv_keep == (idx[None, :] < lens[:, None])).all())
-    if attn_mask.dtype != torch.bool:
+    if content.dtype != torch.bool:
         # a float mask is a padding mask only if it adds nothing to the keys
         # it keeps (else its values are an additive bias)
-        ok = torch.logical_and(ok, (attn_mask.masked_fill(~keep0, 0) == 0).all())
+        ok = torch.logical_and(ok, (content.masked_fill(~keep0, 0) == 0).all())
     ok = bool(ok)
     k = id(attn_mask)
-    _PAD_DECISIONS[k] = (weakref.ref(attn_mask, lambda _r, k=k: _PAD_DECISIONS.pop(k, None)), sig, ok, lens)
+    if ok and not small:
+        _PAD_DECISIONS.pop(k, None)
+        return ok, lens
+    _PAD_DECISIONS[k] = (weakref.ref(attn_mask, lambda _r, k=k: _PAD_DECISIONS.pop(k, None)),
+                         _mask_signature(attn_mask, B, Hq, Nq, Nkv), ok, lens, content if ok else None)
     return ok, lens
 
 
@@ -353,10 +408,21 @@ def _try_padding_varlen(query, key, value, attn_mask, is_causal, scale):
     Hkv, Nkv = key.shape[1], key.shape[2]
     if Nq != Nkv:
         return None
-    # the one host decision, made once per mask tensor (_padding_decision)
+    kept = _kept_decision(attn_mask, B, Hq, Nq, Nkv)
+    if kept is not None:
+        ok, lens, holds = kept
+        # (launched before the answer is read)
+        out = _padded_attention(query, key, value, lens, is_causal, scale) if ok else None
+        if holds:
+            return out
     ok, lens = _padding_decision(attn_mask, B, Hq, Nq, Nkv)
-    if not ok:
-        return None
+    return _padded_attention(query, key, value, lens, is_causal, scale) if ok else None
+
+
+def _padded_attention(query, key, value, lens, is_causal, scale):
+    """Self-attention over the first lens[b] tokens of each batch, the other
+    query rows 0."""
+    B, _, Nq, _ = query.shape
     out = _dense(query, key, value, scale, is_causal, lens)
     if out is not None:
         return out

@@ -180,6 +180,55 @@ def test_padding_decision_cached_per_mask():
     assert k not in M._PAD_DECISIONS
 
 
+def _prefix_mask(lens, N):
+    return (torch.arange(N)[None] < torch.tensor(lens)[:, None])[:, None, None, :]
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.float32])
+def test_padding_decision_follows_the_masks_content(monkeypatch, dtype):
+    """A kept decision is not used for a mask that something else rewrote:
+    .data, like other kernels on the same memory, leaves the version counter
+    as it is. Also for a mask expanded over heads and rows, and for one whose
+    content is too large to keep."""
+    B, H, N = 2, 3, 8
+
+    def mask(lens):
+        m = _prefix_mask(lens, N)
+        return m if dtype == torch.bool else torch.zeros(m.shape).masked_fill(~m, float("-inf"))
+
+    for expand in (False, True):
+        for limit in (M._PAD_COPY_BYTES, 0):
+            monkeypatch.setattr(M, "_PAD_COPY_BYTES", limit)
+            base = mask([8, 4])
+            m = base.expand(B, H, N, N) if expand else base
+            for _ in range(2):
+                ok, lens = M._padding_decision(m, B, H, N, N)
+                assert ok and lens.tolist() == [8, 4]
+            version = m._version
+            base.data.copy_(mask([6, 5]))
+            assert m._version == version
+            ok, lens = M._padding_decision(m, B, H, N, N)
+            assert ok and lens.tolist() == [6, 5]
+            base.data[0, 0, 0, 1] = base[0, 0, 0, 7]        # a hole: no prefix any more
+            assert not M._padding_decision(m, B, H, N, N)[0]
+
+
+def test_padding_decision_of_inference_mode_mask():
+    """A mask made under inference_mode has no version counter to read."""
+    with torch.inference_mode():
+        m = _prefix_mask([5, 2], 8)
+        for _ in range(2):
+            ok, lens = M._padding_decision(m, 2, 3, 8, 8)
+            assert ok and lens.tolist() == [5, 2]
+        m[1, 0, 0, 2] = True
+        assert M._padding_decision(m, 2, 3, 8, 8)[1].tolist() == [5, 3]
+        hole = _prefix_mask([5, 2], 8)
+        hole[:, :, :, 0] = False
+        q = torch.randn(2, 3, 8, 8)
+        assert M._try_padding_varlen(q, q, q, hole, False, 0.3) is None
+    assert M._padding_decision(m, 2, 3, 8, 8)[1].tolist() == [5, 3]
+
+
 def test_binding_rejects_cpu_tensors():
     q = torch.randn(4, 2, 8)
     cu = torch.tensor([0, 4], dtype=torch.int32)

@@ -90,3 +90,58 @@ def test_dense_refusals():
                   ((q.clone().requires_grad_(), q, q), {})):
         assert mt._dense(*a, 0.1, False, **kw) is None, [tuple(t.shape) for t in a]
     assert mt._dense(q, q, q, -0.1, False) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_padding_mask_rewritten_or_made_in_inference_mode(dtype):
+    """Under replace_sdpa() a key-padding mask is taken as it is at each call:
+    rewritten through .data (the version counter stays), made under
+    inference_mode (it has none), turned into another kind of mask; and a call
+    recorded into a graph repeats what it recorded. Valid rows against the
+    original on fp32 copies."""
+    import mtlattn_amd as mt
+    print(f"\n[case] padding mask content {dtype}", flush=True)
+    B, H, N, D = 3, 4, 130, 64
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (randn((B, H, N, D), dtype, g).cuda() for _ in range(3))
+    j = torch.arange(N, device="cuda")
+    orig = torch.nn.functional.scaled_dot_product_attention
+
+    def prefix(lens):
+        return (j[None] < torch.tensor(lens, device="cuda")[:, None])[:, None, None, :]
+
+    def check(m, lens):
+        out = torch.nn.functional.scaled_dot_product_attention(q, k, v, attn_mask=m)
+        ref = orig(q.float().cpu(), k.float().cpu(), v.float().cpu(), attn_mask=prefix(lens).cpu()).cuda()
+        for b, n in enumerate(lens):
+            assert (out[b, :, :n].float() - ref[b, :, :n]).abs().max() < (2e-2 if dtype == torch.bfloat16 else 1e-5)
+            assert not out[b, :, n:].any()
+        return out
+
+    mt.replace_sdpa(min_seqlen=64)
+    try:
+        with torch.no_grad():
+            m = prefix([130, 64, 1])
+            for _ in range(3):
+                check(m, [130, 64, 1])
+            m.data.copy_(prefix([100, 130, 33]))
+            for _ in range(2):
+                want = check(m, [100, 130, 33])
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = torch.nn.functional.scaled_dot_product_attention(q, k, v, attn_mask=m)
+            for _ in range(3):
+                out.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, want)
+                check(m, [100, 130, 33])
+            m.data[:, :, :, 0] = False                      # no prefix any more: padded rows attend too
+            got = torch.nn.functional.scaled_dot_product_attention(q, k, v, attn_mask=m)
+            assert torch.equal(got, orig(q, k, v, attn_mask=m))
+        with torch.inference_mode():
+            m = prefix([5, 130, 70])
+            for _ in range(2):
+                check(m, [5, 130, 70])
+    finally:
+        mt.restore_sdpa()
