@@ -64,7 +64,11 @@ typedef struct mtlattn_problem {
     int32_t num_heads_q;      /* Hq */
     int32_t num_heads_kv;     /* Hkv; Hq % Hkv == 0 */
     int32_t head_dim;         /* D */
-    int32_t max_seqlen_q;     /* caller's bound on q lengths (decode routing only) */
+    int32_t max_seqlen_q;     /* caller's bound on q lengths: up to 16 routes to decode. Too
+                               * small a bound: rows past a sequence's first 16 / (heads per
+                               * group) are computed slowly on calls that decode runs one
+                               * workgroup per item (fewer than 2048 keys a sequence, or K
+                               * and V below 0.9 GB), and left unwritten on the others */
     float scale;              /* logit = scale * q.k (+ bias) */
     int32_t causal;           /* 0 / 1 */
     int32_t window;           /* <= 0: no sliding window */

@@ -339,6 +339,72 @@ __global__ __launch_bounds__(kDecWaves * 64) void decode_split_kernel(DecKParams
     }
 }
 
+// Rows of a head group past the 16 that max_seqlen_q promised (it was too
+// small): one wave each, all the sequence's keys, in fp32 on the VALU -- 64 keys
+// a step, lane = key for the scores, lane = column for the output. Slow and
+// rarely reached (about 1 us a step); the matrix-core passes over 16 rows in a
+// loop cost the calls that never repeat them 5% (1 us of 20).
+template <typename T, int D, bool BIAS, bool PAGED>
+__device__ inline void extra_rows(const DecKParams& p, typename T::raw* __restrict__ out, float* __restrict__ lse_out,
+                                  int s, int hk, int hgi, int w, int nw, int lane) {
+    constexpr int DU = D / 64;                       // output columns per lane: lane + 64 j
+    const SeqRange qr = seq_range(p.cu_q, s, p.total_q), kr = seq_range(p.cu_kv, s, p.total_kv);
+    const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start, coff = kv_len - q_len;
+    auto cache_row = [&](int key) -> int64_t {       // of K and V
+        if (!PAGED) return kr.start + key;
+        const int* bt = p.block_table + (int64_t)s * p.bt_stride;
+        const int col = min(key / p.page_size, (int)min(p.bt_stride, (int64_t)0x7fffffff) - 1);
+        return (int64_t)min(max(bt[col], 0), p.num_pages - 1) * p.page_size + key % p.page_size;
+    };
+    for (int n = 16 + w; n < p.hpb * q_len; n += nw) {
+        const int hh = n / q_len, qi = n - hh * q_len, head = hk * p.g + hgi * p.hpb + hh;
+        const int64_t grow = qr.start + qi;
+        const uint16_t* qp = p.q + grow * p.q_rs + (int64_t)head * D;
+        const float* brow = nullptr;
+        if (BIAS)
+            brow = p.bias + bias_row_offset(grow, s, qr.start, p.bias_qs, p.bias_ss, p.bias_rows) +
+                   (int64_t)head * p.bias_hs;
+        const int lo = p.window > 0 ? max(0, qi + coff - p.window + 1) : 0;
+        const int hi = p.causal ? min(kv_len, qi + coff + 1) : kv_len;
+        float m = kNegInf, l = 0.f, acc[DU] = {};
+        for (int kt = lo; kt < hi; kt += 64) {
+            const int key = min(kt + lane, hi - 1);
+            const uint16_t* kp = p.k + cache_row(key) * p.k_rs + (int64_t)hk * D;
+            float x = 0.f;
+#pragma unroll 2
+            for (int c = 0; c < D; c += 8) {
+                const u32x4_t a = ld16(qp + c), b = ld16(kp + c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x = fmaf(lo16<T>(a[e]), lo16<T>(b[e]), x);
+                    x = fmaf(hi16<T>(a[e]), hi16<T>(b[e]), x);
+                }
+            }
+            x *= p.scale_log2;
+            if (BIAS && key < p.bias_cols) x = fmaf(brow[key], kLog2e, x);
+            x = kt + lane < hi ? x : kNegInf;
+            const float m_new = fmaxf(m, wave_max(x)), m_use = m_new == kNegInf ? 0.f : m_new;
+            const float corr = __builtin_amdgcn_exp2f(m - m_use), e = __builtin_amdgcn_exp2f(x - m_use);
+            m = m_new;
+            l = l * corr + e;
+#pragma unroll
+            for (int j = 0; j < DU; ++j) acc[j] *= corr;
+            for (int i = 0; i < 64 && kt + i < hi; ++i) {
+                const float pi = __shfl(e, i);
+                const uint16_t* vp = p.v + cache_row(kt + i) * p.v_rs + (int64_t)hk * D + lane;
+#pragma unroll
+                for (int j = 0; j < DU; ++j) acc[j] = fmaf(pi, T::to_float(vp[64 * j]), acc[j]);
+            }
+        }
+        l = wave_sum(l);
+        const int64_t rh = grow * p.hq + head;
+#pragma unroll
+        for (int j = 0; j < DU; ++j)
+            out[rh * D + lane + 64 * j] = T::from_float(!(l <= 0.f) ? acc[j] / l : 0.f);
+        if (lse_out != nullptr && lane == 0) lse_out[rh] = !(l <= 0.f) ? m * kLn2 + logf(l) : kNegInf;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Decode with the split inside the workgroup: one workgroup of NW waves per
 // work item (a sequence, or a KV chunk of it) and (kv head, head group). Wave
@@ -359,8 +425,9 @@ __global__ __launch_bounds__(kDecWaves * 64) void decode_split_kernel(DecKParams
 // (64 sequences of 8192 to 65536 keys, 64/8 heads: 1572 against 1713 us).
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool BIAS, bool PAGED, int NW>
-__global__ __launch_bounds__(NW * 64) void decode_wg_kernel(DecKParams p, typename T::raw* __restrict__ out,
-                                                            float* __restrict__ lse_out) {
+// (8 waves, D = 64: two workgroups on a CU)
+__global__ __launch_bounds__(NW * 64, D == 64 && NW == 8 && !PAGED ? 4 : 1) void decode_wg_kernel(
+    DecKParams p, typename T::raw* __restrict__ out, float* __restrict__ lse_out) {
     constexpr int KC = D / 32, DB = D / 16, VU = D / 64;
     constexpr int OROW = D * 4 + 16;                 // bytes of an fp32 O row in LDS (padded: 16 rows, one column)
     constexpr int REGION = 16 * OROW > D * kDecKT * 2 ? 16 * OROW : D * kDecKT * 2;   // per wave: V^T tile, then O
@@ -377,14 +444,14 @@ __global__ __launch_bounds__(NW * 64) void decode_wg_kernel(DecKParams p, typena
     const int slot = wid / p.n_hg;
     int s, ks, ke;
     const bool has_keys = item_range(p, slot, s, ks, ke);
-    if (!has_keys && p.chunk > 0) return;
+    if (!has_keys && p.chunk > 0 && ks > 0) return;
     const SeqRange qr = seq_range(p.cu_q, s, p.total_q);
     const SeqRange kr = seq_range(p.cu_kv, s, p.total_kv);
     const int q_len = qr.end - qr.start, kv_len = kr.end - kr.start;
     if (q_len == 0) return;
     const int coff = kv_len - q_len;
 
-    // (rows past the 16-row group, max_seqlen_q too small, are left untouched)
+    // (rows past the 16-row group: extra_rows, at the end)
     const int rows = min(p.hpb * q_len, 16);
     const bool row_ok = n16 < rows;
     const int hh = row_ok ? n16 / q_len : 0;
@@ -590,12 +657,16 @@ __global__ __launch_bounds__(NW * 64) void decode_wg_kernel(DecKParams p, typena
             if (d == 0) p.lse_part[prow] = lse;
         }
     }
+    // the item of a sequence's first keys sees to the rows past the 16-row group
+    if (p.hpb * q_len > 16 && (whole || ks == 0))
+        extra_rows<T, D, BIAS, PAGED>(p, out, lse_out, s, hk, hgi, w, NW, lane);
 }
 
 // One wave per (row, head): O = sum_i w_i O_i / sum_i w_i over the work items
 // of the row's sequence, w_i = exp(lse_i - max lse). Rows outside every
-// sequence, or beyond the 16-row group (max_seqlen_q too small), are left
-// untouched as the flash forward leaves them.
+// sequence are left untouched as the flash forward leaves them; rows beyond
+// the 16-row group (max_seqlen_q too small) are extra_rows', and untouched
+// after the one-wave kernel.
 template <typename T>
 __global__ __launch_bounds__(256) void decode_combine_kernel(DecKParams p, typename T::raw* __restrict__ out,
                                                              float* __restrict__ lse_out, int d) {

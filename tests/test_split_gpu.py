@@ -80,6 +80,31 @@ def test_decode_workgroup(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window, bi
         _check(f"workspace={ws} ({need} bytes)", out, lse, ref, ref_lse, dtype)
 
 
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,max_q,window,bias", [
+    ([1, 40, 0, 17], [200, 300, 9, 17], 8, 2, 128, torch.bfloat16, 1, 0, None),     # whole sequences
+    ([5, 16, 33], [700, 16, 0], 8, 8, 64, torch.float16, 4, 0, None),               # (one without keys)
+    ([3, 18], [400, 600], 8, 2, 128, torch.bfloat16, 2, 100, "head"),
+    ([1] * 40 + [20], [50] * 41, 32, 8, 128, torch.float16, 3, 0, None),
+    ([20], [1999], 8, 2, 128, torch.bfloat16, 1, 0, None),                          # chunks
+    ([2, 17, 18], [5100, 0, 900], 4, 4, 64, torch.float16, 2, 0, "broadcast"),
+])
+def test_short_calls_with_too_small_max_seqlen_q(q_lens, kv_lens, Hq, Hkv, D, dtype, max_q, window, bias):
+    """Below 2048 keys a sequence max_seqlen_q only routes: sequences with more
+    queries than it says are attended in full."""
+    print(f"\n[case] max_seqlen_q {max_q} for {q_lens[-4:]} D={D} {dtype} {kv_lens[-4:]}", flush=True)
+    q, k, v = _inputs(q_lens, kv_lens, Hq, Hkv, D, dtype, 8)
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    b = None
+    if bias:
+        b = torch.randn(sum(q_lens), 1 if bias == "broadcast" else Hq, max(kv_lens),
+                        generator=torch.Generator().manual_seed(4))
+    ref, ref_lse = oracle.varlen_forward(q, k, v, cq, ck, 1.0 / math.sqrt(D), True, window, b)
+    dev = [t.cuda() for t in (q, k, v, cq, ck)]
+    for ws in (True, False):
+        out, lse, need = _fwd(*dev, max_q, True, window, None if b is None else b.cuda(), ws)
+        _check(f"workspace={ws} ({need} bytes)", out, lse, ref, ref_lse, dtype)
+
+
 @pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,causal,window", [
     ([512, 130], [4096, 9000], 8, 2, 128, torch.bfloat16, True, 0),
     ([32], [6000], 16, 2, 128, torch.float16, True, 0),
