@@ -1437,16 +1437,17 @@ DkvPlan make_dkv_plan(const Geometry& g, int cus) {
                                                   : std::max((double)n_max, 1.1 * (double)work / (double)slots);
     double best = 0.9 * unsplit;
     for (int r = 1; r <= 3; ++r) {
-        if (n_tiles * g.hkv > r * slots) continue;
-        auto wgs = [&](int64_t c) {
-            int64_t x = 0;
-            for (int64_t b = 0; b < nb; ++b) x += std::max<int64_t>(1, (n[b] + c - 1) / c);
-            return x * heads;
+        const int64_t grid = r * slots, c0 = std::max<int64_t>(kDkvMinPiece, (n_max + max_pieces - 1) / max_pieces);
+        if (n_tiles * g.hkv > grid) continue;
+        auto time = [&](int64_t c, int64_t wgs) {
+            return (r == 1 ? (double)c : (double)work / (double)slots + 0.5 * (double)c) + cost * r +
+                   cost * (double)wgs / (double)slots;
         };
-        int64_t c = std::max<int64_t>(kDkvMinPiece, (n_max + max_pieces - 1) / max_pieces);
-        while (c < n_max && wgs(c) > r * slots) ++c;
-        const double t = (r == 1 ? (double)c : (double)work / (double)slots + 0.5 * (double)c) + cost * r +
-                         cost * (double)wgs(c) / (double)slots;
+        // (no piece length that fits the grid can beat this)
+        if (time(std::max(c0, (work + grid - 1) / grid), units) >= best) continue;
+        int64_t wgs = 0;
+        const int64_t c = plan_piece(n, nb, heads, grid, c0, n_max, &wgs);
+        const double t = time(c, wgs);
         if (c < n_max && t < best) {
             best = t;
             // (sequences longer than the average have more pieces)

@@ -582,9 +582,9 @@ DkvPlan dkv_plan(const mtlattn_problem* p) {
 
 // fp32 partial bytes after delta: 16-bit dK/dV's; or fp32 dQ's, then (in the
 // same space, after the dQ splits are summed) dK/dV's
-size_t bwd_part_bytes(const mtlattn_problem* p) {
+size_t bwd_part_bytes(const mtlattn_problem* p, const DkvPlan& plan) {
     if (is16(p->dtype))
-        return (size_t)dkv_part_floats(dkv_plan(p).pieces, p->total_kv, p->num_heads_kv, p->head_dim) * sizeof(float);
+        return (size_t)dkv_part_floats(plan.pieces, p->total_kv, p->num_heads_kv, p->head_dim) * sizeof(float);
     const int64_t fq = f32_dq_part_floats(f32_dq_splits(p), p->total_q, p->num_heads_q, p->head_dim);
     const int64_t fk = f32_dkv_part_floats(f32_dkv_splits(p), p->total_kv, p->num_heads_kv, p->head_dim);
     return (size_t)std::max<int64_t>(fq, fk) * sizeof(float);
@@ -594,7 +594,7 @@ size_t bwd_part_bytes(const mtlattn_problem* p) {
 
 size_t mtlattn_varlen_bwd_workspace_size(const mtlattn_problem* p) {
     if (check_problem(p) != MTLATTN_OK) return 0;
-    const size_t part = bwd_part_bytes(p);
+    const size_t part = bwd_part_bytes(p, dkv_plan(p));
     if (part > 0) return bwd_part_offset(p) + part;
     return bwd_delta_bytes(p);
 }
@@ -755,7 +755,7 @@ int varlen_bwd(const mtlattn_problem* p, const void* q, int64_t q_row_stride, co
     const DkvPlan plan = dkv_plan(p);
     bool cleared = false;
     float* part = nullptr;
-    const size_t part_bytes = bwd_part_bytes(p);
+    const size_t part_bytes = bwd_part_bytes(p, plan);
     if (part_bytes > 0 && workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 &&
         workspace_bytes >= bwd_part_offset(p) + part_bytes)
         part = (float*)((char*)workspace + bwd_part_offset(p));

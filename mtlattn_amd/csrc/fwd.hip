@@ -946,14 +946,12 @@ FwdPlan make_fwd_plan(const Geometry& g, int max_q, int cus, size_t max_bytes) {
         const int64_t grid = std::min(full, ((int64_t)(max_bytes / sizeof(float)) - ints) / (rows * (g.d + 1)) / 8 * 8);
         if (n_tiles * n_hg > grid) continue;
         const size_t bytes = (size_t)(ints + grid * rows * (g.d + 1)) * sizeof(float);
-        auto wgs = [&](int64_t c) {
-            int64_t x = 0;
-            for (int64_t i = 0; i < nt; ++i) x += std::max<int64_t>(1, (n[i] + c - 1) / c);
-            return x * g.num_seqs * n_hg;
-        };
-        int64_t c = min_piece;
-        while (c < n_max && wgs(c) > grid) ++c;
-        const double t = (double)c * (wgs(c) <= cus ? 1. : pair) + kFwdSplitCost * 64. / kt;
+        const double cost = kFwdSplitCost * 64. / kt;
+        // (no piece length that fits the grid can beat this)
+        if ((double)std::max<int64_t>(min_piece, (work + grid - 1) / grid) + cost >= best) continue;
+        int64_t wgs = 0;
+        const int64_t c = plan_piece(n, nt, g.num_seqs * n_hg, grid, min_piece, n_max, &wgs);
+        const double t = (double)c * (wgs <= cus ? 1. : pair) + cost;
         if (c < n_max && t < best) {
             best = t;
             plan.grid = (int)grid;

@@ -2,6 +2,8 @@
 // Included by the kernel sources and by the C ABI (capi.hip); not installed.
 #pragma once
 
+#include <algorithm>
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -63,6 +65,37 @@ struct DenseArgs {
     int nq, nkv;
 };
 inline bool dense_head_dim(int d) { return d == 64 || d == 80 || d == 88 || d == 96 || d == 128; }
+
+// Piece length of a split plan: the smallest c >= c0 for which mult times the
+// pieces of c steps of all tiles (n[0 .. tiles) steps each, at least one piece a
+// tile) are at most `limit`, or n_max if only whole tiles are; *wgs is that
+// count of pieces. By bisection between the bounds that the sum of the steps
+// gives: a plan is made on every call, and at 256 tiles of thousands of steps a
+// search step by step took up to 85 ms.
+inline int64_t plan_piece(const int64_t* n, int64_t tiles, int64_t mult, int64_t limit, int64_t c0, int64_t n_max,
+                          int64_t* wgs) {
+    int64_t sum = 0;
+    for (int64_t i = 0; i < tiles; ++i) sum += n[i];
+    auto count = [&](int64_t c) {
+        int64_t x = 0;
+        for (int64_t i = 0; i < tiles; ++i) x += n[i] > c ? (n[i] + c - 1) / c : 1;
+        return x * mult;
+    };
+    int64_t hi = c0;
+    if (c0 < n_max && (*wgs = count(c0)) > limit) {
+        // lo does not fit; hi does, or is n_max
+        int64_t lo = c0;
+        hi = n_max;
+        if (limit > 0) lo = std::max(lo, (sum * mult + limit - 1) / limit - 1);
+        if (limit > tiles * mult) hi = std::min(hi, sum * mult / (limit - tiles * mult) + 1);
+        while (hi - lo > 1) {
+            const int64_t mid = (lo + hi) / 2;
+            if (count(mid) > limit) lo = mid; else hi = mid;
+        }
+    }
+    *wgs = count(hi);
+    return hi;
+}
 
 // How the 16-bit dK/dV cuts its work (make_dkv_plan): pieces == 1: one
 // workgroup per key block or pair of key blocks; else at most `pieces` pieces

@@ -282,3 +282,24 @@ def test_ctypes_binding_covers_header():
         n = 0 if params.strip() in ("", "void") else params.count(",") + 1
         assert len(capi.SIGNATURES[name][1]) == n, name
     assert capi.lib().mtlattn_abi_version() == capi.ABI_VERSION
+
+
+@pytest.mark.parametrize("entry,kw", [
+    ("mtlattn_varlen_bwd_workspace_size", dict(total_q=32768, total_kv=32768, num_heads_q=32, num_heads_kv=1)),
+    ("mtlattn_varlen_bwd_workspace_size", dict(total_q=65000, total_kv=65000, num_heads_q=32, num_heads_kv=1)),
+    ("mtlattn_varlen_bwd_workspace_size", dict(total_q=32000, total_kv=32000, num_heads_q=32, num_heads_kv=4,
+                                               head_dim=64)),
+    ("mtlattn_varlen_fwd_workspace_size", dict(total_q=2048, total_kv=1 << 20, num_heads_q=8, num_heads_kv=1)),
+])
+def test_plans_take_microseconds(lib, entry, kw):
+    """Every call makes its split plan on the host, also where the sequences
+    are long, the kv heads few and the plan says not to split. (These take 2
+    to 30 us; a search over every piece length took 1.4 to 80 ms.)"""
+    import time
+    p = problem(num_seqs=1, max_seqlen_q=kw["total_q"], **kw)
+    best = 1.0
+    for _ in range(20):
+        t = time.perf_counter()
+        getattr(lib, entry)(ctypes.byref(p))
+        best = min(best, time.perf_counter() - t)
+    assert best < 5e-4, f"{best * 1e6:.0f} us"
