@@ -150,7 +150,8 @@ __global__ __launch_bounds__(NW * 64, kWaves / NW) void fwd_mfma_kernel(FwdKPara
             if (q0 < 0 || q0 >= qr.end - qr.start) return -1;
             return key_tiles<KT>(q0, QT, qr.end - qr.start, kr.end - kr.start, p.causal, p.window).n;
         };
-        if (!find_piece(tiles, p.n_tiles, p.n_hg, p.split_grid, kFwdMinPieceKeys / KT, 0x7fffffff, p.piece_out,
+        // (a tile has no more pieces than the grid has workgroups)
+        if (!find_piece(tiles, p.n_tiles, p.n_hg, p.split_grid, kFwdMinPieceKeys / KT, p.split_grid, p.piece_out,
                         blockIdx.x, pc))
             return;
         if (pc.z == 0 && threadIdx.x == 0) p.first[pc.group * p.n_tiles + pc.t] = pc.id;
