@@ -277,11 +277,23 @@ bool decode_allowed(const mtlattn_problem* p) {
 // (and kv head), which needs no workspace. Waves share a sequence's keys where
 // the flash forward's walk over them is serial: 64 sequences of 256 keys, 32/8
 // heads 29 -> 14 us, one of 1024 27 -> 14, 32 of 64 keys 7.6 -> 7.4.
+// Not 9 to 16 queries of a GQA model with an even group at D = 128 on more than
+// two items per CU: a 16-row group then holds one head, so each head reads the
+// keys, which the flash forward shares over 2 to 8 heads. 64 sequences of 128
+// keys, 16 queries, 32/8 heads 21.6 us flash against 27.2, 256 of 512, 64/8 202
+// against 397; up to 512 items this kernel is ahead (32/8, 16 of 256 keys, 13
+// against 12, 16 of 1900 65 against 43), as at D = 64 (64/8, 64 of 512, 53
+// against 46) and with odd groups, whose heads the flash forward shares not at all.
 DecodePlan short_plan(const mtlattn_problem* p) {
     DecodePlan plan;
     if (!decode_allowed(p)) return plan;
+    const int g = p->num_heads_q / p->num_heads_kv;
+    const int64_t items = decode_groups(p) * p->num_seqs;
+    if (p->head_dim == 128 && g % 2 == 0 && decode_heads_per_group(g, p->max_seqlen_q) == 1 &&
+        items > 2 * (int64_t)device_cus())
+        return plan;
     plan.ns = 1;
-    plan.wg = decode_groups(p) * p->num_seqs > device_cus() ? 4 : 8;
+    plan.wg = items > device_cus() ? 4 : 8;
     return plan;
 }
 

@@ -80,6 +80,30 @@ def test_decode_workgroup(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window, bi
         _check(f"workspace={ws} ({need} bytes)", out, lse, ref, ref_lse, dtype)
 
 
+@pytest.mark.parametrize("n,q,kv,Hq,Hkv,D,window,flash", [
+    (32, 9, 100, 16, 2, 128, 0, False),      # 512 items of one head: the most
+    (33, 9, 100, 16, 2, 128, 0, True),
+    (130, 16, 70, 8, 4, 128, 50, True),
+    (130, 16, 70, 8, 4, 64, 0, False),       # D = 64
+    (180, 12, 60, 6, 2, 128, 0, False),      # odd group
+    (70, 8, 60, 16, 2, 128, 0, False),       # two heads a group
+])
+def test_short_calls_of_many_rows(monkeypatch, n, q, kv, Hq, Hkv, D, window, flash):
+    """The line between one workgroup per head group and the flash forward on
+    short calls of up to 16 queries: the flash side is the flash forward,
+    bitwise, the other is not; both against the oracle."""
+    print(f"\n[case] {n} x {q} queries, {kv} keys, {Hq}/{Hkv} heads D={D} window={window}", flush=True)
+    qs, k, v = _inputs([q] * n, [kv] * n, Hq, Hkv, D, torch.bfloat16, 9)
+    cq, ck = cu_of([q] * n), cu_of([kv] * n)
+    dev = [t.cuda() for t in (qs, k, v, cq, ck)]
+    out, lse, _ = _fwd(*dev, q, True, window, None, True)
+    ref, ref_lse = oracle.varlen_forward(qs, k, v, cq, ck, 1.0 / math.sqrt(D), True, window)
+    _check("short", out, lse, ref, ref_lse, torch.bfloat16)
+    monkeypatch.setenv("MTLATTN_NO_SPLITKV", "1")
+    fout, flse, _ = _fwd(*dev, q, True, window, None, True)
+    assert (torch.equal(out, fout) and torch.equal(lse, flse)) == flash
+
+
 @pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,max_q,window,bias", [
     ([1, 40, 0, 17], [200, 300, 9, 17], 8, 2, 128, torch.bfloat16, 1, 0, None),     # whole sequences
     ([5, 16, 33], [700, 16, 0], 8, 8, 64, torch.float16, 4, 0, None),               # (one without keys)
