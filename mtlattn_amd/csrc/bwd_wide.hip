@@ -8,6 +8,7 @@
 // build.py): the dK / dV accumulators are pinned to the AGPRs by inline asm
 // (mfma32_acc), and the S and dP products' results, which the VALU reads,
 // stay in VGPRs.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -20,12 +21,14 @@ namespace mtlattn {
 
 namespace {
 
-// The t-th key block (KB keys) of all sequences, heavy ones first: in order of
-// falling distance from its sequence's end (under end-aligned causal masking
-// the order of falling work) -- for j = the most blocks of a sequence .. 1, the
-// sequences with at least j blocks, each with its block nb - j, of each of
-// `heads` kv heads -- of `group` sequences at a time. Lane l holds sequence l
-// (num_seqs <= 64). False: there are fewer blocks.
+// The t-th key block (KB keys) of all sequences, heavy ones first within each
+// `group` (at most 64) sequences: in order of falling distance from its
+// sequence's end (under end-aligned causal masking the order of falling work)
+// -- for j = the most blocks of a sequence .. 1, the sequences with at least j
+// blocks, each with its block nb - j, of each of `heads` kv heads. A group's
+// numbers start at `heads` times the tile base of its first sequence
+// (common.h), which leaves a few unused at its end; lane l holds its sequence
+// l. False: no such block.
 //
 // The in-order dispatch then keeps the CUs busy to the end for any number of
 // sequences; workgroups that looped over blocks b and nb - 1 - b (equal work,
@@ -33,47 +36,45 @@ namespace {
 // took, backward, bf16, D = 128, 32/8 heads: 6 x 4096 2930 us against 2590, 16
 // ragged of 500 to 4096 2370 against 2060, 8 x 4096 non-causal (16/4) 4890
 // against 3990; D = 256, 2 x 4096, 16/4 1650 against 1385; 8 x 4096, whose 512 pairs
-// fit 2 rounds, as fast. Grids of 3 and more rounds take one half of the
-// sequences and then the other (launch_wide): sequences that run together
-// share the L2, 8 x 4096 3342 us against 3370 all at once; on smaller grids halves
-// leave a tail (7 x 4096, 16/4 heads, 1600 against 1555), as single sequences do
-// everywhere (8 x 4096 3970).
+// fit 2 rounds, as fast. Sequences that run together share the L2, so a group
+// is as small as leaves it two rounds of blocks (launch_wide): 72 x 4096 32.1 ms
+// against 33.8 in groups of 36, 64 x 1024, 16/8, D = 256 3.07 against 3.50 all at
+// once; groups of one round leave a tail (5 x 4096 2.77 ms against 2.32), as
+// single sequences do (8 x 4096 3970 us).
 template <int KB>
 __device__ inline bool heavy_first_block(const int* cu_kv, int num_seqs, int64_t total_kv, int group, int heads, int t,
                                          int& s, int& blk, int& head) {
     const int lane = threadIdx.x & 63;
+    // the last group that starts at or before t
+    int lo = 0, hi = (num_seqs - 1) / group;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (tile_base(cu_kv, mid * group, KB, total_kv) * heads <= t) lo = mid; else hi = mid - 1;
+    }
+    const int s0 = lo * group;
+    t -= tile_base(cu_kv, s0, KB, total_kv) * heads;
+    if (t < 0) return false;
     int nb = 0;
-    if (lane < num_seqs) {
-        const SeqRange kr = seq_range(cu_kv, lane, total_kv);
+    if (lane < min(group, num_seqs - s0)) {
+        const SeqRange kr = seq_range(cu_kv, s0 + lane, total_kv);
         nb = (kr.end - kr.start + KB - 1) / KB;
     }
-    for (int s0 = 0; s0 < num_seqs; s0 += group) {
-        const int mine = lane >= s0 && lane < s0 + group ? nb : 0;
-        int j = mine, sum = mine;
+    int j = nb;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            j = max(j, __shfl_xor(j, o));
-            sum += __shfl_xor(sum, o);
+    for (int o = 32; o > 0; o >>= 1) j = max(j, __shfl_xor(j, o));
+    for (j = __builtin_amdgcn_readfirstlane(j); j > 0; --j) {
+        const unsigned long long have = __ballot(nb >= j);
+        const int n = __popcll(have);
+        if (t < n * heads) {
+            head = t / n;
+            t -= head * n;
+            const int before = __popcll(have & ((1ull << lane) - 1ull));
+            const int l = __builtin_ctzll(__ballot(before == t && nb >= j));
+            s = s0 + l;
+            blk = __builtin_amdgcn_readlane(nb, l) - j;
+            return true;
         }
-        j = __builtin_amdgcn_readfirstlane(j);
-        sum = __builtin_amdgcn_readfirstlane(sum) * heads;
-        if (t >= sum) {
-            t -= sum;
-            continue;
-        }
-        for (; j > 0; --j) {
-            const unsigned long long have = __ballot(mine >= j);
-            const int n = __popcll(have);
-            if (t < n * heads) {
-                head = t / n;
-                t -= head * n;
-                const int before = __popcll(have & ((1ull << lane) - 1ull));
-                s = __builtin_ctzll(__ballot(before == t && mine >= j));
-                blk = __builtin_amdgcn_readlane(mine, s) - j;
-                return true;
-            }
-            t -= n * heads;
-        }
+        t -= n * heads;
     }
     return false;
 }
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_wide_kernel(BwdKParams p) {
     const int l32 = lane & 31, hi = lane >> 5;
     SplitPiece pc{};
     int s, blk, hk;                                    // sequence, key block, kv head
-    if (!SPLIT && p.causal && p.window <= 0 && p.num_seqs <= 64) {
+    if (!SPLIT && p.causal && p.window <= 0) {
         // (with a multiple of 8 kv heads each XCD takes whole heads, whose
         // workgroups share Q and dO in its L2; else every XCD takes every 8th
         // block of one list)
@@ -691,8 +692,10 @@ hipError_t launch_wide(const BwdArgs& a, hipStream_t st) {
     BwdKParams p = make_params(a);
     p.n_tiles = (int)(a.geo.total_kv / KB) + a.geo.num_seqs + 1;
     const bool split = !OUT_F32 && use_split(a, p.n_tiles);
-    const int ns = a.geo.num_seqs;
-    p.seq_group = ns > 4 && (int64_t)p.n_tiles * a.geo.hkv >= 3 * 256 ? (ns + 1) / 2 : ns;
+    // groups of equal size, of at least two rounds of blocks and at most 64 sequences
+    const int64_t ns = a.geo.num_seqs, blocks_all = std::max<int64_t>(a.geo.total_kv / KB, ns) * a.geo.hkv;
+    const int64_t groups = std::max<int64_t>((ns + 63) / 64, blocks_all / (2 * (int64_t)device_cus()));
+    p.seq_group = (int)((ns + groups - 1) / groups);
     const int64_t blocks = (int64_t)p.n_tiles * a.geo.hkv;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
     if constexpr (!OUT_F32) {

@@ -122,18 +122,6 @@ Geometry make_geo(const mtlattn_problem* p) {
     return g;
 }
 
-int device_cus() {
-    static int cache[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cache[dev] <= 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cache[dev] = n;
-    }
-    return cache[dev];
-}
-
 // Heads per 16-row decode group (largest divisor of g with heads * max_q <= 16).
 int decode_heads_per_group(int g, int max_q) {
     int hpb = 16 / (max_q > 0 ? max_q : 1);

@@ -35,6 +35,18 @@
 
 namespace mtlattn {
 
+int device_cus() {
+    static int cache[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cache[dev] <= 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cache[dev] = n;
+    }
+    return cache[dev];
+}
+
 namespace {
 
 constexpr int kWaves = 8;
@@ -647,19 +659,6 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdKParams p, int nw) {
 }
 
 int gcd_int(int a, int b) { while (b) { const int t = a % b; a = b; b = t; } return a; }
-
-// CUs of the current device (cached per device; 256 if unknown)
-int device_cus() {
-    static int cache[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cache[dev] <= 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cache[dev] = n;
-    }
-    return cache[dev];
-}
 
 // The split variant of each head dim: the same tiles as its unsplit kernel on
 // small grids (4-wave workgroups, two per CU, at D = 64 and 128).

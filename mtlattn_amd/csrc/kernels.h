@@ -9,6 +9,9 @@
 
 namespace mtlattn {
 
+// CUs of the current device (cached per device; 256 if unknown)
+int device_cus();
+
 // Tensor geometry shared by every kernel (the scalar block of the reference's
 // Params, src/ext.mm:44-57, with 64-bit row strides).
 struct Geometry {

@@ -344,7 +344,7 @@ def test_capi_splitkv_and_workspace_errors():
 @pytest.mark.parametrize("lens,Hq,Hkv,D,causal", [
     ([700, 1, 0, 256, 257, 511, 3000], 16, 8, 128, True),       # whole kv heads per XCD
     ([900, 40, 1300], 12, 12, 128, True),                       # one list for all heads
-    ([64] * 66 + [300], 8, 8, 80, True),                        # more sequences than lanes: natural order
+    ([64] * 66 + [300], 8, 8, 80, True),                        # more sequences than lanes
     ([600, 1500] * 10, 8, 8, 128, True),                        # sequences in two halves
     ([513, 130], 4, 4, 256, True),
     ([513, 700, 30], 8, 2, 96, False),
