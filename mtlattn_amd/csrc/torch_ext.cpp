@@ -277,6 +277,7 @@ at::Tensor varlen_attention_bwd_qkvpacked(const at::Tensor& qkv, const at::Tenso
     if (backward_into(q, k, v, o, dout, lse, cu_seqlens, cu_seqlens, scale, causal, window, c10::nullopt,
                       d.select(1, 0), d.select(1, 1), d.select(1, 2)))
         return d;
+    d.reset();
     const auto g = varlen_attention_bwd(q, k, v, o, dout, lse, cu_seqlens, cu_seqlens, scale, causal, window,
                                         c10::nullopt);
     return at::stack({std::get<0>(g), std::get<1>(g), std::get<2>(g)}, 1);
@@ -293,6 +294,8 @@ std::tuple<at::Tensor, at::Tensor> varlen_attention_bwd_kvpacked(
     if (backward_into(q, k, v, o, dout, lse, cu_seqlens_q, cu_seqlens_kv, scale, causal, window, c10::nullopt, dQ,
                       d.select(1, 0), d.select(1, 1)))
         return {dQ, d};
+    dQ.reset();
+    d.reset();
     const auto g = varlen_attention_bwd(q, k, v, o, dout, lse, cu_seqlens_q, cu_seqlens_kv, scale, causal, window,
                                         c10::nullopt);
     return {std::get<0>(g), at::stack({std::get<1>(g), std::get<2>(g)}, 1)};

@@ -50,3 +50,27 @@ def test_packed_gradients_in_place(lens, Hq, Hkv, D, dtype, causal, window):
         out = mt.flash_attn_varlen_qkvpacked_func(qkv, cu, max(lens), causal=causal, window=window)
         d, = torch.autograd.grad(out, qkv, do)
         assert torch.equal(out[:n], ref[:n]) and torch.equal(d, torch.stack((rq, rk, rv), 1))
+
+
+def test_packed_gradient_memory():
+    """Where the gradients are stacked (fp32), the backward holds no tensor for
+    writing in place besides: the three gradients, the stack of them, workspace."""
+    import mtlattn_amd as mt
+    print("\n[case] packed fp32 gradient memory", flush=True)
+    M, H, D = 20000, 8, 64
+    qkv = torch.randn(M, 3, H, D, device="cuda", requires_grad=True)
+    q, kv = (torch.randn(M, *s, H, D, device="cuda", requires_grad=True) for s in ((), (2,)))
+    cu = torch.tensor([0, M // 2, M], dtype=torch.int32, device="cuda")
+    for call, leaves in ((lambda: mt.flash_attn_varlen_qkvpacked_func(qkv, cu, M // 2), [qkv]),
+                         (lambda: mt.flash_attn_varlen_kvpacked_func(q, kv, cu, cu, M // 2, M // 2), [q, kv])):
+        out = call()
+        do = torch.randn_like(out)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        grads = torch.autograd.grad(out, leaves, do)
+        # in tensors of out's size; the half is for delta, a 64th (no split
+        # partials at this size)
+        stacked = 3 if len(leaves) == 1 else 2
+        assert torch.cuda.max_memory_allocated() - before < (3 + stacked + 0.5) * out.numel() * 4
+        del grads, out
