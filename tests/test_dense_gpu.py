@@ -4,7 +4,7 @@ packed path on the same inputs (the same kernels on packed copies)."""
 import pytest
 import torch
 
-from tests.helpers import randn
+from tests.helpers import REF_ATOL, randn
 
 pytestmark = pytest.mark.gpu
 
@@ -145,3 +145,27 @@ def test_padding_mask_rewritten_or_made_in_inference_mode(dtype):
                 check(m, [5, 130, 70])
     finally:
         mt.restore_sdpa()
+
+
+@pytest.mark.parametrize("layout,D,dtype", [("bhnd", 64, torch.bfloat16), ("bnhd", 128, torch.float16)])
+def test_dense_nan(monkeypatch, layout, D, dtype):
+    """NaN in padding rows of q, k and v reaches nothing; NaN in a token's k
+    reaches the rows that see it, as on the packed path."""
+    import mtlattn_amd as mt
+    print(f"\n[case] dense NaN {layout} D={D} {dtype}", flush=True)
+    B, H, N = 3, 4, 200
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (_tensor(layout, B, H, N, D, dtype, g) for _ in range(3))
+    lens = torch.tensor([200, 65, 0], device="cuda", dtype=torch.int32)
+    pad = (torch.arange(N, device="cuda")[None] >= lens[:, None])[:, None, :, None]
+    for causal in (False, True):
+        ref = mt._dense(q, k, v, 0.1, causal, lens)
+        bad = [t.masked_fill(pad, float("nan")) for t in (q, k, v)]
+        assert torch.equal(mt._dense(*bad, 0.1, causal, lens), ref)
+        bad[1][0, 2, 150, 3] = float("nan")
+        out = mt._dense(*bad, 0.1, causal, lens)
+        want = torch.zeros_like(out, dtype=torch.bool)
+        want[0, 2, 150 if causal else 0:] = True
+        assert torch.equal(out.isnan(), want)
+        # (at D = 64 a NaN row makes its wave take the row maxima again: other roundings of P)
+        assert (out.nan_to_num() - ref.masked_fill(want, 0)).abs().max().item() < REF_ATOL[dtype]

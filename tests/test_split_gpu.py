@@ -158,3 +158,130 @@ def test_forward_key_pieces(q_lens, kv_lens, Hq, Hkv, D, dtype, causal, window):
         _check("pieces", out[:n], lse[:n], ref, ref_lse, dtype)
         assert out[n:].isnan().all() and lse[n:].isnan().all(), "rows outside every sequence were written"
     assert torch.equal(runs[0][0][:n], runs[1][0][:n]) and torch.equal(runs[0][1][:n], runs[1][1][:n])
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv,D,dtype,bad_key", [
+    ([1, 3, 2], [300, 40, 700], 8, 2, 128, torch.bfloat16, 900),        # whole sequences (the last one's key)
+    ([1, 2], [2100, 1999], 8, 2, 64, torch.float16, 600),               # chunks of one workgroup
+    ([40, 17], [5000, 2100], 8, 2, 128, torch.bfloat16, 4975),          # key pieces, rows 15 and up
+    ([70], [4000], 4, 4, 80, torch.float16, 10),
+])
+def test_split_forwards_keep_nan_and_infinity(q_lens, kv_lens, Hq, Hkv, D, dtype, bad_key):
+    """A NaN or an infinite logit in one part of a row's keys makes the merged
+    row NaN, as a softmax over all of them does, and no other row; a key of
+    logit -inf drops out. Rows without a key stay 0, LSE -inf."""
+    print(f"\n[case] NaN in split forwards {q_lens} {kv_lens} D={D} {dtype}", flush=True)
+    q, k, v = _inputs(q_lens, kv_lens, Hq, Hkv, D, dtype, 12)
+    q[0, 1, 5] = float("nan")                       # one row of one head
+    k[bad_key, 0, 3] = float("nan")                 # the rows of kv head 0 that see it
+    k[bad_key + 5, Hkv - 1, 7] = float("inf")       # logits +inf or -inf, by the sign of q
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    ref, ref_lse = oracle.varlen_forward(q, k, v, cq, ck, 1.0 / math.sqrt(D), True)
+    want = ref.isnan().any(-1)
+    assert want.any() and not want.all()
+    dev = [t.cuda() for t in (q, k, v, cq, ck)]
+    for ws in (True, False):
+        if not ws and max(q_lens) <= 16 and sum(kv_lens) // len(kv_lens) >= 2048:
+            continue
+        out, lse, need = _fwd(*dev, max(q_lens), True, 0, None, ws)
+        assert torch.equal(out.isnan().any(-1), want) and torch.equal(out.isnan().all(-1), want), f"workspace={ws}"
+        assert lse[ref_lse.isnan()].isnan().all()
+        assert (out.float() - ref)[~want].abs().max().item() < REF_ATOL[dtype]
+        assert (lse - ref_lse)[~want].abs().max().item() < LSE_TOL[dtype]
+
+
+@pytest.mark.parametrize("last", [33, 64])
+def test_forward_key_pieces_at_the_most_tiles(last):
+    """256 row tiles are the most that a split launch numbers; with one more
+    the forward runs unsplit."""
+    print(f"\n[case] forward key pieces, {255 + last // 33} tiles", flush=True)
+    q_lens, kv_lens = [64] * 127 + [last], [1500 + 13 * i for i in range(128)]
+    q, k, v = _inputs(q_lens, kv_lens, 2, 1, 64, torch.bfloat16, 13)
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    ref, ref_lse = oracle.varlen_forward(q, k, v, cq, ck, 0.125, True)
+    out, lse, need = _fwd(*[t.cuda() for t in (q, k, v, cq, ck)], 64, True, 0, None, True)
+    assert (need > 0) == (last == 33)
+    _check("tiles", out, lse, ref, ref_lse, torch.bfloat16)
+
+
+def _bwd(q, k, v, do, out, lse, cq, ck, max_q, causal, nbytes, skew=0):
+    """(dq, dk, dv) of mtlattn_varlen_bwd on NaN-filled outputs with a
+    NaN-filled workspace of nbytes that starts `skew` bytes past an aligned
+    address, and the queried size."""
+    Hq, D, Hkv = q.shape[1], q.shape[2], k.shape[1]
+    p = capi.problem_for(q, k, cq, ck, max_q, 1.0 / math.sqrt(D), causal=causal)
+    need = capi.lib().mtlattn_varlen_bwd_workspace_size(ctypes.byref(p))
+    nbytes = need if nbytes is None else nbytes
+    ws = torch.full((nbytes // 4 + 4,), float("nan"), dtype=torch.float32, device="cuda")
+    g = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    capi.call("mtlattn_varlen_bwd", p, q.data_ptr(), Hq * D, k.data_ptr(), Hkv * D, v.data_ptr(), Hkv * D,
+              out.data_ptr(), Hq * D, do.data_ptr(), Hq * D, lse.data_ptr(), g[0].data_ptr(), g[1].data_ptr(),
+              g[2].data_ptr(), ws.data_ptr() + skew, nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return [t.cpu() for t in g], need
+
+
+@pytest.mark.parametrize("last", [256, 384])
+def test_dkv_pieces_at_the_most_tiles(last):
+    """As above for dK/dV: 256 key blocks in pieces, 257 unsplit."""
+    print(f"\n[case] dK/dV pieces, {255 + last // 256 + last // 384} tiles", flush=True)
+    q_lens, kv_lens = [600 - i for i in range(127)], [128] * 126 + [last]
+    q, k, v = _inputs(q_lens, kv_lens, 4, 1, 64, torch.bfloat16, 14)
+    do = randn(q.shape, torch.bfloat16, torch.Generator().manual_seed(15))
+    cq, ck = cu_of(q_lens), cu_of(kv_lens)
+    dev = [t.cuda() for t in (q, k, v, do, cq, ck)]
+    qd, kd, vd, dod, cqd, ckd = dev
+    out, lse, _ = _fwd(qd, kd, vd, cqd, ckd, 600, False, 0, None, True)
+    grads, need = _bwd(qd, kd, vd, dod, out.cuda(), lse.cuda(), cqd, ckd, 600, False, None)
+    assert (need > lse.numel() * 4) == (last == 256)
+    _, _, *refs = oracle.varlen_forward_backward(q, k, v, do, cq, ck, 0.125, False)
+    for nm, a, r in zip(("dq", "dk", "dv"), grads, refs):
+        assert torch.isfinite(a.float()).all(), nm
+        assert ((a.float() - r).norm() / r.norm()).item() < 8e-3, nm     # P, dS and the output in bf16, 2^-9 each
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,D,dtype", [
+    ([700, 90], 8, 2, 128, torch.bfloat16),
+    ([1000], 8, 2, 64, torch.float16),
+    ([500], 4, 2, 256, torch.bfloat16),
+])
+def test_split_dkv_keeps_nan_and_takes_any_workspace(lens, Hq, Hkv, D, dtype):
+    """dK/dV in pieces (the queried workspace) against the unsplit kernel (a
+    workspace of delta only): NaN rows of dout reach the same gradients. A
+    workspace that is not 16-byte aligned runs unsplit, bitwise, here and in the
+    forward's key pieces."""
+    print(f"\n[case] split dK/dV NaN {lens} {Hq}/{Hkv} D={D} {dtype}", flush=True)
+    q, k, v = _inputs(lens, lens, Hq, Hkv, D, dtype, 16)
+    do = randn(q.shape, dtype, torch.Generator().manual_seed(17))
+    cq, ck = cu_of(lens), cu_of(lens)
+    qd, kd, vd, cqd, ckd = (t.cuda() for t in (q, k, v, cq, ck))
+    out, lse, _ = _fwd(qd, kd, vd, cqd, ckd, max(lens), True, 0, None, True)
+    args = (out.cuda(), lse.cuda(), cqd, ckd, max(lens), True)
+    delta = lse.numel() * 4
+    for bad in (False, True):
+        if bad:
+            do[300, 1] = float("nan")               # (its query head's kv head, the keys it sees)
+        split, need = _bwd(qd, kd, vd, do.cuda(), *args, None)
+        whole, _ = _bwd(qd, kd, vd, do.cuda(), *args, delta)
+        skewed, _ = _bwd(qd, kd, vd, do.cuda(), *args, need, skew=4)
+        assert need > delta
+        for nm, a, b, c in zip(("dq", "dk", "dv"), split, whole, skewed):
+            assert torch.equal(b.isnan(), c.isnan()) and torch.equal(b.nan_to_num(), c.nan_to_num()), nm
+            assert torch.equal(a.isnan(), b.isnan()) and a.isnan().any().item() == bad, nm
+            err = (a.float() - b.float()).nan_to_num().norm() / b.float().nan_to_num().norm()
+            assert err.item() < 8e-3, nm
+
+
+def test_forward_key_pieces_need_an_aligned_workspace():
+    print("\n[case] forward key pieces, workspace alignment", flush=True)
+    q, k, v = _inputs([40], [5000], 8, 2, 128, torch.bfloat16, 18)
+    q, k, v, cq, ck = (t.cuda() for t in (q, k, v, cu_of([40]), cu_of([5000])))
+    ref, _, need = _fwd(q, k, v, cq, ck, 40, True, 0, None, False)
+    assert need > 0
+    p = capi.problem_for(q, k, cq, ck, 40, 1.0 / math.sqrt(128), causal=True)
+    ws = torch.empty(need // 4 + 4, dtype=torch.float32, device="cuda")
+    out = torch.full_like(q, float("nan"))
+    capi.call("mtlattn_varlen_fwd", p, q.data_ptr(), 1024, k.data_ptr(), 256, v.data_ptr(), 256, out.data_ptr(), None,
+              ws.data_ptr() + 4, need, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu(), ref)
