@@ -348,6 +348,14 @@ int mtlattn_unpack_padded(int32_t dtype, int32_t B, int32_t N, int32_t H, int32_
                           const void* src, const int32_t* lens, const int32_t* cu,
                           void* dst, int64_t sb, int64_t sh, int64_t sn, void* stream);
 
+/*
+ * Sets *flag = 1 if any of the `bytes` bytes at a and b (device pointers)
+ * differ, else leaves it; flag is an int32 that the device can write, such as
+ * pinned host memory, cleared by the caller. For the SDPA adapter, which keeps
+ * what it decided about a mask only while the mask's content stays.
+ */
+int mtlattn_content_differs(const void* a, const void* b, int64_t bytes, int32_t* flag, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

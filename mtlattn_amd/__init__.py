@@ -314,22 +314,30 @@ _PAD_DECISIONS = {}
 _PAD_COPY_BYTES = 16 << 20
 
 
-class _Answer:
-    """A device bool on its way to the host; bool() waits for it."""
+class _StillHolds:
+    """Whether a mask's content is still `kept`, asked of the device; bool()
+    waits for the answer."""
 
-    def __init__(self, flag):
-        self._host, self._event = flag, None
-        if flag.is_cuda:
-            with torch.cuda.device(flag.device):
-                self._host = torch.empty((), dtype=torch.bool, pin_memory=True)
-                self._host.copy_(flag, non_blocking=True)
-                self._event = torch.cuda.Event()
-                self._event.record()
+    def __init__(self, content, kept):
+        self._event = None
+        if not content.is_cuda:
+            self._holds = torch.equal(content, kept)
+            return
+        self._flag = torch.zeros((), dtype=torch.int32, pin_memory=True)
+        with torch.cuda.device(content.device):
+            _C.content_differs(content.contiguous(), kept, self._flag)
+            self._event = torch.cuda.Event()
+            self._event.record()
 
     def __bool__(self):
         if self._event is not None:
             self._event.synchronize()
-        return bool(self._host)
+            self._holds, self._event = self._flag.item() == 0, None
+        return self._holds
+
+    def __del__(self):          # (the device may still write the flag)
+        if self._event is not None:
+            self._event.synchronize()
 
 
 def _mask_content(attn_mask):
@@ -354,7 +362,11 @@ def _kept_decision(attn_mask, B, Hq, Nq, Nkv):
     # goes into the graph, as its launches do)
     if not ok or (attn_mask.is_cuda and torch.cuda.is_current_stream_capturing()):
         return ok, lens, True
-    return ok, lens, _Answer((_mask_content(attn_mask) == content).all())
+    if attn_mask.is_cuda:       # (made on another stream, perhaps; freed with the mask)
+        stream = torch.cuda.current_stream(attn_mask.device)
+        lens.record_stream(stream)
+        content.record_stream(stream)
+    return ok, lens, _StillHolds(_mask_content(attn_mask), content)
 
 
 def _padding_decision(attn_mask, B, Hq, Nq, Nkv):
@@ -369,7 +381,7 @@ def _padding_decision(attn_mask, B, Hq, Nq, Nkv):
     content = _mask_content(attn_mask)
     small = content.numel() * content.element_size() <= _PAD_COPY_BYTES
     if small:
-        content = content.clone()
+        content = content.clone(memory_format=torch.contiguous_format)
     keep0 = content if content.dtype == torch.bool else content > -1e30
     try:
         keep = keep0.expand(attn_mask.shape).expand(B, Hq, Nq, Nkv)

@@ -73,6 +73,7 @@ SIGNATURES = {
     "mtlattn_pack_padded": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "mtlattn_unpack_padded": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i64,
                                              _vp]),
+    "mtlattn_content_differs": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp]),
 }
 
 _lib = None

@@ -960,4 +960,12 @@ int mtlattn_unpack_padded(int32_t dtype, int32_t B, int32_t N, int32_t H, int32_
                          "unpack_padded");
 }
 
+int mtlattn_content_differs(const void* a, const void* b, int64_t bytes, int32_t* flag, void* stream) {
+    if (bytes < 0) return fail(MTLATTN_ERR_INVALID, "mtlattn: content_differs: negative size");
+    if (bytes == 0) return ok();
+    if (a == nullptr || b == nullptr || flag == nullptr)
+        return fail(MTLATTN_ERR_INVALID, "mtlattn: content_differs: null pointer");
+    return launch_status(launch_content_differs(a, b, bytes, flag, (hipStream_t)stream), "content_differs");
+}
+
 }  // extern "C"

@@ -211,6 +211,7 @@ hipError_t launch_pad_pack(int esize, int B, int N, int H, int D, const void* sr
                            int64_t sn, const int* lens, int* cu, void* dst, hipStream_t st);
 hipError_t launch_pad_unpack(int esize, int B, int N, int H, int D, const void* src, const int* lens, const int* cu,
                              void* dst, int64_t sb, int64_t sh, int64_t sn, hipStream_t st);
+hipError_t launch_content_differs(const void* a, const void* b, int64_t bytes, int* flag, hipStream_t st);
 
 // Partial rows of the split-KV workspace (fp32 O rows of D values plus one
 // LSE each): kv heads x head groups x work-item slots x 16.

@@ -498,6 +498,19 @@ at::Tensor unpack_padded(const at::Tensor& packed, const at::Tensor& cu, const a
     return out;
 }
 
+// Whether two contiguous GPU tensors differ in any byte, into a cleared int32
+// in pinned host memory, to be read after the current stream has come here.
+void content_differs(const at::Tensor& a, const at::Tensor& b, const at::Tensor& flag) {
+    TORCH_CHECK(a.is_cuda() && b.is_cuda() && a.get_device() == b.get_device() && a.is_contiguous() &&
+                    b.is_contiguous() && a.nbytes() == b.nbytes(),
+                "mtlattn: content_differs expects two contiguous tensors of one size on one GPU");
+    TORCH_CHECK(flag.is_cpu() && flag.is_pinned() && flag.scalar_type() == at::kInt && flag.numel() == 1,
+                "mtlattn: flag must be a pinned int32");
+    const c10::DeviceGuard guard(a.device());
+    check_rc(mtlattn_content_differs(a.data_ptr(), b.data_ptr(), (int64_t)a.nbytes(), flag.data_ptr<int32_t>(),
+                                     current_stream(a)));
+}
+
 bool mpp_available() { return true; }
 
 int64_t gpu_core_count() {
@@ -514,6 +527,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("x"), py::arg("lens"));
     m.def("unpack_padded", &unpack_padded, "Inverse of pack_padded (zeros for padded tokens)", py::arg("packed"),
           py::arg("cu_seqlens"), py::arg("lens"), py::arg("B"), py::arg("N"));
+    m.def("content_differs", &content_differs, "a pinned flag set where two GPU tensors differ", py::arg("a"),
+          py::arg("b"), py::arg("flag"));
     m.def("gpu_core_count", &gpu_core_count, "Compute-unit count of the current device (0 if unknown)");
     m.def("abi_version", [] { return mtlattn_abi_version(); }, "C ABI version of libmtlattn_hip.so");
     m.def("attn_splitkv", &attn_splitkv, "split-KV decode with an explicit split count (test entry)", py::arg("q"),

@@ -169,3 +169,30 @@ def test_dense_nan(monkeypatch, layout, D, dtype):
         assert torch.equal(out.isnan(), want)
         # (at D = 64 a NaN row makes its wave take the row maxima again: other roundings of P)
         assert (out.nan_to_num() - ref.masked_fill(want, 0)).abs().max().item() < REF_ATOL[dtype]
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4099, 1 << 20, (9 << 20) + 5])
+@pytest.mark.parametrize("skew", [0, 3])
+def test_content_differs(n, skew):
+    """One byte of difference anywhere is found: first, last, at the edges of
+    the 16-byte part; the bytes around the tensors do not count."""
+    from mtlattn_amd import _C
+    print(f"\n[case] content_differs {n} bytes at +{skew}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    x = torch.randint(0, 256, (n + skew + 8,), generator=g, dtype=torch.uint8).cuda()
+    y = x.clone()
+    y[n + skew:] += 1
+    a, b = x[skew:skew + n], y[skew:skew + n]
+
+    def differs():
+        flag = torch.zeros((), dtype=torch.int32, pin_memory=True)
+        _C.content_differs(a, b, flag)
+        torch.cuda.synchronize()
+        return flag.item()
+
+    assert differs() == 0
+    for i in sorted({0, n // 2, n - 1, max(0, n // 16 * 16 - 1), min(n - 1, n // 16 * 16)}):
+        b[i] += 1
+        assert differs() == 1, i
+        b[i] -= 1
+    assert differs() == 0
