@@ -33,7 +33,7 @@ namespace {
 // The in-order dispatch then keeps the CUs busy to the end for any number of
 // sequences; workgroups that looped over blocks b and nb - 1 - b (equal work,
 // but in whole rounds of pairs, and 12 VGPRs and 40 SGPRs spilled by the loop)
-// took, backward, bf16, D = 128, 32/8 heads: 6 x 4096 2930 us against 2590, 16
+// took, backward, bf16, D = 128, 32/8 heads: 6 x 4096 2930 us against 2740, 16
 // ragged of 500 to 4096 2370 against 2060, 8 x 4096 non-causal (16/4) 4890
 // against 3990; D = 256, 2 x 4096, 16/4 1650 against 1385; 8 x 4096, whose 512 pairs
 // fit 2 rounds, as fast. Sequences that run together share the L2, so a group

@@ -902,9 +902,9 @@ hipError_t launch_dims(const FwdArgs& a, hipStream_t st) {
 // row tiles that each walk thousands of keys one after the other: there the
 // tiles' keys are cut into pieces of at least 1024, one workgroup each, which
 // fp32 partials of O and the LSE merge. Forward before -> after, bf16 causal,
-// 32/8 heads, D = 128: 512 queries against 8192 keys 148 -> 88 us, 32 against
+// 32/8 heads, D = 128: 512 queries against 8192 keys 148 -> 87 us, 32 against
 // 16384 383 -> 40, 2 x 512 against 8192 to 32768 419 -> 308, 1024 against
-// 32768 771 -> 520 (1.06 PFLOP/s); 8 x 17 against 3000 76 -> 39. The line: the
+// 32768 771 -> 520 (1.04 PFLOP/s); 8 x 17 against 3000 76 -> 39. The line: the
 // split has to save 15% of the walk by this count of key tiles on sequences of
 // the average length, with kFwdSplitCost for the pieces' start and the merge's
 // launch (at 1 x 1500 causal, 384 unsplit workgroups, it lost, 45 -> 56 us).

@@ -101,7 +101,7 @@ inline int64_t plan_piece(const int64_t* n, int64_t tiles, int64_t mult, int64_t
 }
 
 // How the 16-bit dK/dV cuts its work (make_dkv_plan): pieces == 1: one
-// workgroup per key block or pair of key blocks; else at most `pieces` pieces
+// workgroup per key block; else at most `pieces` pieces
 // per key block on a grid of `grid` workgroups.
 struct DkvPlan {
     int pieces = 1, grid = 0;
