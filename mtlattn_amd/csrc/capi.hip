@@ -68,11 +68,11 @@ bool aligned16(const void* ptr, int64_t row_stride, int dtype) {
     return ((uintptr_t)ptr & 15u) == 0 && (row_stride * elem_size(dtype)) % 16 == 0;
 }
 
-// The matrix-core kernels address a staged 64-row tile with 32-bit per-lane
-// byte offsets: row strides below 2^25 elements (the reference passes row
-// strides as uint32, src/ext.mm:48-51). Larger strides take the portable
+// The matrix-core kernels address a staged tile of up to 128 rows with 32-bit
+// per-lane byte offsets: row strides below 2^24 elements (the reference passes
+// row strides as uint32, src/ext.mm:48-51). Larger strides take the portable
 // kernels.
-bool tile_stride_ok(int64_t row_stride) { return row_stride >= 0 && row_stride < (int64_t(1) << 25); }
+bool tile_stride_ok(int64_t row_stride) { return row_stride >= 0 && row_stride < (int64_t(1) << 24); }
 
 // Shape/flag checks shared by every entry (src/ext.mm:306-331).
 int check_problem(const mtlattn_problem* p) {

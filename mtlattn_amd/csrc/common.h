@@ -286,7 +286,7 @@ __device__ inline void lds_dma16s(const void* sbase, uint32_t voff, const char* 
 // base is scalar). A tile that runs past row_end recomputes the offsets with
 // rows >= row_end reading row row_end - 1 (finite data the kernels mask
 // out). The offsets are 32-bit: callers keep ROWS * 2 * rs below 2^32 (row
-// strides below 2^25 elements for 64-row tiles).
+// strides below 2^24 elements for 128-row tiles).
 template <int D, int ROWS, int NW, int DV = D>
 struct TileStager {
     static_assert(DV % 8 == 0 && DV <= D, "head dim");

@@ -285,3 +285,25 @@ def test_forward_key_pieces_need_an_aligned_workspace():
               ws.data_ptr() + 4, need, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert torch.equal(out.cpu(), ref)
+
+
+@pytest.mark.parametrize("stride", [(1 << 24) - 8, (1 << 24) + 8])
+def test_row_strides_around_the_tile_limit(stride):
+    """128-row tiles reach 32-bit byte offsets at row strides of 2^24 elements:
+    below, the last row of a tile; at and above, the portable kernels. Against
+    the same rows packed."""
+    import mtlattn as mt
+    print(f"\n[case] row stride {stride}", flush=True)
+    n, H, D = 130, 2, 96                             # (head dims 80 to 96: 128-key tiles)
+    g = torch.Generator().manual_seed(19)
+    q, k, v = (randn((n, H, D), torch.bfloat16, g).cuda() for _ in range(3))
+    cu = cu_of([n], "cuda")
+    wide = torch.empty((n - 1) * stride + 2 * H * D, dtype=torch.bfloat16, device="cuda")
+    ks, vs = (wide.as_strided((n, H, D), (stride, D, 1), i * H * D) for i in range(2))
+    ks.copy_(k)
+    vs.copy_(v)
+    with torch.no_grad():
+        for causal in (False, True):
+            ref = mt.varlen_attention(q, k, v, cu, cu, n, causal=causal)
+            out = mt.varlen_attention(q, ks, vs, cu, cu, n, causal=causal)
+            assert (out.float() - ref.float()).abs().max().item() < REF_ATOL[torch.bfloat16]
